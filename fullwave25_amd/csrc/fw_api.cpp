@@ -731,7 +731,7 @@ int setup_fused_boundary(fw_sim* s, const fw::BoundaryLists& bl) {
     const char* env = getenv("FULLWAVE_HIP_FUSED_BOUNDARY");  // "0": a launch of its own (tests)
     if (env && env[0] == '0') return FW_OK;
     const fw::LaunchCfg& c = s->cfg_p;
-    const int tile_w = c.variant == 2 ? 256 : (c.width == 64 || c.width == 256 ? c.width : 128);
+    const int tile_w = c.variant == 2 ? fw::tile2d_width(c.chunk) : (c.width == 64 || c.width == 256 ? c.width : 128);
     const int rows = c.variant == 2 ? c.chunk : (c.chunk < 2 ? 2 : c.chunk);
     const unsigned gx = (unsigned)((s->ds.ny + tile_w - 1) / tile_w);
     std::vector<int32_t> pts;

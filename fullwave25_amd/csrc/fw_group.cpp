@@ -26,10 +26,9 @@ struct fw_group {
     int32_t* points = nullptr;  // every member's points grouped by tile (GroupBoundary lists)
     int ntiles = 0;
     uint32_t blocks = 0;
-    int variant = 1;  // 1: marching kernels (width lanes, chunk rows); 2: tiled (256 x chunk)
+    int variant = 1;  // 1: marching kernels (width lanes, chunk rows); 2: tiled (chunk rows)
     int width = 256, chunk = 16, max_ndmap = 1;
-    int coef_sets = 1;      // LDS coefficient sets of the tiled kernels (largest member)
-    bool all_coded = true;  // every member reads coded relaxation coefficients
+    bool fast = true;  // every member reads coded coefficients and has the same weights on both axes
     // steady steps replayed from a captured graph of graph_steps steps (0: plain launches); the
     // boundary pass adds the device counter base_dev, which each replay advances
     int64_t graph_steps = 0;
@@ -161,7 +160,7 @@ int build(fw_group* g) {
         unsigned gx, gy;
         int64_t chunk = g->chunk;
         if (g->variant == 2) {
-            gx = fw::group_tiles_x(s->ds.ny, 256);
+            gx = fw::group_tiles_x(s->ds.ny, fw::tile2d_width(g->chunk));
             gy = fw::group_tile_rows(s->ds.nx, g->chunk);
         } else {
             gx = fw::group_tiles_x(s->ds.ny, g->width);
@@ -177,7 +176,7 @@ int build(fw_group* g) {
         fw::BoundaryLists bl;
         int rc = fw::resolve_boundary(s->d, s->ds.sx, s->ds.sy, s->icc, s->outc, s->zero, &bl);
         if (rc != FW_OK) return rc;
-        const int tile_w = g->variant == 2 ? 256 : g->width;
+        const int tile_w = g->variant == 2 ? fw::tile2d_width(g->chunk) : g->width;
         const fw::PointTable ps = fw::point_table(s->ds.nx, s->ds.ny, gx, tile_w, (int)chunk, bl, &pts);
         for (int b = 0; b < s->nshots; ++b) {
             fw::GroupTile t{};
@@ -198,9 +197,7 @@ int build(fw_group* g) {
             slots.push_back(ps);
         }
         if (s->ds.ndmap > g->max_ndmap) g->max_ndmap = s->ds.ndmap;
-        const int sets = s->ds.ndmap * (s->ds.coef_axes_same ? 1 : 2);
-        if (sets > g->coef_sets) g->coef_sets = sets;
-        if (!s->ds.rcode) g->all_coded = false;
+        if (!s->ds.rcode || !s->ds.coef_axes_same) g->fast = false;
         g->shots_of.push_back(s->nshots);
     }
     if (blocks >= (1ull << 32)) return fw::set_error(FW_ERR_INVALID, "the group has too many tiles for one launch");
@@ -246,8 +243,8 @@ hipError_t launch_stencil(const fw_group* g, bool velocity, bool boundary = fals
                           int64_t it = 0) {
     const fw::GroupStep gs{boundary ? g->bounds : nullptr, base, it};
     if (g->variant == 2)
-        return fw::launch_group_tile2d(g->tiles, g->ntiles, g->blocks, g->chunk, g->coef_sets, g->all_coded, velocity,
-                                       gs, g->stream);
+        return fw::launch_group_tile2d(g->tiles, g->ntiles, g->blocks, g->chunk, g->max_ndmap * (g->fast ? 1 : 2),
+                                       g->fast, velocity, gs, g->stream);
     return fw::launch_group_2d(g->tiles, g->ntiles, g->blocks, g->width, g->max_ndmap, velocity, gs, g->stream);
 }
 
@@ -377,7 +374,7 @@ int fw_group_create_shaped(fw_sim* const* sims, int32_t n, int32_t variant, int3
     if (variant < 0 || variant > 2)
         return fw::set_error(FW_ERR_INVALID, "group variant must be 1 (marching), 2 (tiled) or 0 (timed)");
     if (variant == 2) {
-        if (width != 0 && width != 256) return fw::set_error(FW_ERR_INVALID, "tiled groups are 256 columns wide");
+        if (width != 0 && width != 256) return fw::set_error(FW_ERR_INVALID, "tiled groups take width 256 or 0 (256 lanes a workgroup; no tile is 256 columns wide)");
         if (chunk != 0 && chunk != 8 && chunk != 16 && chunk != 32)
             return fw::set_error(FW_ERR_INVALID, "tiled group rows must be 8, 16 or 32 (0: timed)");
     } else {

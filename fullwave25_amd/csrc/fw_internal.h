@@ -148,6 +148,34 @@ __device__ __forceinline__ CodedCoef cell_coef(const DevSim& s, uint32_t c) {
     return coef_of_code<VEL, UNIFORM>(s, c, gld16(s.rcode, c));
 }
 
+// The arithmetic of the update, one rounding order for every forward kernel (contraction by the
+// compiler is off, so that the families, their shapes and paths agree bit for bit).
+// one tap of an axial stencil: acc + w (hi - lo)
+__device__ __forceinline__ float tap(float acc, float w, float hi, float lo) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(w, hi - lo, acc);
+}
+// a memory variable: b m + a D
+__device__ __forceinline__ float memory_step(float b, float m, float a, float D) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(b, m, a * D);
+}
+// a corrected derivative: D / kappa + (q1 + q2)
+__device__ __forceinline__ float corrected(float D, float ik, float q1, float q2) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(D, ik, q1 + q2);
+}
+// v - dt / rho_bar u, rho_bar the mean of the two voxels' densities
+__device__ __forceinline__ float velocity_step(float v, float dt, float rho0, float rho1, float u) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(-(dt / (0.5f * (rho0 + rho1))), u, v);
+}
+// p - dt K div
+__device__ __forceinline__ float pressure_step(float p, float dt, float K, float div) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(-(dt * K), div, p);
+}
+
 // The fields of one shot of the batch.
 __host__ __device__ inline DevSim shot_view(const DevSim& s, int shot) {
     DevSim t = s;
@@ -318,8 +346,8 @@ enum KernelKind { kVelocity = 0, kPressure = 1, kBoundary = 2, kNumKinds = 3 };
 //   variant 0: per-cell kernels (one thread per cell)
 //   variant 1: x-marching kernels; `width` lanes per workgroup along the contiguous axis
 //              (2D: 64, 128 or 256; 3D: fixed 64 x 8 tile) and `chunk` planes per workgroup
-//   variant 2: 2D tiled kernels with 4-wide vector access; tiles of `chunk` rows (8, 16, 32)
-//              by 256 columns (needs ny % 4 == 0)
+//   variant 2: 2D tiled kernels with 4-wide vector access; workgroups of `width` = 256 lanes on
+//              tiles of `chunk` rows (8, 16, 32) by tile2d_width(chunk) columns (needs ny % 4 == 0)
 //   variant 3: 3D x-marching kernels with software pipelining (planes and per-cell operands
 //              loaded one iteration ahead); `width` = workgroup size 512 or 1024
 //   variant 4: as 3, with the per-cell operands loaded at the top of their own iteration
@@ -331,6 +359,7 @@ struct LaunchCfg {
 
 bool streaming_supported(const DevSim& s);
 bool tile2d_supported(const DevSim& s);
+int tile2d_width(int rows);  // columns of the tile of `rows` rows (8, 16 or 32)
 hipError_t launch_velocity(const DevSim& s, const LaunchCfg& cfg, hipStream_t st);
 hipError_t launch_pipe3d(const DevSim& s, const LaunchCfg& cfg, bool velocity, hipStream_t st);
 // gs.g non-null (2D marching and tiled kernels, untaped steps: pressure_fuses_boundary): the
@@ -350,12 +379,12 @@ unsigned group_tiles_y(int64_t nx, int chunk);
 // the pressure launches (velocity == false) also do each member's boundary work of the step (gs)
 hipError_t launch_group_2d(const GroupTile* t, int n, uint32_t blocks, int width, int max_ndmap, bool velocity,
                            const GroupStep& gs, hipStream_t st);
-// grouped tiled 2D kernels (isotropic relaxation, ny % 4 == 0): 256 columns x `rows` rows
-// (8, 16 or 32) per workgroup; coef_sets: the most coefficient sets any member stages in LDS
-// (ndmap, times 2 unless its axes share their sets); all_coded: every member has codes (the
-// kernel then holds the coded path only, fewer registers)
+// grouped tiled 2D kernels (isotropic relaxation, ny % 4 == 0): tile2d_width(rows) columns x `rows`
+// rows (8, 16 or 32) per workgroup; fast: every member has codes and the same weights on both axes
+// (the kernel then holds that path only, fewer registers); coef_sets: the most coefficient sets any
+// member stages in LDS (ndmap, times 2 unless fast)
 unsigned group_tile_rows(int64_t nx, int rows);
-hipError_t launch_group_tile2d(const GroupTile* t, int n, uint32_t blocks, int rows, int coef_sets, bool all_coded,
+hipError_t launch_group_tile2d(const GroupTile* t, int n, uint32_t blocks, int rows, int coef_sets, bool fast,
                                bool velocity, const GroupStep& gs, hipStream_t st);
 hipError_t launch_reciprocal(float* data, int64_t n, hipStream_t st);
 // [nshots][ncoords][ntic] -> [nshots][ntic][ncoords]

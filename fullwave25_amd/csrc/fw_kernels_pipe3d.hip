@@ -350,42 +350,41 @@ __global__ __launch_bounds__(PZ3 * TY) void k_velocity_pipe3d(DevSim batch, int 
                 const float* w = SAME ? ws : coefp<UNIFORM, SAME>(coefs, cur.dc, 0);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (q[7 + m] - q[8 - m]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], q[7 + m], q[8 - m]);
                 float tr = 0.f;
                 tr += (A(pp, 1, 0) - A(p0, 1, 0)) + (A(pp, -1, 0) - A(p0, -1, 0));
                 tr += (A(pp, 0, 1) - A(p0, 0, 1)) + (A(pp, 0, -1) - A(p0, 0, -1));
-                D[0] = acc + w[8] * tr;
+                D[0] = __builtin_fmaf(w[8], tr, acc);
             }
             {
                 const float* w = SAME ? ws : coefp<UNIFORM, SAME>(coefs, cur.dc, 1);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (A(p0, m, 0) - A(p0, -(m - 1), 0));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], A(p0, m, 0), A(p0, -(m - 1), 0));
                 float tr = 0.f;
                 tr += (A(pp, 1, 0) - A(pp, 0, 0)) + (A(pm, 1, 0) - A(pm, 0, 0));
                 tr += (A(p0, 1, 1) - A(p0, 0, 1)) + (A(p0, 1, -1) - A(p0, 0, -1));
-                D[1] = acc + w[8] * tr;
+                D[1] = __builtin_fmaf(w[8], tr, acc);
             }
             {
                 const float* w = SAME ? ws : coefp<UNIFORM, SAME>(coefs, cur.dc, 2);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (A(p0, 0, m) - A(p0, 0, -(m - 1)));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], A(p0, 0, m), A(p0, 0, -(m - 1)));
                 float tr = 0.f;
                 tr += (A(pp, 0, 1) - A(pp, 0, 0)) + (A(pm, 0, 1) - A(pm, 0, 0));
                 tr += (A(p0, 1, 1) - A(p0, 1, 0)) + (A(p0, -1, 1) - A(p0, -1, 0));
-                D[2] = acc + w[8] * tr;
+                D[2] = __builtin_fmaf(w[8], tr, acc);
             }
             const float rnb[3] = {cur.rho_x, cur.rho_y, cur.rho_z};
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
                 const int ax = ISO ? 0 : a;
-                const float qq1 = cur.b[ax][0] * cur.psi[a][0] + cur.a[ax][0] * D[a];
-                const float qq2 = cur.b[ax][1] * cur.psi[a][1] + cur.a[ax][1] * D[a];
+                const float qq1 = memory_step(cur.b[ax][0], cur.psi[a][0], cur.a[ax][0], D[a]);
+                const float qq2 = memory_step(cur.b[ax][1], cur.psi[a][1], cur.a[ax][1], D[a]);
                 gstnt(s.psi[a][0], c, qq1);
                 gstnt(s.psi[a][1], c, qq2);
-                const float rho_bar = 0.5f * (rho_i + rnb[a]);
-                gst(s.v[a], c, cur.v[a] - s.dt / rho_bar * (D[a] * cur.ik[ax] + (qq1 + qq2)));
+                gst(s.v[a], c, velocity_step(cur.v[a], s.dt, rho_i, rnb[a], corrected(D[a], cur.ik[ax], qq1, qq2)));
             }
         }
         rho_i = cur.rho_x;
@@ -534,43 +533,43 @@ __global__ __launch_bounds__(PZ3 * TY) void k_pressure_pipe3d(DevSim batch, int 
                 const float* w = SAME ? ws : coefp<UNIFORM, SAME>(coefs, cur.dc, 0);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (q[7 + m] - q[8 - m]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], q[7 + m], q[8 - m]);
                 float tr = 0.f;
                 tr += (X(x0, 1, 0) - X(xm, 1, 0)) + (X(x0, -1, 0) - X(xm, -1, 0));
                 tr += (X(x0, 0, 1) - X(xm, 0, 1)) + (X(x0, 0, -1) - X(xm, 0, -1));
-                D[0] = acc + w[8] * tr;
+                D[0] = __builtin_fmaf(w[8], tr, acc);
             }
             {
                 const float* w = SAME ? ws : coefp<UNIFORM, SAME>(coefs, cur.dc, 1);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (Y(y0, m - 1, 0) - Y(y0, -m, 0));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], Y(y0, m - 1, 0), Y(y0, -m, 0));
                 float tr = 0.f;
                 tr += (Y(yp, 0, 0) - Y(yp, -1, 0)) + (Y(ym, 0, 0) - Y(ym, -1, 0));
                 tr += (Y(y0, 0, 1) - Y(y0, -1, 1)) + (Y(y0, 0, -1) - Y(y0, -1, -1));
-                D[1] = acc + w[8] * tr;
+                D[1] = __builtin_fmaf(w[8], tr, acc);
             }
             {
                 const float* w = SAME ? ws : coefp<UNIFORM, SAME>(coefs, cur.dc, 2);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (Z(z0, 0, m - 1) - Z(z0, 0, -m));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], Z(z0, 0, m - 1), Z(z0, 0, -m));
                 float tr = 0.f;
                 tr += (Z(zp, 0, 0) - Z(zp, 0, -1)) + (Z(zm, 0, 0) - Z(zm, 0, -1));
                 tr += (Z(z0, 1, 0) - Z(z0, 1, -1)) + (Z(z0, -1, 0) - Z(z0, -1, -1));
-                D[2] = acc + w[8] * tr;
+                D[2] = __builtin_fmaf(w[8], tr, acc);
             }
             float div = 0.f;
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
                 const int ax = ISO ? 0 : a;
-                const float qq1 = cur.b[ax][0] * cur.phi[a][0] + cur.a[ax][0] * D[a];
-                const float qq2 = cur.b[ax][1] * cur.phi[a][1] + cur.a[ax][1] * D[a];
+                const float qq1 = memory_step(cur.b[ax][0], cur.phi[a][0], cur.a[ax][0], D[a]);
+                const float qq2 = memory_step(cur.b[ax][1], cur.phi[a][1], cur.a[ax][1], D[a]);
                 gstnt(s.phi[a][0], c, qq1);
                 gstnt(s.phi[a][1], c, qq2);
-                div += D[a] * cur.ik[ax] + (qq1 + qq2);
+                div += corrected(D[a], cur.ik[ax], qq1, qq2);
             }
-            gst(s.p, c, cur.p - s.dt * cur.K * div);
+            gst(s.p, c, pressure_step(cur.p, s.dt, cur.K, div));
         }
         if (AHEAD) cur = nxt;
     }

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(256) void k_velocity_simple(DevSim batch) {
         const int64_t sa = stride[a];
         float acc = 0.f;
 #pragma unroll
-        for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (p[c + m * sa] - p[c - (m - 1) * sa]);
+        for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], p[c + m * sa], p[c - (m - 1) * sa]);
         float tr = 0.f;
 #pragma unroll
         for (int b = 0; b < ND; ++b) {
@@ -50,19 +50,19 @@ __global__ __launch_bounds__(256) void k_velocity_simple(DevSim batch) {
             const int64_t sb = stride[b];
             tr += (p[c + sa + sb] - p[c + sb]) + (p[c + sa - sb] - p[c - sb]);
         }
-        const float D = acc + w[8] * tr;
-        const float rho_bar = 0.5f * (rho_c + s.rho[c + sa]);
+        const float D = __builtin_fmaf(w[8], tr, acc);
+        const float rho_n = s.rho[c + sa];
         if (EXPO) {
-            s.v[a][c] = decay * (s.v[a][c] - s.dt / rho_bar * D);
+            s.v[a][c] = decay * velocity_step(s.v[a][c], s.dt, rho_c, rho_n, D);
             if (TAPE) s.tape_u[a][c] = decay * D;
             continue;
         }
-        const float q1 = s.bv[a][0][c] * s.psi[a][0][c] + s.av[a][0][c] * D;
-        const float q2 = s.bv[a][1][c] * s.psi[a][1][c] + s.av[a][1][c] * D;
+        const float q1 = memory_step(s.bv[a][0][c], s.psi[a][0][c], s.av[a][0][c], D);
+        const float q2 = memory_step(s.bv[a][1][c], s.psi[a][1][c], s.av[a][1][c], D);
         s.psi[a][0][c] = q1;
         s.psi[a][1][c] = q2;
-        const float u = D * s.ikv[a][c] + (q1 + q2);
-        s.v[a][c] -= s.dt / rho_bar * u;
+        const float u = corrected(D, s.ikv[a][c], q1, q2);
+        s.v[a][c] = velocity_step(s.v[a][c], s.dt, rho_c, rho_n, u);
         if (TAPE) s.tape_u[a][c] = u;
     }
 }
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_pressure_simple(DevSim batch) {
         const int64_t sa = stride[a];
         float acc = 0.f;
 #pragma unroll
-        for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (va[c + (m - 1) * sa] - va[c - m * sa]);
+        for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], va[c + (m - 1) * sa], va[c - m * sa]);
         float tr = 0.f;
 #pragma unroll
         for (int b = 0; b < ND; ++b) {
@@ -92,21 +92,21 @@ __global__ __launch_bounds__(256) void k_pressure_simple(DevSim batch) {
             const int64_t sb = stride[b];
             tr += (va[c + sb] - va[c - sa + sb]) + (va[c - sb] - va[c - sa - sb]);
         }
-        const float D = acc + w[8] * tr;
+        const float D = __builtin_fmaf(w[8], tr, acc);
         if (EXPO) {
             div += D;
             continue;
         }
-        const float q1 = s.bp[a][0][c] * s.phi[a][0][c] + s.ap[a][0][c] * D;
-        const float q2 = s.bp[a][1][c] * s.phi[a][1][c] + s.ap[a][1][c] * D;
+        const float q1 = memory_step(s.bp[a][0][c], s.phi[a][0][c], s.ap[a][0][c], D);
+        const float q2 = memory_step(s.bp[a][1][c], s.phi[a][1][c], s.ap[a][1][c], D);
         s.phi[a][0][c] = q1;
         s.phi[a][1][c] = q2;
-        div += D * s.ikp[a][c] + (q1 + q2);
+        div += corrected(D, s.ikp[a][c], q1, q2);
     }
     if (EXPO)
-        s.p[c] = s.aexp[c] * (s.p[c] - s.dt * s.K[c] * div);
+        s.p[c] = s.aexp[c] * pressure_step(s.p[c], s.dt, s.K[c], div);
     else
-        s.p[c] -= s.dt * s.K[c] * div;
+        s.p[c] = pressure_step(s.p[c], s.dt, s.K[c], div);
     if (TAPE) s.tape_div[c] = div;
 }
 

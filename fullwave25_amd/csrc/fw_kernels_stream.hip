@@ -136,32 +136,30 @@ __device__ __forceinline__ void velocity_2d_tile(const DevSim& s, unsigned bx, u
                 const float* w = coef_row<UNIFORM>(lds_coef, R.dc, 0);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (q[7 + m] - q[8 - m]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], q[7 + m], q[8 - m]);
                 float tr = 0.f;
                 tr += (rp[1] - r0[1]) + (rp[-1] - r0[-1]);
-                const float D = acc + w[8] * tr;
-                const float qq1 = R.b1[0] * R.ps1[0] + R.a1[0] * D;
-                const float qq2 = R.b2[0] * R.ps2[0] + R.a2[0] * D;
+                const float D = __builtin_fmaf(w[8], tr, acc);
+                const float qq1 = memory_step(R.b1[0], R.ps1[0], R.a1[0], D);
+                const float qq2 = memory_step(R.b2[0], R.ps2[0], R.a2[0], D);
                 gstnt(s.psi[0][0], c, qq1);
                 gstnt(s.psi[0][1], c, qq2);
-                const float rho_bar = 0.5f * (rho_i + R.rho_next);
-                gst32(s.v[0], c, R.v[0] - s.dt / rho_bar * (D * R.ik[0] + (qq1 + qq2)));
+                gst32(s.v[0], c, velocity_step(R.v[0], s.dt, rho_i, R.rho_next, corrected(D, R.ik[0], qq1, qq2)));
             }
             {  // y: axial from row r in LDS, transverse from rows r-1, r+1 at j, j+1
                 constexpr int ax = ISO ? 0 : 1;
                 const float* w = coef_row<UNIFORM>(lds_coef, R.dc, 1);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (r0[m] - r0[-(m - 1)]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], r0[m], r0[-(m - 1)]);
                 float tr = 0.f;
                 tr += (rp[1] - rp[0]) + (rm[1] - rm[0]);
-                const float D = acc + w[8] * tr;
-                const float qq1 = R.b1[ax] * R.ps1[1] + R.a1[ax] * D;
-                const float qq2 = R.b2[ax] * R.ps2[1] + R.a2[ax] * D;
+                const float D = __builtin_fmaf(w[8], tr, acc);
+                const float qq1 = memory_step(R.b1[ax], R.ps1[1], R.a1[ax], D);
+                const float qq2 = memory_step(R.b2[ax], R.ps2[1], R.a2[ax], D);
                 gstnt(s.psi[1][0], c, qq1);
                 gstnt(s.psi[1][1], c, qq2);
-                const float rho_bar = 0.5f * (rho_i + R.rho_right);
-                gst32(s.v[1], c, R.v[1] - s.dt / rho_bar * (D * R.ik[ax] + (qq1 + qq2)));
+                gst32(s.v[1], c, velocity_step(R.v[1], s.dt, rho_i, R.rho_right, corrected(D, R.ik[ax], qq1, qq2)));
             }
         }
         rho_i = R.rho_next;
@@ -305,32 +303,32 @@ __device__ __forceinline__ void pressure_2d_tile(const DevSim& s, unsigned bx, u
                 const float* w = coef_row<UNIFORM>(lds_coef, R.dc, 0);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (q[7 + m] - q[8 - m]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], q[7 + m], q[8 - m]);
                 float tr = 0.f;
                 tr += (x0[1] - xm[1]) + (x0[-1] - xm[-1]);
-                const float D = acc + w[8] * tr;
-                const float qq1 = R.b1[0] * R.ph1[0] + R.a1[0] * D;
-                const float qq2 = R.b2[0] * R.ph2[0] + R.a2[0] * D;
+                const float D = __builtin_fmaf(w[8], tr, acc);
+                const float qq1 = memory_step(R.b1[0], R.ph1[0], R.a1[0], D);
+                const float qq2 = memory_step(R.b2[0], R.ph2[0], R.a2[0], D);
                 gstnt(s.phi[0][0], c, qq1);
                 gstnt(s.phi[0][1], c, qq2);
-                div += D * R.ik[0] + (qq1 + qq2);
+                div += corrected(D, R.ik[0], qq1, qq2);
             }
             {
                 constexpr int ax = ISO ? 0 : 1;
                 const float* w = coef_row<UNIFORM>(lds_coef, R.dc, 1);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (y0[m - 1] - y0[-m]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], y0[m - 1], y0[-m]);
                 float tr = 0.f;
                 tr += (yp[0] - yp[-1]) + (ym[0] - ym[-1]);
-                const float D = acc + w[8] * tr;
-                const float qq1 = R.b1[ax] * R.ph1[1] + R.a1[ax] * D;
-                const float qq2 = R.b2[ax] * R.ph2[1] + R.a2[ax] * D;
+                const float D = __builtin_fmaf(w[8], tr, acc);
+                const float qq1 = memory_step(R.b1[ax], R.ph1[1], R.a1[ax], D);
+                const float qq2 = memory_step(R.b2[ax], R.ph2[1], R.a2[ax], D);
                 gstnt(s.phi[1][0], c, qq1);
                 gstnt(s.phi[1][1], c, qq2);
-                div += D * R.ik[ax] + (qq1 + qq2);
+                div += corrected(D, R.ik[ax], qq1, qq2);
             }
-            gst32(s.p, c, R.p - s.dt * R.K * div);
+            gst32(s.p, c, pressure_step(R.p, s.dt, R.K, div));
         }
     };
 

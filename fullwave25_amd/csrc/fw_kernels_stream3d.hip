@@ -101,53 +101,50 @@ __global__ __launch_bounds__(TZ * TY) void k_velocity_3d(DevSim batch, int chunk
                 const float* w = coef3<UNIFORM>(coefs, s.dcmap, c, 0);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (q[7 + m] - q[8 - m]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], q[7 + m], q[8 - m]);
                 float tr = 0.f;
                 tr += (A(pp, 1, 0) - A(p0, 1, 0)) + (A(pp, -1, 0) - A(p0, -1, 0));
                 tr += (A(pp, 0, 1) - A(p0, 0, 1)) + (A(pp, 0, -1) - A(p0, 0, -1));
-                const float D = acc + w[8] * tr;
-                const float qq1 = s.bv[0][0][c] * s.psi[0][0][c] + s.av[0][0][c] * D;
-                const float qq2 = s.bv[0][1][c] * s.psi[0][1][c] + s.av[0][1][c] * D;
+                const float D = __builtin_fmaf(w[8], tr, acc);
+                const float qq1 = memory_step(s.bv[0][0][c], s.psi[0][0][c], s.av[0][0][c], D);
+                const float qq2 = memory_step(s.bv[0][1][c], s.psi[0][1][c], s.av[0][1][c], D);
                 s.psi[0][0][c] = qq1;
                 s.psi[0][1][c] = qq2;
-                const float rho_bar = 0.5f * (rho_i + rho_next);
-                s.v[0][c] -= s.dt / rho_bar * (D * s.ikv[0][c] + (qq1 + qq2));
+                s.v[0][c] = velocity_step(s.v[0][c], s.dt, rho_i, rho_next, corrected(D, s.ikv[0][c], qq1, qq2));
             }
             // y
             {
                 const float* w = coef3<UNIFORM>(coefs, s.dcmap, c, 1);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (A(p0, m, 0) - A(p0, -(m - 1), 0));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], A(p0, m, 0), A(p0, -(m - 1), 0));
                 float tr = 0.f;
                 tr += (A(pp, 1, 0) - A(pp, 0, 0)) + (A(pm, 1, 0) - A(pm, 0, 0));
                 tr += (A(p0, 1, 1) - A(p0, 0, 1)) + (A(p0, 1, -1) - A(p0, 0, -1));
-                const float D = acc + w[8] * tr;
+                const float D = __builtin_fmaf(w[8], tr, acc);
                 const int ax = ISO ? 0 : 1;
-                const float qq1 = s.bv[ax][0][c] * s.psi[1][0][c] + s.av[ax][0][c] * D;
-                const float qq2 = s.bv[ax][1][c] * s.psi[1][1][c] + s.av[ax][1][c] * D;
+                const float qq1 = memory_step(s.bv[ax][0][c], s.psi[1][0][c], s.av[ax][0][c], D);
+                const float qq2 = memory_step(s.bv[ax][1][c], s.psi[1][1][c], s.av[ax][1][c], D);
                 s.psi[1][0][c] = qq1;
                 s.psi[1][1][c] = qq2;
-                const float rho_bar = 0.5f * (rho_i + s.rho[c + sy]);
-                s.v[1][c] -= s.dt / rho_bar * (D * s.ikv[ax][c] + (qq1 + qq2));
+                s.v[1][c] = velocity_step(s.v[1][c], s.dt, rho_i, s.rho[c + sy], corrected(D, s.ikv[ax][c], qq1, qq2));
             }
             // z
             {
                 const float* w = coef3<UNIFORM>(coefs, s.dcmap, c, 2);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (A(p0, 0, m) - A(p0, 0, -(m - 1)));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], A(p0, 0, m), A(p0, 0, -(m - 1)));
                 float tr = 0.f;
                 tr += (A(pp, 0, 1) - A(pp, 0, 0)) + (A(pm, 0, 1) - A(pm, 0, 0));
                 tr += (A(p0, 1, 1) - A(p0, 1, 0)) + (A(p0, -1, 1) - A(p0, -1, 0));
-                const float D = acc + w[8] * tr;
+                const float D = __builtin_fmaf(w[8], tr, acc);
                 const int ax = ISO ? 0 : 2;
-                const float qq1 = s.bv[ax][0][c] * s.psi[2][0][c] + s.av[ax][0][c] * D;
-                const float qq2 = s.bv[ax][1][c] * s.psi[2][1][c] + s.av[ax][1][c] * D;
+                const float qq1 = memory_step(s.bv[ax][0][c], s.psi[2][0][c], s.av[ax][0][c], D);
+                const float qq2 = memory_step(s.bv[ax][1][c], s.psi[2][1][c], s.av[ax][1][c], D);
                 s.psi[2][0][c] = qq1;
                 s.psi[2][1][c] = qq2;
-                const float rho_bar = 0.5f * (rho_i + s.rho[c + 1]);
-                s.v[2][c] -= s.dt / rho_bar * (D * s.ikv[ax][c] + (qq1 + qq2));
+                s.v[2][c] = velocity_step(s.v[2][c], s.dt, rho_i, s.rho[c + 1], corrected(D, s.ikv[ax][c], qq1, qq2));
             }
         }
         rho_i = rho_next;
@@ -213,50 +210,50 @@ __global__ __launch_bounds__(TZ * TY) void k_pressure_3d(DevSim batch, int chunk
                 const float* w = coef3<UNIFORM>(coefs, s.dcmap, c, 0);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (q[7 + m] - q[8 - m]);
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], q[7 + m], q[8 - m]);
                 float tr = 0.f;
                 tr += (X(x0, 1, 0) - X(xm, 1, 0)) + (X(x0, -1, 0) - X(xm, -1, 0));
                 tr += (X(x0, 0, 1) - X(xm, 0, 1)) + (X(x0, 0, -1) - X(xm, 0, -1));
-                const float D = acc + w[8] * tr;
-                const float qq1 = s.bp[0][0][c] * s.phi[0][0][c] + s.ap[0][0][c] * D;
-                const float qq2 = s.bp[0][1][c] * s.phi[0][1][c] + s.ap[0][1][c] * D;
+                const float D = __builtin_fmaf(w[8], tr, acc);
+                const float qq1 = memory_step(s.bp[0][0][c], s.phi[0][0][c], s.ap[0][0][c], D);
+                const float qq2 = memory_step(s.bp[0][1][c], s.phi[0][1][c], s.ap[0][1][c], D);
                 s.phi[0][0][c] = qq1;
                 s.phi[0][1][c] = qq2;
-                div += D * s.ikp[0][c] + (qq1 + qq2);
+                div += corrected(D, s.ikp[0][c], qq1, qq2);
             }
             {
                 const float* w = coef3<UNIFORM>(coefs, s.dcmap, c, 1);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (Y(y0, m - 1, 0) - Y(y0, -m, 0));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], Y(y0, m - 1, 0), Y(y0, -m, 0));
                 float tr = 0.f;
                 tr += (Y(yp, 0, 0) - Y(yp, -1, 0)) + (Y(ym, 0, 0) - Y(ym, -1, 0));
                 tr += (Y(y0, 0, 1) - Y(y0, -1, 1)) + (Y(y0, 0, -1) - Y(y0, -1, -1));
-                const float D = acc + w[8] * tr;
+                const float D = __builtin_fmaf(w[8], tr, acc);
                 const int ax = ISO ? 0 : 1;
-                const float qq1 = s.bp[ax][0][c] * s.phi[1][0][c] + s.ap[ax][0][c] * D;
-                const float qq2 = s.bp[ax][1][c] * s.phi[1][1][c] + s.ap[ax][1][c] * D;
+                const float qq1 = memory_step(s.bp[ax][0][c], s.phi[1][0][c], s.ap[ax][0][c], D);
+                const float qq2 = memory_step(s.bp[ax][1][c], s.phi[1][1][c], s.ap[ax][1][c], D);
                 s.phi[1][0][c] = qq1;
                 s.phi[1][1][c] = qq2;
-                div += D * s.ikp[ax][c] + (qq1 + qq2);
+                div += corrected(D, s.ikp[ax][c], qq1, qq2);
             }
             {
                 const float* w = coef3<UNIFORM>(coefs, s.dcmap, c, 2);
                 float acc = 0.f;
 #pragma unroll
-                for (int m = 1; m <= 8; ++m) acc += w[m - 1] * (Z(z0, 0, m - 1) - Z(z0, 0, -m));
+                for (int m = 1; m <= 8; ++m) acc = tap(acc, w[m - 1], Z(z0, 0, m - 1), Z(z0, 0, -m));
                 float tr = 0.f;
                 tr += (Z(zp, 0, 0) - Z(zp, 0, -1)) + (Z(zm, 0, 0) - Z(zm, 0, -1));
                 tr += (Z(z0, 1, 0) - Z(z0, 1, -1)) + (Z(z0, -1, 0) - Z(z0, -1, -1));
-                const float D = acc + w[8] * tr;
+                const float D = __builtin_fmaf(w[8], tr, acc);
                 const int ax = ISO ? 0 : 2;
-                const float qq1 = s.bp[ax][0][c] * s.phi[2][0][c] + s.ap[ax][0][c] * D;
-                const float qq2 = s.bp[ax][1][c] * s.phi[2][1][c] + s.ap[ax][1][c] * D;
+                const float qq1 = memory_step(s.bp[ax][0][c], s.phi[2][0][c], s.ap[ax][0][c], D);
+                const float qq2 = memory_step(s.bp[ax][1][c], s.phi[2][1][c], s.ap[ax][1][c], D);
                 s.phi[2][0][c] = qq1;
                 s.phi[2][1][c] = qq2;
-                div += D * s.ikp[ax][c] + (qq1 + qq2);
+                div += corrected(D, s.ikp[ax][c], qq1, qq2);
             }
-            s.p[c] -= s.dt * s.K[c] * div;
+            s.p[c] = pressure_step(s.p[c], s.dt, s.K[c], div);
         }
     }
 }

@@ -1,12 +1,25 @@
 // Tiled 2D kernels with 4-wide vector access (gfx950).
 //
-// A workgroup of 256 lanes (4 wavefronts) owns a tile of TX rows x 256 columns. It first stages
-// the input field(s) of the tile plus the stencil halo into LDS with 16-byte loads, then every
-// lane computes 4 consecutive cells (one float4 column quad) on TX / 4 rows. All per-cell maps
-// and memory variables move as float4 (one 16-byte load or store per quad), which is what lets
-// the HBM stream approach the copy-kernel rate; the stencil operands come from LDS. Rows of a
-// tile are independent once the tile is staged, so each lane issues the loads of all its rows
-// without waiting at barriers.
+// A workgroup of 256 lanes (4 wavefronts) owns a tile of TX rows x TW columns. It stages the input
+// field(s) of the tile plus the stencil halo into LDS with 16-byte loads, then every lane updates
+// 4 consecutive cells (one float4 column quad) a pass. All per-cell maps and memory variables
+// move as float4, which is what lets the HBM stream approach the copy-kernel rate; the stencil
+// operands come from LDS.
+//
+// What bounds it, and why it is laid out so (us a step, velocity + pressure, 4256 x 2208 / 1152^2 /
+// 672^2 cells, coded coefficients):
+//   * large grids stream at the rate of a 9-read, 6-write probe (5.8 TB/s); small ones wait for
+//     memory: a chain of code -> table row -> arithmetic -> store per workgroup, with too few
+//     workgroups to hide it. So the staging loads, the first pass's operands and the table row
+//     are all issued before the first of them is waited for, and the tiles are small (1024 or 2048
+//     cells): 185 / 42 / 27 -> 183 / 34.4 / 18.0 against 256-column tiles staged by a loop of
+//     load, wait and store.
+//   * tiles nearer to square stage fewer halo cells: 2.1-3.2 staged cells of p per updated one
+//     instead of 2.1-3.1 of tiles four times as wide, at half or a quarter of the cells a
+//     workgroup.
+//   * a row gather of each cell's coefficients costs 13 % of the velocity kernel. Media are
+//     piecewise constant, so most wavefronts hold one code: those read the row and the stencil
+//     weights once with scalar loads (WaveCoef): 183 -> 177 at 4256 x 2208.
 //
 // Requires ny % 4 == 0 (16-byte aligned rows). Arithmetic order is the per-cell kernels'.
 #include "fw_internal.h"
@@ -15,9 +28,17 @@ namespace fw {
 
 namespace {
 
-constexpr int kTW = 256;        // columns per tile
-constexpr int kLanes = 256;     // threads per workgroup
-constexpr int kQuads = kTW / 4; // column quads per tile row (64: one wavefront)
+constexpr int kLanes = 256;  // threads per workgroup
+
+// A tile shape: TX rows x TW columns, updated in passes of kRows rows (each lane one quad a pass).
+template <int TW_, int TX_>
+struct Shape {
+    static constexpr int TW = TW_, TX = TX_;
+    static constexpr int kQuads = TW / 4;           // column quads per tile row
+    static constexpr int kRows = kLanes / kQuads;   // tile rows per pass
+    static constexpr int kPasses = TX / kRows;
+    static_assert(TX % kRows == 0, "whole passes");
+};
 
 struct alignas(16) F4 {
     float x, y, z, w;
@@ -125,27 +146,50 @@ __device__ inline uint2 quad_codes(const DevSim& s, int64_t i, int64_t jq) {
 // same stencil offset) they touch consecutive words: the LDS serves these single-float reads
 // without bank conflicts, where a row-major tile (lanes 4 floats apart) conflicts four ways.
 //
-// Stage rows [r0, r0 + nrows) x columns [j0 - hl, j0 + kTW + hr) of f into lds (tile column 0
-// is j0 - hl). hl and hr are multiples of 4; ny % 4 == 0, so every quad is either entirely
-// inside [0, ny) or entirely outside (then zero). Rows outside [0, nx) are zero.
-__device__ inline void stage_tile(float* lds, const float* __restrict__ f, int64_t r0, int nrows, int64_t j0,
-                                  int hl, int hr, int pitch, int64_t nx, int64_t ny) {
-    const int qpr = (kTW + hl + hr) / 4;  // quads per row
-    const int total = nrows * qpr;
-    for (int t = threadIdx.x; t < total; t += kLanes) {
-        const int row = t / qpr, qd = t - row * qpr;
-        const int64_t r = r0 + row;
-        const int64_t jj = j0 - hl + 4 * qd;
-        F4 v{0.f, 0.f, 0.f, 0.f};
-        if (r >= 0 && r < nx && jj >= 0 && jj < ny) v = ld4(f, (uint32_t)(r * ny + jj));
-        float* dst = lds + row * pitch + qd;
-        const int plane = pitch / 4;
-        dst[0] = v.x;
-        dst[plane] = v.y;
-        dst[2 * plane] = v.z;
-        dst[3 * plane] = v.w;
+// The staged region of one field: NROWS rows x (TW + HL + HR) columns in rows of PITCH floats
+// (pitch mod 32 keeps the rows that one half of a wavefront reads on different banks). Each lane owns
+// fixed quads of it and issues all of their loads (load) before it stores any (store), so the
+// staging takes one memory latency: looping over load-and-store took one per quad, 7 in a row for
+// the 23 x 272 tile of a pressure workgroup.
+template <int TW, int NROWS_, int HL_, int HR_>
+struct Staged {
+    static constexpr int NROWS = NROWS_, HL = HL_;
+    static constexpr int QPR = (TW + HL_ + HR_) / 4;       // quads per row
+    static constexpr int MOD = TW >= 128 ? 0 : TW == 64 ? 16 : 24;
+    static constexpr int PITCH = TW >= 128 ? 4 * QPR : (4 * QPR - MOD + 31) / 32 * 32 + MOD;
+    static constexpr int PLANE = PITCH / 4;
+    static constexpr int NQ = NROWS * QPR;
+    static constexpr int NL = (NQ + kLanes - 1) / kLanes;  // quads per lane
+    float v[NROWS * PITCH];
+};
+template <class T>
+struct StageRegs {
+    F4 q[T::NL];
+    // Rows [r0, r0 + NROWS) x columns [j0 - HL, ...) of f; quads outside the grid (no updated cell's
+    // stencil reaches one) repeat the nearest one, so that the loads need no branch.
+    __device__ inline void load(const float* __restrict__ f, int r0, int j0, int nx, int ny) {
+#pragma unroll
+        for (int l = 0; l < T::NL; ++l) {
+            const int t = min((int)threadIdx.x + l * kLanes, T::NQ - 1);
+            const int row = t / T::QPR, qd = t - row * T::QPR;
+            const int r = min(max(r0 + row, 0), nx - 1), jj = min(max(j0 - T::HL + 4 * qd, 0), ny - 4);
+            q[l] = ld4(f, (uint32_t)(r * ny + jj));
+        }
     }
-}
+    __device__ inline void store(T& tile) const {
+#pragma unroll
+        for (int l = 0; l < T::NL; ++l) {
+            const int t = threadIdx.x + l * kLanes;
+            const int row = t / T::QPR, qd = t - row * T::QPR;
+            if (l == T::NL - 1 && t >= T::NQ) continue;
+            float* dst = tile.v + row * T::PITCH + qd;
+            dst[0] = q[l].x;
+            dst[T::PLANE] = q[l].y;
+            dst[2 * T::PLANE] = q[l].z;
+            dst[3 * T::PLANE] = q[l].w;
+        }
+    }
+};
 
 // Element at row offset dr and column offset dc from tile row `row` of the lane's quad base
 // `lb` (= lds + row * pitch + qd): K = hl + e + dc is the column within the quad grid (hl + e
@@ -157,13 +201,13 @@ __device__ inline float tl(const float* lb, int dr, int col) {
 }
 
 // LDS coefficient sets: [set][axis][kCS], or [set][kCS] when both axes share their sets (equal
-// spacings; `axes` = 1), which halves the table and lets one more workgroup fit on a CU. Each
-// set of 9 weights is padded to 12 floats, so a cell reads its weights as two 16-byte loads
-// and one 4-byte load.
+// spacings; SAME), which halves the table, lets one more workgroup fit on a CU, and lets a cell read
+// its weights once for both axes. Each set of 9 weights is padded to 12 floats, so a cell reads
+// them as two 16-byte loads and one 4-byte load.
 constexpr int kCS = 12;
-template <bool UNIFORM>
-__device__ inline const float* cset(const float* lds_coef, int dc, int axis, int axes) {
-    return lds_coef + ((UNIFORM ? 0 : dc) * axes + (axes > 1 ? axis : 0)) * kCS;
+template <bool UNIFORM, bool SAME>
+__device__ inline const float* cset(const float* lds_coef, int dc, int axis) {
+    return lds_coef + ((UNIFORM ? 0 : dc) * (SAME ? 1 : 2) + (SAME ? 0 : axis)) * kCS;
 }
 
 struct W9 {
@@ -175,276 +219,405 @@ __device__ inline W9 weights(const float* c) {
 }
 
 // Stage the coefficient sets into LDS (all axes, or axis 0 only when they are the same).
-template <bool UNIFORM>
-__device__ inline int stage_coef(float* lds_coef, const DevSim& s) {
-    const int axes = s.coef_axes_same ? 1 : 2;
-    const int nsets = UNIFORM ? 1 : s.ndmap;
-    for (int t = threadIdx.x; t < nsets * axes * kNCoef; t += kLanes) {
-        const int set = t / kNCoef, k = t - set * kNCoef;  // set: (sound speed) * axes + axis
-        lds_coef[set * kCS + k] = s.coef[(axes == 2 ? set : set * 2) * kNCoef + k];
+template <bool UNIFORM, bool SAME>
+__device__ inline void stage_coef(float* lds_coef, const DevSim& s) {
+    constexpr int axes = SAME ? 1 : 2;
+    const int n = (UNIFORM ? 1 : s.ndmap) * axes * kNCoef;
+    for (int t0 = 0; t0 < n; t0 += 4 * kLanes) {  // four loads in flight a lane
+        float v[4];
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const int t = t0 + l * kLanes + threadIdx.x, set = t / kNCoef, k = t - set * kNCoef;
+            v[l] = t < n ? s.coef[(SAME ? set * 2 : set) * kNCoef + k] : 0.f;
+        }
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const int t = t0 + l * kLanes + threadIdx.x, set = t / kNCoef, k = t - set * kNCoef;
+            if (t < n) lds_coef[set * kCS + k] = v[l];
+        }
     }
-    return axes;
 }
 
-// velocity: p tile rows i0-7 .. i0+TX+7 (TX + 15 rows), columns j0-8 .. j0+TW+8
-template <int TX>
-struct VelTile {
-    static constexpr int PITCH = kTW + 16;
-    static constexpr int NROWS = TX + 15;
-    float P[NROWS * PITCH];
+// The coefficients of one quad as the arithmetic reads them. QuadCoef: each cell its own, in vector
+// registers, with its weights from LDS.
+template <bool UNIFORM, bool ISO, bool SAME>
+struct QuadCoef {
+    static constexpr int NA = ISO ? 1 : 2;
+    F4 ik_[NA], b1_[NA], b2_[NA], a1_[NA], a2_[NA];
+    I4 dc;
+    __device__ float ik(int a, int e) const { return ik_[ISO ? 0 : a][e]; }
+    __device__ float a1(int a, int e) const { return a1_[ISO ? 0 : a][e]; }
+    __device__ float a2(int a, int e) const { return a2_[ISO ? 0 : a][e]; }
+    __device__ float b1(int a, int e) const { return b1_[ISO ? 0 : a][e]; }
+    __device__ float b2(int a, int e) const { return b2_[ISO ? 0 : a][e]; }
+    __device__ W9 w(const DevSim&, const float* lds_coef, int a, int e) const {
+        return weights(cset<UNIFORM, SAME>(lds_coef, dc[e], a));
+    }
+};
+// WaveCoef: every cell of the wavefront has the same code, so the row and the weights are read once
+// with scalar loads and stay in scalar registers.
+typedef const __attribute__((address_space(4))) float* scalar_ptr;
+__device__ inline scalar_ptr as_scalar(const float* p) { return (scalar_ptr)(uintptr_t)p; }
+template <bool UNIFORM, bool SAME>
+struct WaveCoef {
+    float ik_, a1_, a2_, b1_, b2_;
+    int dc;
+    __device__ float ik(int, int) const { return ik_; }
+    __device__ float a1(int, int) const { return a1_; }
+    __device__ float a2(int, int) const { return a2_; }
+    __device__ float b1(int, int) const { return b1_; }
+    __device__ float b2(int, int) const { return b2_; }
+    __device__ W9 w(const DevSim& s, const float*, int a, int) const {
+        const scalar_ptr c = as_scalar(s.coef) + ((UNIFORM ? 0 : dc * 2) + (SAME ? 0 : a)) * kNCoef;
+        W9 r;
+#pragma unroll
+        for (int k = 0; k < kNCoef; ++k) r.w[k] = c[k];
+        return r;
+    }
+    // the values again as the (active) lanes' common ones: across a branch the compiler takes them for
+    // per-lane values
+    __device__ void rejoin() {
+        for (float* f : {&ik_, &a1_, &a2_, &b1_, &b2_}) *f = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(*f)));
+        dc = __builtin_amdgcn_readfirstlane(dc);
+    }
+    __device__ void load(const float* tab, uint32_t code) {
+        const scalar_ptr row = as_scalar(tab) + code * kCodeStride;
+        ik_ = row[0];
+        a1_ = row[1];
+        a2_ = row[2];
+        b1_ = row[3];
+        b2_ = row[4];
+        dc = __float_as_int(row[5]);
+    }
 };
 
-// The velocity update of tile (bx, by) of grid s: columns [bx * 256, bx * 256 + 256), rows
-// [8 + by * TX, 8 + by * TX + TX). TAPE: also the adjoint tape (DevSim::tape_u; 0 in the ghost
-// columns of a quad).
-template <int TX, bool UNIFORM, bool ISO, bool CODED, bool TAPE = false>
-__device__ inline void velocity_tile(const DevSim& s, unsigned bx, unsigned by, VelTile<TX>& L, float* lds_coef) {
-    constexpr int PITCH = VelTile<TX>::PITCH;
-    constexpr int NROWS = VelTile<TX>::NROWS;
-    float* P = L.P;
+// Whether all the quads of this wavefront's active lanes (`cw`: a lane's four codes) have one code
+// that is not the escape; `code` is it then.
+__device__ inline bool wave_code(uint2 cw, uint32_t* code) {
+    const uint32_t c0 = __builtin_amdgcn_readfirstlane(cw.x);
+    *code = c0 & 0xffffu;
+    return (c0 >> 16) == *code && *code != kCodeEscape && __all(cw.x == c0 && cw.y == c0);
+}
+
+// velocity: p rows i0-7 .. i0+TX+7, columns j0-8 .. j0+TW+7
+template <class S>
+struct VelTile {
+    using P = Staged<S::TW, S::TX + 15, 8, 8>;
+    P p;
+};
+
+// operands of one quad of the velocity update
+struct VelQuad {
+    F4 rho0, rho1, ps1[2], ps2[2], v[2];
+    float rho_r;
+};
+
+__device__ inline void load_vel_quad(const DevSim& s, VelQuad& o, uint32_t c) {
+    o.rho0 = ld4(s.rho, c);
+    o.rho1 = ld4(s.rho, c + (uint32_t)s.ny);
+    o.rho_r = ld1(s.rho, c + 4);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        o.ps1[a] = ld4nt(s.psi[a][0], c);
+        o.ps2[a] = ld4nt(s.psi[a][1], c);
+        o.v[a] = ld4(s.v[a], c);
+    }
+}
+
+// The velocity update of the quad at element c with coefficients k; lb: its base in the staged p.
+template <int PITCH, bool SAME, bool TAPE, class Coef>
+__device__ inline void velocity_quad(const DevSim& s, uint32_t c, VelQuad& o, const Coef& k, const float* lb,
+                                     const float* lds_coef) {
+    const float dt = s.dt;
+    auto pa = [&](int e, int dr, int dc_) { return tl<PITCH, 8>(lb, dr, e + dc_); };
+    F4 tu[2];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        W9 wv = k.w(s, lds_coef, 0, e);
+        {
+            float acc = 0.f;
+#pragma unroll
+            for (int m = 1; m <= 8; ++m) acc = tap(acc, wv.w[m - 1], pa(e, m, 0), pa(e, -(m - 1), 0));
+            float tr = 0.f;
+            tr += (pa(e, 1, 1) - pa(e, 0, 1)) + (pa(e, 1, -1) - pa(e, 0, -1));
+            const float D = __builtin_fmaf(wv.w[8], tr, acc);
+            const float q1 = memory_step(k.b1(0, e), o.ps1[0][e], k.a1(0, e), D);
+            const float q2 = memory_step(k.b2(0, e), o.ps2[0][e], k.a2(0, e), D);
+            o.ps1[0][e] = q1;
+            o.ps2[0][e] = q2;
+            const float u = corrected(D, k.ik(0, e), q1, q2);
+            o.v[0][e] = velocity_step(o.v[0][e], dt, o.rho0[e], o.rho1[e], u);
+            if (TAPE) tu[0][e] = u;
+        }
+        {
+            if (!SAME) wv = k.w(s, lds_coef, 1, e);
+            float acc = 0.f;
+#pragma unroll
+            for (int m = 1; m <= 8; ++m) acc = tap(acc, wv.w[m - 1], pa(e, 0, m), pa(e, 0, -(m - 1)));
+            float tr = 0.f;
+            tr += (pa(e, 1, 1) - pa(e, 1, 0)) + (pa(e, -1, 1) - pa(e, -1, 0));
+            const float D = __builtin_fmaf(wv.w[8], tr, acc);
+            const float q1 = memory_step(k.b1(1, e), o.ps1[1][e], k.a1(1, e), D);
+            const float q2 = memory_step(k.b2(1, e), o.ps2[1][e], k.a2(1, e), D);
+            o.ps1[1][e] = q1;
+            o.ps2[1][e] = q2;
+            const float rho_right = e < 3 ? o.rho0[e + 1] : o.rho_r;
+            const float u = corrected(D, k.ik(1, e), q1, q2);
+            o.v[1][e] = velocity_step(o.v[1][e], dt, o.rho0[e], rho_right, u);
+            if (TAPE) tu[1][e] = u;
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        st4nt(s.psi[a][0], c, o.ps1[a]);
+        st4nt(s.psi[a][1], c, o.ps2[a]);
+        st4(s.v[a], c, o.v[a]);
+        if (TAPE) st4(s.tape_u[a], c, tu[a]);
+    }
+}
+
+// The velocity update of tile (bx, by) of grid s: columns [bx * TW, bx * TW + TW), rows
+// [8 + by * TX, 8 + by * TX + TX). TAPE: also the adjoint tape (DevSim::tape_u). The ghost border is
+// two quads wide and ny % 4 == 0, so a quad is updated whole or not at all: its four cells run
+// as one straight line of code, which shares the columns that their stencils read (a test per cell
+// kept them apart: 144 LDS words a quad and axis pair instead of 93, and no overlap between cells).
+template <class S, bool UNIFORM, bool ISO, bool CODED, bool SAME, bool TAPE = false>
+__device__ inline void velocity_tile(const DevSim& s, unsigned bx, unsigned by, VelTile<S>& L, float* lds_coef) {
+    using T = typename VelTile<S>::P;
     const int64_t nx = s.nx, ny = s.ny;
-    const int64_t j0 = (int64_t)bx * kTW;
-    const int64_t i0 = kHalo + (int64_t)by * TX;
-    const int qd = threadIdx.x % kQuads;
-    const int ty = threadIdx.x / kQuads;
+    const int64_t j0 = (int64_t)bx * S::TW;
+    const int64_t i0 = kHalo + (int64_t)by * S::TX;
+    const int qd = threadIdx.x % S::kQuads;
+    const int ty = threadIdx.x / S::kQuads;
     const int64_t jq = j0 + 4 * qd;  // first column of this lane's quad
-    uint2 cw_next = jq < ny ? quad_codes<CODED>(s, i0 + ty, jq) : uint2{0u, 0u};
-    const int axes = stage_coef<UNIFORM>(lds_coef, s);
-    stage_tile(P, s.p, i0 - 7, NROWS, j0, 8, 8, PITCH, nx, ny);
+    const bool active = jq >= kHalo && jq < ny - kHalo;
+    uint2 cw = active ? quad_codes<CODED>(s, i0 + ty, jq) : uint2{0u, 0u};
+    StageRegs<T> st;
+    st.load(s.p, (int)i0 - 7, (int)j0, (int)nx, (int)ny);
+    VelQuad o;
+    QuadCoef<UNIFORM, ISO, SAME> kq;
+    WaveCoef<UNIFORM, SAME> kw;
+    bool wave = false;
+    auto load_coef = [&](uint32_t c) {
+        uint32_t code = 0;
+        wave = CODED && wave_code(cw, &code);
+        if (wave) kw.load(s.rtab_v, code);
+        else quad_coef<CODED, UNIFORM, true, QuadCoef<UNIFORM, ISO, SAME>::NA>(s, c, cw, kq.ik_, kq.b1_, kq.b2_, kq.a1_, kq.a2_, kq.dc);
+    };
+    if (active && i0 + ty < nx - kHalo) {
+        const uint32_t c = (uint32_t)((i0 + ty) * ny + jq);
+        load_vel_quad(s, o, c);
+        load_coef(c);
+    }
+    stage_coef<UNIFORM, SAME>(lds_coef, s);
+    st.store(L.p);
     __syncthreads();
 
-    if (jq >= ny) return;
-    const float dt = s.dt;
+    if (!active) return;
 #pragma unroll 1
-    for (int m = 0; m < TX / 4; ++m) {
-        const int lr = ty + 4 * m;  // row within the tile
+    for (int m = 0; m < S::kPasses; ++m) {
+        const int lr = ty + S::kRows * m;  // row within the tile
         const int64_t i = i0 + lr;
         if (i >= nx - kHalo) break;
         const uint32_t c = (uint32_t)(i * ny + jq);
-        const uint2 cw = cw_next;
-        if (m + 1 < TX / 4) cw_next = quad_codes<CODED>(s, i + 4, jq);
-        const F4 rho0 = ld4(s.rho, c);
-        const F4 rho1 = ld4(s.rho, c + (uint32_t)ny);
-        const float rho_r = (jq + 4 < ny) ? ld1(s.rho, c + 4) : 0.f;
-        I4 dc;
-        F4 ik[2], b1[2], b2[2], a1[2], a2[2];
-        constexpr int NA = ISO ? 1 : 2;
-        quad_coef<CODED, UNIFORM, true, NA>(s, c, cw, ik, b1, b2, a1, a2, dc);
-        F4 ps1[2], ps2[2], v[2];
-        F4 tu[2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            if (TAPE) tu[a] = F4{0.f, 0.f, 0.f, 0.f};
-            ps1[a] = ld4nt(s.psi[a][0], c);
-            ps2[a] = ld4nt(s.psi[a][1], c);
-            v[a] = ld4(s.v[a], c);
+        if (m > 0) {
+            load_vel_quad(s, o, c);
+            load_coef(c);
         }
+        if (m + 1 < S::kPasses) cw = quad_codes<CODED>(s, i + S::kRows, jq);
         // LDS row of tile row lr is lr + 7; column j is tile column j - j0 + 8
-        const float* lb = P + (lr + 7) * PITCH + qd;
-        auto pa = [&](int e, int dr, int dc_) { return tl<PITCH, 8>(lb, dr, e + dc_); };
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int64_t j = jq + e;
-            if (j < kHalo || j >= ny - kHalo) continue;
-            {
-                const W9 wv = weights(cset<UNIFORM>(lds_coef, dc[e], 0, axes));
-                float acc = 0.f;
-#pragma unroll
-                for (int k = 1; k <= 8; ++k) acc += wv.w[k - 1] * (pa(e, k, 0) - pa(e, -(k - 1), 0));
-                float tr = 0.f;
-                tr += (pa(e, 1, 1) - pa(e, 0, 1)) + (pa(e, 1, -1) - pa(e, 0, -1));
-                const float D = acc + wv.w[8] * tr;
-                const float q1 = b1[0][e] * ps1[0][e] + a1[0][e] * D;
-                const float q2 = b2[0][e] * ps2[0][e] + a2[0][e] * D;
-                ps1[0][e] = q1;
-                ps2[0][e] = q2;
-                const float rho_bar = 0.5f * (rho0[e] + rho1[e]);
-                const float u = D * ik[0][e] + (q1 + q2);
-                v[0][e] -= dt / rho_bar * u;
-                if (TAPE) tu[0][e] = u;
-            }
-            {
-                constexpr int ax = ISO ? 0 : 1;
-                const W9 wv = weights(cset<UNIFORM>(lds_coef, dc[e], 1, axes));
-                float acc = 0.f;
-#pragma unroll
-                for (int k = 1; k <= 8; ++k) acc += wv.w[k - 1] * (pa(e, 0, k) - pa(e, 0, -(k - 1)));
-                float tr = 0.f;
-                tr += (pa(e, 1, 1) - pa(e, 1, 0)) + (pa(e, -1, 1) - pa(e, -1, 0));
-                const float D = acc + wv.w[8] * tr;
-                const float q1 = b1[ax][e] * ps1[1][e] + a1[ax][e] * D;
-                const float q2 = b2[ax][e] * ps2[1][e] + a2[ax][e] * D;
-                ps1[1][e] = q1;
-                ps2[1][e] = q2;
-                const float rho_right = e < 3 ? rho0[e + 1] : rho_r;
-                const float rho_bar = 0.5f * (rho0[e] + rho_right);
-                const float u = D * ik[ax][e] + (q1 + q2);
-                v[1][e] -= dt / rho_bar * u;
-                if (TAPE) tu[1][e] = u;
-            }
-        }
-        // cells outside the active columns keep their loaded values, so whole quads store back
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            st4nt(s.psi[a][0], c, ps1[a]);
-            st4nt(s.psi[a][1], c, ps2[a]);
-            st4(s.v[a], c, v[a]);
-            if (TAPE) st4(s.tape_u[a], c, tu[a]);
+        const float* lb = L.p.v + (lr + 7) * T::PITCH + qd;
+        if (CODED && __builtin_amdgcn_readfirstlane(wave)) {
+            kw.rejoin();
+            velocity_quad<T::PITCH, SAME, TAPE>(s, c, o, kw, lb, lds_coef);
+        } else {
+            velocity_quad<T::PITCH, SAME, TAPE>(s, c, o, kq, lb, lds_coef);
         }
     }
 }
 
-// pressure: vx tile rows i0-8 .. i0+TX+6 (TX + 15 rows), columns j0-4 .. j0+TW+4;
-//           vy tile rows i0-1 .. i0+TX (TX + 2 rows), columns j0-8 .. j0+TW+8
-template <int TX>
+// pressure: vx rows i0-8 .. i0+TX+6, columns j0-4 .. j0+TW+3;
+//           vy rows i0-1 .. i0+TX, columns j0-8 .. j0+TW+7
+template <class S>
 struct PreTile {
-    static constexpr int XP = kTW + 8;
-    static constexpr int XR = TX + 15;
-    static constexpr int YP = kTW + 16;
-    static constexpr int YR = TX + 2;
-    float VX[XR * XP];
-    float VY[YR * YP];
+    using X = Staged<S::TW, S::TX + 15, 4, 4>;
+    using Y = Staged<S::TW, S::TX + 2, 8, 8>;
+    X x;
+    Y y;
 };
+
+// operands of one quad of the pressure update
+struct PreQuad {
+    F4 p, K, ph1[2], ph2[2];
+};
+
+__device__ inline void load_pre_quad(const DevSim& s, PreQuad& o, uint32_t c) {
+    o.p = ld4(s.p, c);
+    o.K = ld4(s.K, c);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        o.ph1[a] = ld4nt(s.phi[a][0], c);
+        o.ph2[a] = ld4nt(s.phi[a][1], c);
+    }
+}
+
+// The pressure update of the quad at element c; xb, yb: its base in the staged vx and vy.
+template <int XP, int YP, bool SAME, bool TAPE, class Coef>
+__device__ inline void pressure_quad(const DevSim& s, uint32_t c, PreQuad& o, const Coef& k, const float* xb,
+                                     const float* yb, const float* lds_coef) {
+    const float dt = s.dt;
+    auto xa = [&](int e, int dr, int dc_) { return tl<XP, 4>(xb, dr, e + dc_); };
+    auto ya = [&](int e, int dr, int dc_) { return tl<YP, 8>(yb, dr, e + dc_); };
+    F4 td;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float div = 0.f;
+        W9 wv = k.w(s, lds_coef, 0, e);
+        {
+            float acc = 0.f;
+#pragma unroll
+            for (int m = 1; m <= 8; ++m) acc = tap(acc, wv.w[m - 1], xa(e, m - 1, 0), xa(e, -m, 0));
+            float tr = 0.f;
+            tr += (xa(e, 0, 1) - xa(e, -1, 1)) + (xa(e, 0, -1) - xa(e, -1, -1));
+            const float D = __builtin_fmaf(wv.w[8], tr, acc);
+            const float q1 = memory_step(k.b1(0, e), o.ph1[0][e], k.a1(0, e), D);
+            const float q2 = memory_step(k.b2(0, e), o.ph2[0][e], k.a2(0, e), D);
+            o.ph1[0][e] = q1;
+            o.ph2[0][e] = q2;
+            div += corrected(D, k.ik(0, e), q1, q2);
+        }
+        {
+            if (!SAME) wv = k.w(s, lds_coef, 1, e);
+            float acc = 0.f;
+#pragma unroll
+            for (int m = 1; m <= 8; ++m) acc = tap(acc, wv.w[m - 1], ya(e, 0, m - 1), ya(e, 0, -m));
+            float tr = 0.f;
+            tr += (ya(e, 1, 0) - ya(e, 1, -1)) + (ya(e, -1, 0) - ya(e, -1, -1));
+            const float D = __builtin_fmaf(wv.w[8], tr, acc);
+            const float q1 = memory_step(k.b1(1, e), o.ph1[1][e], k.a1(1, e), D);
+            const float q2 = memory_step(k.b2(1, e), o.ph2[1][e], k.a2(1, e), D);
+            o.ph1[1][e] = q1;
+            o.ph2[1][e] = q2;
+            div += corrected(D, k.ik(1, e), q1, q2);
+        }
+        o.p[e] = pressure_step(o.p[e], dt, o.K[e], div);
+        if (TAPE) td[e] = div;
+    }
+    st4(s.p, c, o.p);
+    if (TAPE) st4(s.tape_div, c, td);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        st4nt(s.phi[a][0], c, o.ph1[a]);
+        st4nt(s.phi[a][1], c, o.ph2[a]);
+    }
+}
 
 // The pressure update of tile (bx, by) of grid s (as velocity_tile; TAPE: DevSim::tape_div).
-template <int TX, bool UNIFORM, bool ISO, bool CODED, bool TAPE = false>
-__device__ inline void pressure_tile(const DevSim& s, unsigned bx, unsigned by, PreTile<TX>& L, float* lds_coef) {
-    constexpr int XP = PreTile<TX>::XP;
-    constexpr int XR = PreTile<TX>::XR;
-    constexpr int YP = PreTile<TX>::YP;
-    constexpr int YR = PreTile<TX>::YR;
-    float* VX = L.VX;
-    float* VY = L.VY;
+template <class S, bool UNIFORM, bool ISO, bool CODED, bool SAME, bool TAPE = false>
+__device__ inline void pressure_tile(const DevSim& s, unsigned bx, unsigned by, PreTile<S>& L, float* lds_coef) {
+    using X = typename PreTile<S>::X;
+    using Y = typename PreTile<S>::Y;
     const int64_t nx = s.nx, ny = s.ny;
-    const int64_t j0 = (int64_t)bx * kTW;
-    const int64_t i0 = kHalo + (int64_t)by * TX;
-    const int qd = threadIdx.x % kQuads;
-    const int ty = threadIdx.x / kQuads;
+    const int64_t j0 = (int64_t)bx * S::TW;
+    const int64_t i0 = kHalo + (int64_t)by * S::TX;
+    const int qd = threadIdx.x % S::kQuads;
+    const int ty = threadIdx.x / S::kQuads;
     const int64_t jq = j0 + 4 * qd;
-    uint2 cw_next = jq < ny ? quad_codes<CODED>(s, i0 + ty, jq) : uint2{0u, 0u};
-    const int axes = stage_coef<UNIFORM>(lds_coef, s);
-    stage_tile(VX, s.v[0], i0 - 8, XR, j0, 4, 4, XP, nx, ny);
-    stage_tile(VY, s.v[1], i0 - 1, YR, j0, 8, 8, YP, nx, ny);
+    const bool active = jq >= kHalo && jq < ny - kHalo;
+    uint2 cw = active ? quad_codes<CODED>(s, i0 + ty, jq) : uint2{0u, 0u};
+    StageRegs<X> sx;
+    StageRegs<Y> sy;
+    sx.load(s.v[0], (int)i0 - 8, (int)j0, (int)nx, (int)ny);
+    sy.load(s.v[1], (int)i0 - 1, (int)j0, (int)nx, (int)ny);
+    PreQuad o;
+    QuadCoef<UNIFORM, ISO, SAME> kq;
+    WaveCoef<UNIFORM, SAME> kw;
+    bool wave = false;
+    auto load_coef = [&](uint32_t c) {
+        uint32_t code = 0;
+        wave = CODED && wave_code(cw, &code);
+        if (wave) kw.load(s.rtab_p, code);
+        else quad_coef<CODED, UNIFORM, false, QuadCoef<UNIFORM, ISO, SAME>::NA>(s, c, cw, kq.ik_, kq.b1_, kq.b2_, kq.a1_, kq.a2_, kq.dc);
+    };
+    if (active && i0 + ty < nx - kHalo) {
+        const uint32_t c = (uint32_t)((i0 + ty) * ny + jq);
+        load_pre_quad(s, o, c);
+        load_coef(c);
+    }
+    stage_coef<UNIFORM, SAME>(lds_coef, s);
+    sx.store(L.x);
+    sy.store(L.y);
     __syncthreads();
 
-    if (jq >= ny) return;
-    const float dt = s.dt;
+    if (!active) return;
 #pragma unroll 1
-    for (int m = 0; m < TX / 4; ++m) {
-        const int lr = ty + 4 * m;
+    for (int m = 0; m < S::kPasses; ++m) {
+        const int lr = ty + S::kRows * m;
         const int64_t i = i0 + lr;
         if (i >= nx - kHalo) break;
         const uint32_t c = (uint32_t)(i * ny + jq);
-        const uint2 cw = cw_next;
-        if (m + 1 < TX / 4) cw_next = quad_codes<CODED>(s, i + 4, jq);
-        F4 pv = ld4(s.p, c);
-        const F4 K = ld4(s.K, c);
-        I4 dc;
-        constexpr int NA = ISO ? 1 : 2;
-        F4 ik[2], b1[2], b2[2], a1[2], a2[2];
-        quad_coef<CODED, UNIFORM, false, NA>(s, c, cw, ik, b1, b2, a1, a2, dc);
-        F4 ph1[2], ph2[2];
-        F4 td = F4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            ph1[a] = ld4nt(s.phi[a][0], c);
-            ph2[a] = ld4nt(s.phi[a][1], c);
+        if (m > 0) {
+            load_pre_quad(s, o, c);
+            load_coef(c);
         }
-        const float* xb = VX + (lr + 8) * XP + qd;  // vx(i, .): tile column j - j0 + 4
-        const float* yb = VY + (lr + 1) * YP + qd;  // vy(i, .): tile column j - j0 + 8
-        auto xa = [&](int e, int dr, int dc_) { return tl<XP, 4>(xb, dr, e + dc_); };
-        auto ya = [&](int e, int dr, int dc_) { return tl<YP, 8>(yb, dr, e + dc_); };
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int64_t j = jq + e;
-            if (j < kHalo || j >= ny - kHalo) continue;
-            float div = 0.f;
-            {
-                const W9 wv = weights(cset<UNIFORM>(lds_coef, dc[e], 0, axes));
-                float acc = 0.f;
-#pragma unroll
-                for (int k = 1; k <= 8; ++k) acc += wv.w[k - 1] * (xa(e, k - 1, 0) - xa(e, -k, 0));
-                float tr = 0.f;
-                tr += (xa(e, 0, 1) - xa(e, -1, 1)) + (xa(e, 0, -1) - xa(e, -1, -1));
-                const float D = acc + wv.w[8] * tr;
-                const float q1 = b1[0][e] * ph1[0][e] + a1[0][e] * D;
-                const float q2 = b2[0][e] * ph2[0][e] + a2[0][e] * D;
-                ph1[0][e] = q1;
-                ph2[0][e] = q2;
-                div += D * ik[0][e] + (q1 + q2);
-            }
-            {
-                constexpr int ax = ISO ? 0 : 1;
-                const W9 wv = weights(cset<UNIFORM>(lds_coef, dc[e], 1, axes));
-                float acc = 0.f;
-#pragma unroll
-                for (int k = 1; k <= 8; ++k) acc += wv.w[k - 1] * (ya(e, 0, k - 1) - ya(e, 0, -k));
-                float tr = 0.f;
-                tr += (ya(e, 1, 0) - ya(e, 1, -1)) + (ya(e, -1, 0) - ya(e, -1, -1));
-                const float D = acc + wv.w[8] * tr;
-                const float q1 = b1[ax][e] * ph1[1][e] + a1[ax][e] * D;
-                const float q2 = b2[ax][e] * ph2[1][e] + a2[ax][e] * D;
-                ph1[1][e] = q1;
-                ph2[1][e] = q2;
-                div += D * ik[ax][e] + (q1 + q2);
-            }
-            pv[e] -= dt * K[e] * div;
-            if (TAPE) td[e] = div;
-        }
-        st4(s.p, c, pv);
-        if (TAPE) st4(s.tape_div, c, td);
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            st4nt(s.phi[a][0], c, ph1[a]);
-            st4nt(s.phi[a][1], c, ph2[a]);
+        if (m + 1 < S::kPasses) cw = quad_codes<CODED>(s, i + S::kRows, jq);
+        const float* xb = L.x.v + (lr + 8) * X::PITCH + qd;  // vx(i, .): tile column j - j0 + 4
+        const float* yb = L.y.v + (lr + 1) * Y::PITCH + qd;  // vy(i, .): tile column j - j0 + 8
+        if (CODED && __builtin_amdgcn_readfirstlane(wave)) {
+            kw.rejoin();
+            pressure_quad<X::PITCH, Y::PITCH, SAME, TAPE>(s, c, o, kw, xb, yb, lds_coef);
+        } else {
+            pressure_quad<X::PITCH, Y::PITCH, SAME, TAPE>(s, c, o, kq, xb, yb, lds_coef);
         }
     }
 }
 
-template <int TX, bool UNIFORM, bool ISO, bool CODED, bool TAPE>
+template <class S, bool UNIFORM, bool ISO, bool CODED, bool SAME, bool TAPE>
 __global__ __launch_bounds__(kLanes) void k_velocity_tile(DevSim batch) {
-    __shared__ __attribute__((aligned(16))) VelTile<TX> L;
+    __shared__ __attribute__((aligned(16))) VelTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
-    velocity_tile<TX, UNIFORM, ISO, CODED, TAPE>(shot_view(batch, blockIdx.z), blockIdx.x, blockIdx.y, L, lds_coef);
+    velocity_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>(shot_view(batch, blockIdx.z), blockIdx.x, blockIdx.y, L, lds_coef);
 }
 
 // gs.g non-null: each workgroup then also does the step's source, pressure-release and sensor
 // work of its tile (tile blockIdx.y * gridDim.x + blockIdx.x of shot blockIdx.z), as the group
 // kernels do
-template <int TX, bool UNIFORM, bool ISO, bool CODED, bool TAPE>
+template <class S, bool UNIFORM, bool ISO, bool CODED, bool SAME, bool TAPE>
 __global__ __launch_bounds__(kLanes) void k_pressure_tile(DevSim batch, GroupStep gs) {
-    __shared__ __attribute__((aligned(16))) PreTile<TX> L;
+    __shared__ __attribute__((aligned(16))) PreTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
     TileWork w{};
     if (gs.g) {
         const GroupBoundary& e = gs.g[blockIdx.z];
         w = tile_work(e, blockIdx.y * gridDim.x + blockIdx.x, e.step0 + gs.it + (gs.base ? *gs.base : 0));
     }
-    pressure_tile<TX, UNIFORM, ISO, CODED, TAPE>(shot_view(batch, blockIdx.z), blockIdx.x, blockIdx.y, L, lds_coef);
+    pressure_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>(shot_view(batch, blockIdx.z), blockIdx.x, blockIdx.y, L, lds_coef);
     if (!gs.g) return;
     __syncthreads();
     tile_boundary(w);
 }
 
 // grouped launches: the tiles of several grids (different sizes and media, isotropic
-// relaxation) in one 1D launch. ALL_CODED: every grid reads coded coefficients; otherwise each
-// grid takes the coded or the per-cell-map path by its own handle.
-template <int TX, bool ALL_CODED>
+// relaxation) in one 1D launch. FAST: every grid reads coded coefficients and has the same weights on
+// both axes; otherwise each grid takes the coded or the per-cell-map path by its own handle, with the
+// sets of both axes staged.
+template <class S, bool FAST>
 __global__ __launch_bounds__(kLanes) void k_velocity_tile_group(const GroupTile* __restrict__ t, int n) {
-    __shared__ __attribute__((aligned(16))) VelTile<TX> L;
+    __shared__ __attribute__((aligned(16))) VelTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
     const int m = group_entry(t, n);
     const DevSim s = t[m].s;
     const unsigned local = blockIdx.x - t[m].start;
     const unsigned bx = local % t[m].gx, by = local / t[m].gx;
-    if (ALL_CODED || s.rcode) velocity_tile<TX, false, true, true>(s, bx, by, L, lds_coef);
-    else velocity_tile<TX, false, true, false>(s, bx, by, L, lds_coef);
+    if (FAST) velocity_tile<S, false, true, true, true>(s, bx, by, L, lds_coef);
+    else if (s.rcode) velocity_tile<S, false, true, true, false>(s, bx, by, L, lds_coef);
+    else velocity_tile<S, false, true, false, false>(s, bx, by, L, lds_coef);
 }
 
 // the pressure update of the tile, then its share of the step's boundary work (gs.g non-null)
-template <int TX, bool ALL_CODED>
+template <class S, bool FAST>
 __global__ __launch_bounds__(kLanes) void k_pressure_tile_group(const GroupTile* __restrict__ t, int n, GroupStep gs) {
-    __shared__ __attribute__((aligned(16))) PreTile<TX> L;
+    __shared__ __attribute__((aligned(16))) PreTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
     const int m = group_entry(t, n);
     const DevSim s = t[m].s;
@@ -452,55 +625,66 @@ __global__ __launch_bounds__(kLanes) void k_pressure_tile_group(const GroupTile*
     const unsigned bx = local % t[m].gx, by = local / t[m].gx;
     TileWork w{};
     if (gs.g) w = tile_work(gs.g[m], local, gs.g[m].step0 + gs.it + (gs.base ? *gs.base : 0));
-    if (ALL_CODED || s.rcode) pressure_tile<TX, false, true, true>(s, bx, by, L, lds_coef);
-    else pressure_tile<TX, false, true, false>(s, bx, by, L, lds_coef);
+    if (FAST) pressure_tile<S, false, true, true, true>(s, bx, by, L, lds_coef);
+    else if (s.rcode) pressure_tile<S, false, true, true, false>(s, bx, by, L, lds_coef);
+    else pressure_tile<S, false, true, false, false>(s, bx, by, L, lds_coef);
     if (!gs.g) return;
     __syncthreads();
     tile_boundary(w);
 }
 
-template <int TX, bool ALL_CODED>
+template <class S, bool FAST>
 hipError_t launch_group_tile(const GroupTile* t, int n, uint32_t blocks, int lds, bool velocity, const GroupStep& gs,
                              hipStream_t st) {
-    if (velocity) hipLaunchKernelGGL((k_velocity_tile_group<TX, ALL_CODED>), dim3(blocks), dim3(kLanes), lds, st, t, n);
-    else hipLaunchKernelGGL((k_pressure_tile_group<TX, ALL_CODED>), dim3(blocks), dim3(kLanes), lds, st, t, n, gs);
+    if (velocity) hipLaunchKernelGGL((k_velocity_tile_group<S, FAST>), dim3(blocks), dim3(kLanes), lds, st, t, n);
+    else hipLaunchKernelGGL((k_pressure_tile_group<S, FAST>), dim3(blocks), dim3(kLanes), lds, st, t, n, gs);
     return hipGetLastError();
 }
 
-template <int TX>
-hipError_t launch_group_tile_any(const GroupTile* t, int n, uint32_t blocks, int lds, bool all_coded, bool velocity,
+template <class S>
+hipError_t launch_group_tile_any(const GroupTile* t, int n, uint32_t blocks, int lds, bool fast, bool velocity,
                                  const GroupStep& gs, hipStream_t st) {
-    return all_coded ? launch_group_tile<TX, true>(t, n, blocks, lds, velocity, gs, st)
-                     : launch_group_tile<TX, false>(t, n, blocks, lds, velocity, gs, st);
+    return fast ? launch_group_tile<S, true>(t, n, blocks, lds, velocity, gs, st)
+                : launch_group_tile<S, false>(t, n, blocks, lds, velocity, gs, st);
 }
 
-template <int TX, bool TAPE = false>
-hipError_t launch_tile(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st) {
-    const bool u = s.ndmap == 1;
-    const int lds = (u ? 1 : s.ndmap) * (s.coef_axes_same ? 1 : 2) * kCS * 4;
+template <class S, bool UNIFORM, bool ISO, bool CODED, bool SAME, bool TAPE>
+void launch_tile_kernel(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st) {
+    const int lds = (UNIFORM ? 1 : s.ndmap) * (SAME ? 1 : 2) * kCS * 4;
     const int64_t rows = s.nx - 2 * kHalo;
-    const dim3 g((unsigned)((s.ny + kTW - 1) / kTW), (unsigned)((rows + TX - 1) / TX), (unsigned)s.nshots);
-    const dim3 b(kLanes);
-    const bool coded = s.isotropic && s.rcode;
-    if (velocity) {
-        if (u && coded) hipLaunchKernelGGL((k_velocity_tile<TX, true, true, true, TAPE>), g, b, lds, st, s);
-        else if (u && s.isotropic) hipLaunchKernelGGL((k_velocity_tile<TX, true, true, false, TAPE>), g, b, lds, st, s);
-        else if (u) hipLaunchKernelGGL((k_velocity_tile<TX, true, false, false, TAPE>), g, b, lds, st, s);
-        else if (coded) hipLaunchKernelGGL((k_velocity_tile<TX, false, true, true, TAPE>), g, b, lds, st, s);
-        else if (s.isotropic) hipLaunchKernelGGL((k_velocity_tile<TX, false, true, false, TAPE>), g, b, lds, st, s);
-        else hipLaunchKernelGGL((k_velocity_tile<TX, false, false, false, TAPE>), g, b, lds, st, s);
-    } else {
-        if (u && coded) hipLaunchKernelGGL((k_pressure_tile<TX, true, true, true, TAPE>), g, b, lds, st, s, gs);
-        else if (u && s.isotropic) hipLaunchKernelGGL((k_pressure_tile<TX, true, true, false, TAPE>), g, b, lds, st, s, gs);
-        else if (u) hipLaunchKernelGGL((k_pressure_tile<TX, true, false, false, TAPE>), g, b, lds, st, s, gs);
-        else if (coded) hipLaunchKernelGGL((k_pressure_tile<TX, false, true, true, TAPE>), g, b, lds, st, s, gs);
-        else if (s.isotropic) hipLaunchKernelGGL((k_pressure_tile<TX, false, true, false, TAPE>), g, b, lds, st, s, gs);
-        else hipLaunchKernelGGL((k_pressure_tile<TX, false, false, false, TAPE>), g, b, lds, st, s, gs);
-    }
+    const dim3 g((unsigned)((s.ny + S::TW - 1) / S::TW), (unsigned)((rows + S::TX - 1) / S::TX), (unsigned)s.nshots);
+    if (velocity) hipLaunchKernelGGL((k_velocity_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>), g, dim3(kLanes), lds, st, s);
+    else hipLaunchKernelGGL((k_pressure_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>), g, dim3(kLanes), lds, st, s, gs);
+}
+
+template <class S, bool SAME, bool TAPE>
+hipError_t launch_tile_same(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st) {
+    const bool u = s.ndmap == 1, coded = s.isotropic && s.rcode;
+    if (u && coded) launch_tile_kernel<S, true, true, true, SAME, TAPE>(s, velocity, gs, st);
+    else if (u && s.isotropic) launch_tile_kernel<S, true, true, false, SAME, TAPE>(s, velocity, gs, st);
+    else if (u) launch_tile_kernel<S, true, false, false, SAME, TAPE>(s, velocity, gs, st);
+    else if (coded) launch_tile_kernel<S, false, true, true, SAME, TAPE>(s, velocity, gs, st);
+    else if (s.isotropic) launch_tile_kernel<S, false, true, false, SAME, TAPE>(s, velocity, gs, st);
+    else launch_tile_kernel<S, false, false, false, SAME, TAPE>(s, velocity, gs, st);
     return hipGetLastError();
+}
+
+template <class S, bool TAPE = false>
+hipError_t launch_tile(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st) {
+    return s.coef_axes_same ? launch_tile_same<S, true, TAPE>(s, velocity, gs, st)
+                            : launch_tile_same<S, false, TAPE>(s, velocity, gs, st);
 }
 
 }  // namespace
+
+// The tile shape that each row count stands for.
+using Tile8 = Shape<128, 8>;
+using Tile16 = Shape<128, 16>;
+using Tile32 = Shape<64, 32>;
+
+int tile2d_width(int rows) {
+    return rows == 8 ? Tile8::TW : rows == 32 ? Tile32::TW : Tile16::TW;
+}
 
 // The most sound speeds (coefficient sets) the tiled kernels stage: two padded sets (one per
 // axis, unequal spacings) of every sound speed next to the largest tile must fit in the 160 KiB of
@@ -508,9 +692,9 @@ hipError_t launch_tile(const DevSim& s, bool velocity, const GroupStep& gs, hipS
 // largest member's sets next to the same tiles).
 constexpr int kMaxTileSets = 768;
 constexpr size_t kLdsPerWorkgroup = size_t(160) << 10;
-static_assert(sizeof(PreTile<32>) + size_t(2) * kMaxTileSets * kCS * sizeof(float) <= kLdsPerWorkgroup,
+static_assert(sizeof(PreTile<Tile32>) + size_t(2) * kMaxTileSets * kCS * sizeof(float) <= kLdsPerWorkgroup,
               "tiled pressure kernel: 32-row tile plus the staged sets exceeds the LDS of a workgroup");
-static_assert(sizeof(VelTile<32>) + size_t(2) * kMaxTileSets * kCS * sizeof(float) <= kLdsPerWorkgroup,
+static_assert(sizeof(VelTile<Tile32>) + size_t(2) * kMaxTileSets * kCS * sizeof(float) <= kLdsPerWorkgroup,
               "tiled velocity kernel: 32-row tile plus the staged sets exceeds the LDS of a workgroup");
 
 bool tile2d_supported(const DevSim& s) {
@@ -519,23 +703,23 @@ bool tile2d_supported(const DevSim& s) {
 
 unsigned group_tile_rows(int64_t nx, int rows) { return (unsigned)((nx - 2 * kHalo + rows - 1) / rows); }
 
-hipError_t launch_group_tile2d(const GroupTile* t, int n, uint32_t blocks, int rows, int coef_sets, bool all_coded,
+hipError_t launch_group_tile2d(const GroupTile* t, int n, uint32_t blocks, int rows, int coef_sets, bool fast,
                                bool velocity, const GroupStep& gs, hipStream_t st) {
     if (n <= 0 || blocks == 0) return hipSuccess;
     const int lds = coef_sets * kCS * 4;  // the largest member's staged sets (stage_coef)
     switch (rows) {
-        case 8: return launch_group_tile_any<8>(t, n, blocks, lds, all_coded, velocity, gs, st);
-        case 32: return launch_group_tile_any<32>(t, n, blocks, lds, all_coded, velocity, gs, st);
-        default: return launch_group_tile_any<16>(t, n, blocks, lds, all_coded, velocity, gs, st);
+        case 8: return launch_group_tile_any<Tile8>(t, n, blocks, lds, fast, velocity, gs, st);
+        case 32: return launch_group_tile_any<Tile32>(t, n, blocks, lds, fast, velocity, gs, st);
+        default: return launch_group_tile_any<Tile16>(t, n, blocks, lds, fast, velocity, gs, st);
     }
 }
 
 hipError_t launch_tile2d(const DevSim& s, const LaunchCfg& cfg, bool velocity, const GroupStep& gs, hipStream_t st) {
-    if (s.tape_div) return launch_tile<8, true>(s, velocity, GroupStep{}, st);  // taped steps: 8-row tiles
+    if (s.tape_div) return launch_tile<Tile8, true>(s, velocity, GroupStep{}, st);  // taped steps: 8-row tiles
     switch (cfg.chunk) {
-        case 8: return launch_tile<8>(s, velocity, gs, st);
-        case 32: return launch_tile<32>(s, velocity, gs, st);
-        default: return launch_tile<16>(s, velocity, gs, st);
+        case 8: return launch_tile<Tile8>(s, velocity, gs, st);
+        case 32: return launch_tile<Tile32>(s, velocity, gs, st);
+        default: return launch_tile<Tile16>(s, velocity, gs, st);
     }
 }
 

@@ -148,7 +148,8 @@ int fw_sim_set_field(fw_sim* sim, const char* name, const float* values, size_t 
  * kernel). It has no counterpart in the reference, whose binary fixes its kernels.
  * variant 0 = per-cell kernels, 1 = x-marching kernels with
  * `width` lanes per workgroup along the contiguous axis and `chunk` planes per workgroup,
- * 2 = 2D tiled kernels with 4-wide vector access on tiles of `chunk` rows x 256 columns,
+ * 2 = 2D tiled kernels with 4-wide vector access (workgroups of `width` = 256 lanes on tiles of
+ * `chunk` rows),
  * 3 / 4 = 3D software-pipelined x-marching kernels (workgroups of `width` = 512 or 1024 lanes;
  * per-cell operands loaded one iteration ahead / at the top of their iteration).
  * Chosen on the first run by timing the candidates on the handle's own arrays, separately for
@@ -211,8 +212,8 @@ typedef struct fw_group fw_group;
 int fw_group_create(fw_sim* const* sims, int32_t n, int32_t width, int32_t chunk, fw_group** out);
 int fw_group_config(const fw_group* group, int32_t* width, int32_t* chunk);
 /* The same with the kernel family chosen: variant 1 is the x-marching kernels above
- * (fw_group_create); variant 2 the tiled float4 kernels, 256 columns x `chunk` rows (8, 16 or
- * 32; 0: timed) per workgroup, for members with ny % 4 == 0 and at most 768 sound speeds
+ * (fw_group_create); variant 2 the tiled float4 kernels, `chunk` rows (8, 16 or 32; 0: timed)
+ * per workgroup of 256 lanes, for members with ny % 4 == 0 and at most 768 sound speeds
  * (FW_ERR_UNSUPPORTED otherwise); variant 0 times both families (the tiled one when every
  * member takes it) with width and chunk 0. Each member's records equal fw_sim_run with the same family and shape bit for bit
  * ("tile:<chunk>" for variant 2). fw_group_shape reports the family and shape in use. */

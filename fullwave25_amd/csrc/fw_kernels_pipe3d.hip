@@ -579,12 +579,13 @@ template <int TY, bool AHEAD>
 void launch_pipe(bool velocity, const DevSim& s, int chunk, hipStream_t st) {
     const bool u = s.ndmap == 1;
     const int nsets = u ? 1 : s.ndmap;
-    const bool same = s.coef_axes_same != 0 && nsets <= kLdsSetsSame;
+    const bool coded = s.isotropic && s.rcode;
+    // the SAME kernels are coded ones; the others copy three sets per sound speed to LDS
+    const bool same = coded && s.coef_axes_same != 0 && nsets <= kLdsSetsSame;
     const int lds = same ? nsets * kNCoef * 4 : (nsets > kLdsSetsP ? 0 : nsets * 3 * kNCoef * 4);
     const dim3 g((unsigned)((s.nz + PZ3 - 1) / PZ3), (unsigned)((s.ny + TY - 1) / TY),
                  (unsigned)((s.nx - 2 * kHalo + chunk - 1) / chunk * s.nshots));
     const dim3 b(PZ3 * TY);
-    const bool coded = s.isotropic && s.rcode;
     if (velocity) {
         if (u && coded && same)
             hipLaunchKernelGGL((k_velocity_pipe3d<TY, true, true, AHEAD, true, true>), g, b, lds, st, s, chunk);

@@ -62,3 +62,47 @@ def test_2d_families_agree_bit_for_bit(monkeypatch, shape, kind):
         for codes in (True, False):
             for got, ref in zip(run(inp, s, monkeypatch, codes), want):
                 np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("kind", ["one", "patches", "cells"])
+@pytest.mark.parametrize("shape", [(17, 19, 21), (21, 26, 96), (18, 33, 131)])
+def test_3d_families_agree_bit_for_bit(monkeypatch, shape, kind):
+    inp = medium(shape, kind, nt=10)
+    if kind == "patches":
+        inp = dataclasses.replace(inp, dz=inp.dx * 1.2)
+    want = run(inp, "percell", monkeypatch)
+    assert np.abs(want[1]).max() > 0
+    for s in ("percell", "stream:512:5", "pipe:512:4", "pipelite:512:7", "pipelite:1024:3"):
+        print(f"{shape} {kind}: {s}", flush=True)
+        for codes in (True, False):
+            for got, ref in zip(run(inp, s, monkeypatch, codes), want):
+                np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("model", ["isotropic", "per_axis", "exponential"])
+@pytest.mark.parametrize("shape", [(17, 17), (21, 65), (40, 200), (17, 18, 19), (19, 21, 67)])
+def test_per_cell_boundary_work_matches_boundary_launch(monkeypatch, shape, model):
+    """The per-cell pressure kernels do the step's sources, pressure release and sensors for the points
+    of their tiles: points in the ghost border, at the grid's corners and on tile edges, repeated and on
+    each other, equal to the boundary pass launched on its own, bit for bit."""
+    rng = np.random.default_rng(3)
+    nd = len(shape)
+    corners = np.stack(np.meshgrid(*[[0, n - 1] for n in shape], indexing="ij"), -1).reshape(-1, nd)
+    inside = np.stack([rng.integers(0, n, 40) for n in shape], 1)
+    edge = inside.copy()
+    edge[:, -1] = np.minimum(rng.choice([8, 63, 64, 65], 40), shape[-1] - 1)
+    src, out, air = (np.concatenate([corners, inside[i::3], edge[i::3]]) for i in range(3))
+    out = np.concatenate([out, src[4:], air[:6], out[:3]])
+    sig = rng.standard_normal((len(src), 9)).astype(np.float32)
+    kw = {"isotropic": model != "per_axis"}
+    if model == "exponential":
+        kw = {"a_exp": 0.98 + 0.02 * rng.random(shape)}
+    inp = raw_inputs(shape, c=rng.choice([1500.0, 1523.0], size=shape), rho=950 + 100 * rng.random(shape), nt=17, icc=src,
+                     icmat=sig, outc=out, icczero=air, modt=2, **kw)
+    got = {}
+    for fused in ("1", "0"):
+        monkeypatch.setenv("FULLWAVE_HIP_FUSED_BOUNDARY", fused)
+        got[fused] = run(inp, "percell", monkeypatch)
+    assert np.abs(got["1"][0]).max() > 0
+    for a, b in zip(got["1"], got["0"]):
+        np.testing.assert_array_equal(a, b)

@@ -145,6 +145,7 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
     int rc = fw::prepare(f);
     if (rc != FW_OK) return rc;
     tape_kernels(f);
+    if ((rc = fw::refit_boundary(f)) != FW_OK) return rc;
     size_t free_b = 0, total_b = 0;
     if (checkpoint_every == 0) ADJ_HIP(hipMemGetInfo(&free_b, &total_b));
     fw_adj* a = new fw_adj();

@@ -371,10 +371,17 @@ int check_coords(const fw_desc& d, int64_t sx, int64_t sy, const std::vector<int
     return FW_OK;
 }
 
-// Time one configuration of one stencil kernel, `reps` launches after one warm-up.
+// Time one configuration of one stencil kernel, `reps` launches after one warm-up. A pressure kernel that
+// leaves the boundary work to a launch of its own is timed with that launch, injecting nothing (the
+// state and the records stay zero).
 int time_config(fw_sim* s, const fw::LaunchCfg& cfg, bool velocity, int reps, float* ms) {
+    fw::DevBoundary none = s->db;
+    none.ntic = 0;
+    const bool apart = !velocity && !fw::pressure_fuses_boundary(s->ds, cfg);
     auto launch = [&] {
-        return velocity ? fw::launch_velocity(s->ds, cfg, s->stream) : fw::launch_pressure(s->ds, cfg, s->stream);
+        if (velocity) return fw::launch_velocity(s->ds, cfg, s->stream);
+        const hipError_t e = fw::launch_pressure(s->ds, cfg, s->stream);
+        return e == hipSuccess && apart ? fw::launch_boundary(s->ds, none, 0, s->d.modt, s->stream) : e;
     };
     FW_HIP(launch());
     FW_HIP(hipEventRecord(s->ev[0], s->stream));
@@ -563,16 +570,19 @@ bool codes_wanted(const fw_sim* s) {
     return !(env && env[0] == '0');
 }
 
+// free a device array of `alloc` by name, if there is one
+void drop(fw_sim* s, const char* name) {
+    auto it = s->dev.find(name);
+    if (it == s->dev.end()) return;
+    dev_free(s, it->second);
+    s->dev.erase(it);
+}
+
 void drop_codes(fw_sim* s) {
-    for (const char* name : {"_rcode", "_rtab_v", "_rtab_p"}) {
-        auto it = s->dev.find(name);
-        if (it == s->dev.end()) continue;
-        dev_free(s, it->second);
-        s->dev.erase(it);
-    }
+    for (const char* name : {"_rcode", "_rtab_v", "_rtab_p", "_rwide_v", "_rwide_p"}) drop(s, name);
     s->ds.rcode = nullptr;
-    s->ds.rtab_v = nullptr;
-    s->ds.rtab_p = nullptr;
+    s->ds.rtab_v = s->ds.rtab_p = nullptr;
+    s->ds.rwide_v = s->ds.rwide_p = nullptr;
     s->ncodes = 0;
     s->coded_cells = 0;
 }
@@ -682,6 +692,15 @@ int encode_relaxation(fw_sim* s) {
         s->ds.rtab_p = (const float*)tp;
         s->ncodes = n;
         s->coded_cells = covered;
+        if (n <= fw::kMaxWideCodes && s->ds.coef_axes_same) {  // rows with weights for the per-cell kernels
+            void *wv, *wp;
+            if ((r = alloc(s, "_rwide_v", (size_t)n * fw::kWideStride * 4, &wv)) != FW_OK) return r;
+            if ((r = alloc(s, "_rwide_p", (size_t)n * fw::kWideStride * 4, &wp)) != FW_OK) return r;
+            FW_HIP(fw::launch_code_widen((const float*)tv, s->ds.coef, n, s->ndim, (float*)wv, s->stream));
+            FW_HIP(fw::launch_code_widen((const float*)tp, s->ds.coef, n, s->ndim, (float*)wp, s->stream));
+            s->ds.rwide_v = (const float*)wv;
+            s->ds.rwide_p = (const float*)wp;
+        }
         return FW_OK;
     };
     const int rc = run();
@@ -723,19 +742,33 @@ std::vector<fw::GroupBoundary> fused_entries(const fw_sim* s, const fw::GroupBou
 }
 
 // Group the handle's points by the tiles of its pressure kernel when that kernel can do the
-// step's boundary work (2D marching or tiled kernels; not for a fixed-region handle, whose
-// footprint does not count these lists).
+// step's boundary work (the per-cell kernels, 2D marching or tiled kernels; not for a fixed-region
+// handle, whose footprint does not count these lists).
+// A table of more points than this (the whole domain recorded, say) takes longer to group (13 ns a
+// point) than a thousand steps' launches of the pass on its own take (3 to 5 us each).
+constexpr size_t kMaxFusedPoints = size_t(1) << 18;
+
 int setup_fused_boundary(fw_sim* s, const fw::BoundaryLists& bl) {
     s->fused_boundary = false;
+    drop(s, "_fpoints");
+    drop(s, "_fbound");
     if (s->fixed_base || !fw::pressure_fuses_boundary(s->ds, s->cfg_p)) return FW_OK;
+    if (bl.src_lin.size() + bl.zero_lin.size() + bl.out_lin.size() > kMaxFusedPoints) return FW_OK;
     const char* env = getenv("FULLWAVE_HIP_FUSED_BOUNDARY");  // "0": a launch of its own (tests)
     if (env && env[0] == '0') return FW_OK;
     const fw::LaunchCfg& c = s->cfg_p;
-    const int tile_w = c.variant == 2 ? fw::tile2d_width(c.chunk) : (c.width == 64 || c.width == 256 ? c.width : 128);
-    const int rows = c.variant == 2 ? c.chunk : (c.chunk < 2 ? 2 : c.chunk);
-    const unsigned gx = (unsigned)((s->ds.ny + tile_w - 1) / tile_w);
     std::vector<int32_t> pts;
-    const fw::PointTable pt = fw::point_table(s->ds.nx, s->ds.ny, gx, tile_w, rows, bl, &pts);
+    fw::PointTable pt;
+    if (c.variant == 0) {
+        const int64_t pitch = s->ndim == 2 ? s->ds.sx : s->ds.sy;
+        pt = fw::point_table_rows(fw::cell_first_row(s->ds), fw::cell_row_count(s->ds), pitch, fw::cell_tiles_x(s->ds),
+                                  fw::kCellTileCols, fw::kCellTileRows, bl, &pts);
+    } else {
+        const int tile_w = c.variant == 2 ? fw::tile2d_width(c.chunk) : (c.width == 64 || c.width == 256 ? c.width : 128);
+        const int rows = c.variant == 2 ? c.chunk : (c.chunk < 2 ? 2 : c.chunk);
+        const unsigned gx = (unsigned)((s->ds.ny + tile_w - 1) / tile_w);
+        pt = fw::point_table(s->ds.nx, s->ds.ny, gx, tile_w, rows, bl, &pts);
+    }
     void* p;
     int rc;
     if ((rc = alloc(s, "_fpoints", pts.size() * 4, &p)) != FW_OK) return rc;
@@ -862,7 +895,8 @@ int launch_step(fw_sim* s, bool timed, double* ms) {
     int rc;
     rc = timed_launch(fw::kVelocity, [&] { return fw::launch_velocity(s->ds, s->cfg_v, s->stream); });
     if (rc != FW_OK) return rc;
-    if (s->fused_boundary && !s->ds.tape_div) {  // the pressure launch does the boundary work
+    // the pressure launch does the boundary work where its kernel can (a taped step's may be another)
+    if (s->fused_boundary && fw::pressure_fuses_boundary(s->ds, s->cfg_p)) {
         const fw::GroupStep gs{s->fbound, nullptr, s->step};
         rc = timed_launch(fw::kPressure, [&] { return fw::launch_pressure(s->ds, s->cfg_p, s->stream, gs); });
         if (rc != FW_OK) return rc;
@@ -1030,6 +1064,12 @@ int set_error(int code, const char* fmt, ...) {
 }
 
 int prepare(fw_sim* s) { return s->ready ? FW_OK : finalize(s); }
+
+int refit_boundary(fw_sim* s) {
+    BoundaryLists bl;
+    const int rc = resolve_boundary(s->d, s->ds.sx, s->ds.sy, s->icc, s->outc, s->zero, &bl);
+    return rc != FW_OK ? rc : setup_fused_boundary(s, bl);
+}
 
 int forward_step(fw_sim* s) { return launch_step(s, false, nullptr); }
 

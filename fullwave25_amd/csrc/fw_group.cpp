@@ -38,18 +38,20 @@ struct fw_group {
 
 namespace fw {
 
-void points_by_tile(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const std::vector<int64_t>& lin,
-                    std::vector<int32_t>* off, std::vector<int32_t>* idx) {
-    const unsigned gy = (unsigned)((nx - 2 * kHalo + rows - 1) / rows);
-    const size_t ntiles = (size_t)gx * gy;
+namespace {
+
+// points_by_tile over contiguous rows [first, first + count) of `pitch` elements
+void points_by_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows,
+                    const std::vector<int64_t>& lin, std::vector<int32_t>* off, std::vector<int32_t>* idx) {
+    const size_t ntiles = (size_t)gx * (size_t)((count + rows - 1) / rows);
     std::vector<int64_t> owner(lin.size(), -1);
     off->assign(ntiles + 1, 0);
     for (size_t q = 0; q < lin.size(); ++q) {
         if (lin[q] < 0) continue;
-        int64_t i = lin[q] / ny;
-        const int64_t j = lin[q] % ny;
-        i = i < kHalo ? kHalo : (i > nx - kHalo - 1 ? nx - kHalo - 1 : i);
-        const int64_t t = ((i - kHalo) / rows) * (int64_t)gx + j / tile_w;
+        int64_t i = lin[q] / pitch;
+        const int64_t j = lin[q] % pitch;
+        i = i < first ? first : (i > first + count - 1 ? first + count - 1 : i);
+        const int64_t t = ((i - first) / rows) * (int64_t)gx + j / tile_w;
         owner[q] = t;
         ++(*off)[(size_t)t + 1];
     }
@@ -60,8 +62,20 @@ void points_by_tile(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, c
         if (owner[q] >= 0) (*idx)[(size_t)fill[(size_t)owner[q]]++] = (int32_t)q;
 }
 
+}  // namespace
+
+void points_by_tile(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const std::vector<int64_t>& lin,
+                    std::vector<int32_t>* off, std::vector<int32_t>* idx) {
+    points_by_rows(kHalo, nx - 2 * kHalo, ny, gx, tile_w, rows, lin, off, idx);
+}
+
 PointTable point_table(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const BoundaryLists& bl,
                        std::vector<int32_t>* tab) {
+    return point_table_rows(kHalo, nx - 2 * kHalo, ny, gx, tile_w, rows, bl, tab);
+}
+
+PointTable point_table_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows,
+                            const BoundaryLists& bl, std::vector<int32_t>* tab) {
     auto align4 = [&] {
         while (tab->size() % 4) tab->push_back(0);
     };
@@ -71,7 +85,7 @@ PointTable point_table(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows
     };
     std::vector<int32_t> off[3], idx[3];
     const std::vector<int64_t>* lists[3] = {&bl.src_lin, &bl.zero_lin, &bl.out_lin};
-    for (int k = 0; k < 3; ++k) points_by_tile(nx, ny, gx, tile_w, rows, *lists[k], &off[k], &idx[k]);
+    for (int k = 0; k < 3; ++k) points_by_rows(first, count, pitch, gx, tile_w, rows, *lists[k], &off[k], &idx[k]);
     PointTable pt{};
     pt.ntiles = (int32_t)(off[0].size() - 1);
     align4();

@@ -55,6 +55,11 @@ struct DevSim {
     const uint16_t* rcode;
     const float* rtab_v;
     const float* rtab_p;
+    // the same rows with the stencil weights of the row's set, kWideStride floats {1/kappa, a1, a2, b1,
+    // b2, w_1..w_8, e, 0, 0}, for the per-cell kernels (null: more than kMaxWideCodes codes, or axes
+    // with weights of their own)
+    const float* rwide_v;
+    const float* rwide_p;
 
     // adjoint tape of the step (null: none). When tape_div is set, the velocity kernel also
     // writes, at every updated cell, tape_u[a][c] = D+_a p / kappa + psi1' + psi2' (exponential
@@ -70,6 +75,10 @@ constexpr int kCodeVals = 11;          // values per tuple: velocity side, press
 constexpr int kCodeStride = 8;         // floats per table row (one 16-byte and one 8-byte load)
 constexpr uint32_t kCodeEscape = 0xffff;  // the cell's tuple has no code
 constexpr int kMaxCodes = 65535;       // codes 0 .. 65534
+constexpr int kWideStride = 16;        // floats per row with weights
+constexpr int kMaxWideCodes = 16384;   // 1 MB a table: it stays in the L2 of every XCD
+// the per-cell kernels' tiles: rows of contiguous cells by columns
+constexpr int kCellTileRows = 4, kCellTileCols = 64;
 constexpr uint32_t kCodeSlotsSmall = 1u << 16;  // hash table slots, first try
 constexpr uint32_t kCodeSlots = 1u << 22;       // hash table slots, when the first try overflows
 constexpr int kCodeMaxProbe = 128;
@@ -107,6 +116,11 @@ template <class T>
 __device__ __forceinline__ T gld16(const T* __restrict__ base, uint32_t i) {  // 2-byte elements
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (i << 1));
 }
+
+// Read-only tables through the scalar data cache: where every lane of a wavefront reads the same
+// element, one scalar load into scalar registers serves them all.
+typedef const __attribute__((address_space(4))) float* scalar_ptr;
+__device__ __forceinline__ scalar_ptr as_scalar(const float* p) { return (scalar_ptr)(uintptr_t)p; }
 
 // Relaxation coefficients and coefficient-set index of one cell.
 struct CodedCoef {
@@ -200,6 +214,15 @@ __device__ inline int shot_of_block(const DevSim& s, unsigned& zl) {
     return (int)shot;
 }
 
+// Workgroup b of n runs on XCD b % 8 (round-robin dispatch). Taking tile xcd_order(b, n) instead of b
+// gives each XCD one contiguous run of the tiles in row-major order, so that neighbouring tiles, whose
+// stencils read the same rows, share an L2. A bijection of [0, n) for any n.
+__device__ __forceinline__ uint32_t xcd_order(uint32_t b, uint32_t n) {
+    constexpr uint32_t kXcds = 8;
+    const uint32_t xcd = b % kXcds, k = b / kXcds, q = n / kXcds, r = n % kXcds;
+    return xcd * q + (xcd < r ? xcd : r) + k;
+}
+
 // Largest z extent of a launch grid.
 constexpr unsigned kMaxGridZ = 65535;
 
@@ -243,13 +266,13 @@ struct GroupTile {
     int32_t chunk;  // rows per workgroup for this grid
 };
 
-// The entry of a grouped launch that owns workgroup blockIdx.x: the last with start <= it
+// The entry of a grouped launch that owns tile b: the last with start <= it
 // (binary search over the table; every lane of the workgroup reads the same entries).
-__device__ inline int group_entry(const GroupTile* __restrict__ t, int n) {
+__device__ inline int group_entry(const GroupTile* __restrict__ t, int n, uint32_t b) {
     int lo = 0, hi = n - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (t[mid].start <= blockIdx.x) lo = mid;
+        if (t[mid].start <= b) lo = mid;
         else hi = mid - 1;
     }
     return lo;
@@ -357,12 +380,19 @@ struct LaunchCfg {
     int chunk = 32;
 };
 
+// the per-cell kernels (gs as for launch_pressure), their tiles across and in all, and the rows of
+// contiguous cells that they cover
+hipError_t launch_simple(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st);
+unsigned cell_tiles_x(const DevSim& s);
+int64_t cell_tiles(const DevSim& s);
+int64_t cell_first_row(const DevSim& s);
+int64_t cell_row_count(const DevSim& s);
 bool streaming_supported(const DevSim& s);
 bool tile2d_supported(const DevSim& s);
 int tile2d_width(int rows);  // columns of the tile of `rows` rows (8, 16 or 32)
 hipError_t launch_velocity(const DevSim& s, const LaunchCfg& cfg, hipStream_t st);
 hipError_t launch_pipe3d(const DevSim& s, const LaunchCfg& cfg, bool velocity, hipStream_t st);
-// gs.g non-null (2D marching and tiled kernels, untaped steps: pressure_fuses_boundary): the
+// gs.g non-null (pressure_fuses_boundary: the per-cell, the 2D marching and the tiled kernels): the
 // pressure launch also does the step's sources, pressure release and sensors (tile_boundary;
 // gs.g holds one entry per shot, whose points are grouped by the tiles of `cfg`)
 hipError_t launch_pressure(const DevSim& s, const LaunchCfg& cfg, hipStream_t st, const GroupStep& gs = GroupStep{});
@@ -404,6 +434,8 @@ hipError_t launch_code_assign(const CodeMaps& m, int64_t n, const unsigned long 
                               const uint16_t* slot_code, uint16_t* code, int32_t* status, hipStream_t st);
 hipError_t launch_code_table(const CodeMaps& m, int32_t ncodes, const int32_t* rep_of_code, float* tab_v, float* tab_p,
                              hipStream_t st);
+// rows with weights from a code table and the coefficient table of nd axes
+hipError_t launch_code_widen(const float* tab, const float* coef, int32_t ncodes, int nd, float* wide, hipStream_t st);
 hipError_t launch_code_verify(const CodeMaps& m, int64_t n, const uint16_t* code, int32_t ncodes, const float* tab_v,
                               const float* tab_p, int32_t* status, hipStream_t st);
 // The sparse part of a reverse step, in one launch: the records' weights added at the distinct

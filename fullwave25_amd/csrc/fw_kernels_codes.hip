@@ -157,6 +157,19 @@ __global__ __launch_bounds__(256) void k_code_table(CodeMaps m, int32_t ncodes, 
     rv[6] = rv[7] = rp[6] = rp[7] = 0.f;
 }
 
+// A code's row with the weights of its coefficient set (DevSim::rwide_v, rwide_p).
+__global__ __launch_bounds__(256) void k_code_widen(const float* tab, const float* coef, int32_t ncodes, int nd,
+                                                    float* wide) {
+    const int32_t id = blockIdx.x * blockDim.x + threadIdx.x;
+    if (id >= ncodes) return;
+    const float* r = tab + (int64_t)id * kCodeStride;
+    float* o = wide + (int64_t)id * kWideStride;
+    const float* w = coef + (int64_t)__float_as_int(r[5]) * nd * kNCoef;
+    for (int k = 0; k < 5; ++k) o[k] = r[k];
+    for (int k = 0; k < kNCoef; ++k) o[5 + k] = w[k];
+    o[14] = o[15] = 0.f;
+}
+
 __global__ __launch_bounds__(256) void k_code_verify(CodeMaps m, int64_t n, const uint16_t* code, int32_t ncodes,
                                                      const float* tab_v, const float* tab_p, int32_t* status) {
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
@@ -204,6 +217,12 @@ hipError_t launch_code_table(const CodeMaps& m, int32_t ncodes, const int32_t* r
     if (ncodes <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_code_table, dim3((unsigned)((ncodes + 255) / 256)), dim3(256), 0, st, m, ncodes, rep_of_code,
                        tab_v, tab_p);
+    return hipGetLastError();
+}
+
+hipError_t launch_code_widen(const float* tab, const float* coef, int32_t ncodes, int nd, float* wide, hipStream_t st) {
+    if (ncodes <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_code_widen, dim3((unsigned)((ncodes + 255) / 256)), dim3(256), 0, st, tab, coef, ncodes, nd, wide);
     return hipGetLastError();
 }
 

@@ -16,8 +16,6 @@
 
 namespace fw {
 
-hipError_t launch_velocity_simple(const DevSim& s, hipStream_t st);
-hipError_t launch_pressure_simple(const DevSim& s, hipStream_t st);
 hipError_t launch_velocity_3d(const DevSim& s, const LaunchCfg& cfg, hipStream_t st);
 hipError_t launch_pressure_3d(const DevSim& s, const LaunchCfg& cfg, hipStream_t st);
 
@@ -370,7 +368,7 @@ __global__ __launch_bounds__(TY) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 template <int TY>
 __global__ __launch_bounds__(TY) void k_velocity_2d_group(const GroupTile* __restrict__ t, int n) {
     extern __shared__ float lds_coef[];
-    const int m = group_entry(t, n);
+    const int m = group_entry(t, n, blockIdx.x);
     const DevSim s = t[m].s;
     const int chunk = t[m].chunk;
     const unsigned local = blockIdx.x - t[m].start;
@@ -384,7 +382,7 @@ template <int TY>
 __global__ __launch_bounds__(TY) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_pressure_2d_group(
     const GroupTile* __restrict__ t, int n, GroupStep gs) {
     extern __shared__ float lds_coef[];
-    const int m = group_entry(t, n);
+    const int m = group_entry(t, n, blockIdx.x);
     const DevSim s = t[m].s;
     const int chunk = t[m].chunk;
     const unsigned local = blockIdx.x - t[m].start;
@@ -479,27 +477,32 @@ bool tape_capable(const DevSim& s, const LaunchCfg& cfg) {
 // per-cell kernels otherwise (the only families that write it).
 hipError_t launch_velocity(const DevSim& s, const LaunchCfg& cfg, hipStream_t st) {
     if (cfg.variant == 2 && tile2d_supported(s)) return launch_tile2d(s, cfg, true, GroupStep{}, st);
-    if (s.tape_div) return launch_velocity_simple(s, st);
+    if (s.tape_div) return launch_simple(s, true, GroupStep{}, st);
     if ((cfg.variant == 3 || cfg.variant == 4) && s.ndim == 3 && streaming_supported(s))
         return launch_pipe3d(s, cfg, true, st);
-    if (cfg.variant == 0 || !streaming_supported(s)) return launch_velocity_simple(s, st);
+    if (cfg.variant == 0 || !streaming_supported(s)) return launch_simple(s, true, GroupStep{}, st);
     if (s.ndim == 3) return launch_velocity_3d(s, cfg, st);
     return launch_2d_any(s, cfg, true, GroupStep{}, st);
 }
 
+// The per-cell kernels' point table has three offsets a tile: beyond this many tiles (67 M cells;
+// the launch it saves is under 1 % of a step there) the boundary pass is a launch of its own.
+constexpr int64_t kMaxPointTiles = 1 << 18;
+
 bool pressure_fuses_boundary(const DevSim& s, const LaunchCfg& cfg) {
-    if (s.tape_div || s.ndim != 2) return false;
-    if (cfg.variant == 2) return tile2d_supported(s);
-    return cfg.variant == 1 && streaming_supported(s);
+    if (cfg.variant == 0) return cell_tiles(s) <= kMaxPointTiles;
+    if (s.ndim != 2) return false;
+    if (cfg.variant == 2) return tile2d_supported(s) && !(s.tape_div && cfg.chunk != 8);  // taped: 8-row tiles
+    return cfg.variant == 1 && !s.tape_div && streaming_supported(s);
 }
 
 hipError_t launch_pressure(const DevSim& s, const LaunchCfg& cfg, hipStream_t st, const GroupStep& gs) {
     if (gs.g && !pressure_fuses_boundary(s, cfg)) return hipErrorInvalidValue;
     if (cfg.variant == 2 && tile2d_supported(s)) return launch_tile2d(s, cfg, false, gs, st);
-    if (s.tape_div) return launch_pressure_simple(s, st);
+    if (s.tape_div) return launch_simple(s, false, gs, st);
     if ((cfg.variant == 3 || cfg.variant == 4) && s.ndim == 3 && streaming_supported(s))
         return launch_pipe3d(s, cfg, false, st);
-    if (cfg.variant == 0 || !streaming_supported(s)) return launch_pressure_simple(s, st);
+    if (cfg.variant == 0 || !streaming_supported(s)) return launch_simple(s, false, gs, st);
     if (s.ndim == 3) return launch_pressure_3d(s, cfg, st);
     return launch_2d_any(s, cfg, false, gs, st);
 }

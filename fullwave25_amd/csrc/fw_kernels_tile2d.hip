@@ -256,8 +256,6 @@ struct QuadCoef {
 };
 // WaveCoef: every cell of the wavefront has the same code, so the row and the weights are read once
 // with scalar loads and stay in scalar registers.
-typedef const __attribute__((address_space(4))) float* scalar_ptr;
-__device__ inline scalar_ptr as_scalar(const float* p) { return (scalar_ptr)(uintptr_t)p; }
 template <bool UNIFORM, bool SAME>
 struct WaveCoef {
     float ik_, a1_, a2_, b1_, b2_;
@@ -572,26 +570,36 @@ __device__ inline void pressure_tile(const DevSim& s, unsigned bx, unsigned by, 
     }
 }
 
+// The tile of this workgroup within its shot, in row-major order: each XCD takes a contiguous run of
+// them, so that the halo rows that neighbouring tiles stage come from one L2. us a step against the
+// launch order: 672^2 cells 17.5 -> 15.0, 1152^2 33.7 -> 32.0, 4256 x 2208 176.5 -> 174.0 (at the
+// fastest shape of each).
+__device__ inline uint32_t shot_tile() {
+    return xcd_order(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+}
+
 template <class S, bool UNIFORM, bool ISO, bool CODED, bool SAME, bool TAPE>
 __global__ __launch_bounds__(kLanes) void k_velocity_tile(DevSim batch) {
     __shared__ __attribute__((aligned(16))) VelTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
-    velocity_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>(shot_view(batch, blockIdx.z), blockIdx.x, blockIdx.y, L, lds_coef);
+    const uint32_t t = shot_tile();
+    velocity_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>(shot_view(batch, blockIdx.z), t % gridDim.x, t / gridDim.x, L, lds_coef);
 }
 
 // gs.g non-null: each workgroup then also does the step's source, pressure-release and sensor
-// work of its tile (tile blockIdx.y * gridDim.x + blockIdx.x of shot blockIdx.z), as the group
+// work of its tile (tile shot_tile() of shot blockIdx.z), as the group
 // kernels do
 template <class S, bool UNIFORM, bool ISO, bool CODED, bool SAME, bool TAPE>
 __global__ __launch_bounds__(kLanes) void k_pressure_tile(DevSim batch, GroupStep gs) {
     __shared__ __attribute__((aligned(16))) PreTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
+    const uint32_t t = shot_tile();
     TileWork w{};
     if (gs.g) {
         const GroupBoundary& e = gs.g[blockIdx.z];
-        w = tile_work(e, blockIdx.y * gridDim.x + blockIdx.x, e.step0 + gs.it + (gs.base ? *gs.base : 0));
+        w = tile_work(e, t, e.step0 + gs.it + (gs.base ? *gs.base : 0));
     }
-    pressure_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>(shot_view(batch, blockIdx.z), blockIdx.x, blockIdx.y, L, lds_coef);
+    pressure_tile<S, UNIFORM, ISO, CODED, SAME, TAPE>(shot_view(batch, blockIdx.z), t % gridDim.x, t / gridDim.x, L, lds_coef);
     if (!gs.g) return;
     __syncthreads();
     tile_boundary(w);
@@ -605,9 +613,10 @@ template <class S, bool FAST>
 __global__ __launch_bounds__(kLanes) void k_velocity_tile_group(const GroupTile* __restrict__ t, int n) {
     __shared__ __attribute__((aligned(16))) VelTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
-    const int m = group_entry(t, n);
+    const uint32_t gid = xcd_order(blockIdx.x, gridDim.x);
+    const int m = group_entry(t, n, gid);
     const DevSim s = t[m].s;
-    const unsigned local = blockIdx.x - t[m].start;
+    const unsigned local = gid - t[m].start;
     const unsigned bx = local % t[m].gx, by = local / t[m].gx;
     if (FAST) velocity_tile<S, false, true, true, true>(s, bx, by, L, lds_coef);
     else if (s.rcode) velocity_tile<S, false, true, true, false>(s, bx, by, L, lds_coef);
@@ -619,9 +628,10 @@ template <class S, bool FAST>
 __global__ __launch_bounds__(kLanes) void k_pressure_tile_group(const GroupTile* __restrict__ t, int n, GroupStep gs) {
     __shared__ __attribute__((aligned(16))) PreTile<S> L;
     extern __shared__ __attribute__((aligned(16))) float lds_coef[];
-    const int m = group_entry(t, n);
+    const uint32_t gid = xcd_order(blockIdx.x, gridDim.x);
+    const int m = group_entry(t, n, gid);
     const DevSim s = t[m].s;
-    const unsigned local = blockIdx.x - t[m].start;
+    const unsigned local = gid - t[m].start;
     const unsigned bx = local % t[m].gx, by = local / t[m].gx;
     TileWork w{};
     if (gs.g) w = tile_work(gs.g[m], local, gs.g[m].step0 + gs.it + (gs.base ? *gs.base : 0));
@@ -715,7 +725,7 @@ hipError_t launch_group_tile2d(const GroupTile* t, int n, uint32_t blocks, int r
 }
 
 hipError_t launch_tile2d(const DevSim& s, const LaunchCfg& cfg, bool velocity, const GroupStep& gs, hipStream_t st) {
-    if (s.tape_div) return launch_tile<Tile8, true>(s, velocity, GroupStep{}, st);  // taped steps: 8-row tiles
+    if (s.tape_div) return launch_tile<Tile8, true>(s, velocity, gs, st);  // taped steps: 8-row tiles
     switch (cfg.chunk) {
         case 8: return launch_tile<Tile8>(s, velocity, gs, st);
         case 32: return launch_tile<Tile32>(s, velocity, gs, st);

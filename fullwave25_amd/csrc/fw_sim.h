@@ -38,7 +38,7 @@ struct fw_sim {
     int64_t step = 0;
     int64_t rec_cap = 0;
     fw::LaunchCfg cfg_v, cfg_p;  // velocity and pressure kernels, chosen independently
-    // 2D marching or tiled pressure kernels: the step's sources, pressure release and sensors
+    // per-cell, 2D marching or tiled pressure kernels: the step's sources, pressure release and sensors
     // run inside the pressure launch (one entry per shot, points grouped by the kernel's tiles)
     bool fused_boundary = false;
     fw::GroupBoundary* fbound = nullptr;
@@ -73,6 +73,7 @@ namespace fw {
 // host helpers of fw_api.cpp used by the adjoint
 int set_error(int code, const char* fmt, ...);
 int prepare(fw_sim* s);                    // check inputs, resolve coordinates, pick kernels
+int refit_boundary(fw_sim* s);             // the point table again, after a change of the pressure kernel
 int forward_step(fw_sim* s);               // one time step on the handle's stream
 hipError_t grid_to_host(const fw_sim* s, void* dst, const void* src, size_t esize);  // padded -> compact
 // Host-side set-up of a handle, without device access.
@@ -105,6 +106,10 @@ struct PointTable {
 };
 PointTable point_table(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const BoundaryLists& bl,
                        std::vector<int32_t>* tab);
+// The same for the per-cell kernels: tiles of `tile_w` cells by `rows` rows from contiguous row `first`
+// of `count` rows (`pitch` elements each).
+PointTable point_table_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows,
+                            const BoundaryLists& bl, std::vector<int32_t>* tab);
 // Coefficient table [ndmap][ndim][9] (w_1..w_8, e) from dmap [9][2][ndmap] with each axis's spacing
 // folded in; *axes_same = 1 when every axis has the same set for each sound speed.
 std::vector<float> coefficient_table(const fw_desc& d, const std::vector<float>& dmap, int* axes_same);

@@ -106,3 +106,25 @@ def test_per_cell_boundary_work_matches_boundary_launch(monkeypatch, shape, mode
     assert np.abs(got["1"][0]).max() > 0
     for a, b in zip(got["1"], got["0"]):
         np.testing.assert_array_equal(a, b)
+
+
+def test_checkpointed_run_on_other_kernels_keeps_its_points(monkeypatch):
+    """An adjoint replaces marching kernels by the tiled ones: the untaped steps of a checkpointed
+    forward run then record the same traces as a plain run, bit for bit."""
+    from fullwave25_amd.adjoint import HipAdjoint
+
+    monkeypatch.delenv("FULLWAVE_HIP_KERNELS", raising=False)
+    rng = np.random.default_rng(9)
+    shape = (60, 300)
+    pts = np.stack([rng.integers(8, n - 8, 200) for n in shape], 1)
+    sig = rng.standard_normal((50, 30)).astype(np.float32)
+    inp = raw_inputs(shape, c=rng.choice([1500.0, 1523.0], size=shape), nt=30, icc=pts[:50], icmat=sig, outc=pts[40:190],
+                     icczero=pts[190:])
+    pin = {k: {"variant": "stream", "width": 64, "chunk": 5} for k in ("velocity", "pressure")}
+    with engine.HipSimulation(inp) as sim:
+        sim.run(inp.nt)
+        want = sim.sensors()
+    with HipAdjoint(inp, checkpoint_every=7, kernel_config=pin) as adj:
+        got = adj.forward()
+    assert np.abs(want).max() > 0
+    np.testing.assert_array_equal(got, want)

@@ -587,6 +587,41 @@ void drop_codes(fw_sim* s) {
     s->coded_cells = 0;
 }
 
+// Per-axis maps that are the same on every axis (what the reference's front end writes: it ramps every
+// per-axis copy identically) run the isotropic kernels: one set of maps, coded, instead of two or
+// three (1152^2 cells: 100 -> 58 bytes a cell in the velocity kernel). Compared bit for bit on the
+// device whenever a map is new; the same values enter the same arithmetic, so results do not change.
+int match_axes(fw_sim* s) {
+    const fw_desc& d = s->d;
+    s->ds.isotropic = d.isotropic;
+    if (d.isotropic || d.attenuation_model != 0 || s->fixed_base) return FW_OK;
+    fw::MapPairs m{};
+    for (int a = 1; a < s->ndim; ++a) {
+        auto pair = [&](const float* x, const float* y) {
+            m.a[m.n] = x;
+            m.b[m.n++] = y;
+        };
+        pair(s->ds.ikv[0], s->ds.ikv[a]);
+        pair(s->ds.ikp[0], s->ds.ikp[a]);
+        for (int nu = 0; nu < fw::kNRelax; ++nu) {
+            pair(s->ds.av[0][nu], s->ds.av[a][nu]);
+            pair(s->ds.bv[0][nu], s->ds.bv[a][nu]);
+            pair(s->ds.ap[0][nu], s->ds.ap[a][nu]);
+            pair(s->ds.bp[0][nu], s->ds.bp[a][nu]);
+        }
+    }
+    Stage flag;
+    int32_t differ = 1;
+    hipError_t e = flag.get(s, 4);
+    if (e == hipSuccess) e = hipMemsetAsync(flag.p, 0, 4, s->stream);
+    if (e == hipSuccess) e = fw::launch_maps_differ(m, s->ncell, (int32_t*)flag.p, s->stream);
+    if (e == hipSuccess) e = copy_sync(s, &differ, flag.p, 4, hipMemcpyDeviceToHost);
+    const hipError_t e2 = flag.release(s);
+    FW_HIP(e != hipSuccess ? e : e2);
+    s->ds.isotropic = differ ? 0 : 1;
+    return FW_OK;
+}
+
 // Code the isotropic relaxation maps and dcmap (kernels and the steps in fw_kernels_codes.hip).
 // Leaves the handle on the per-cell maps when the model is not isotropic relaxation, when codes
 // are switched off, when the codes would cover less than half of the cells, or when any check
@@ -594,7 +629,7 @@ void drop_codes(fw_sim* s) {
 int encode_relaxation(fw_sim* s) {
     drop_codes(s);
     const fw_desc& d = s->d;
-    if (d.attenuation_model != 0 || !d.isotropic || !codes_wanted(s)) return FW_OK;
+    if (d.attenuation_model != 0 || !s->ds.isotropic || !codes_wanted(s)) return FW_OK;
     if (s->ncell >= ((int64_t)1 << 30)) return FW_OK;  // the marching kernels' 32-bit offsets
     fw::CodeMaps m{};
     const char* names[fw::kCodeVals - 1] = {"kappau", "apmlu1", "apmlu2", "bpmlu1", "bpmlu2",
@@ -721,7 +756,8 @@ int recode(fw_sim* s) {
         (void)hipGraphExecDestroy(s->graph);
         s->graph = nullptr;
     }
-    return encode_relaxation(s);
+    const int rc = match_axes(s);
+    return rc != FW_OK ? rc : encode_relaxation(s);
 }
 
 // The boundary entries of a handle whose pressure kernel does the step's boundary work: one per
@@ -869,7 +905,7 @@ int finalize(fw_sim* s) {
     s->ds.rho = (const float*)s->dev["rho"];
     s->ds.dcmap = (const int32_t*)s->dev["dcmap"];
     s->ds.ndmap = (int32_t)d.ndmap;
-    s->ds.isotropic = d.isotropic;
+    if ((rc = match_axes(s)) != FW_OK) return rc;
     if ((rc = encode_relaxation(s)) != FW_OK) return rc;
     if ((rc = choose_kernels(s)) != FW_OK) return rc;
     if ((rc = setup_fused_boundary(s, bl)) != FW_OK) return rc;
@@ -1310,7 +1346,7 @@ int fw_sim_upload(fw_sim* s, const char* name_c, const void* host, size_t bytes)
         s->have[name] = true;
         const bool relaxation_map = name.rfind("kappa", 0) == 0 || name.rfind("apml", 0) == 0 ||
                                     name.rfind("bpml", 0) == 0 || name == "dcmap";
-        if (s->ready && relaxation_map && d.isotropic) return recode(s);
+        if (s->ready && relaxation_map && d.attenuation_model == 0) return recode(s);
         return FW_OK;
     }
     if (name == "dmap") {
@@ -1486,8 +1522,8 @@ int fw_sim_relaxation_codes(fw_sim* s, int32_t* n_codes, double* coded_fraction)
         int rc = finalize(s);
         if (rc != FW_OK) return rc;
     }
-    *n_codes = s->ncodes;
-    if (coded_fraction) *coded_fraction = s->ncell ? (double)s->coded_cells / (double)s->ncell : 0.0;
+    *n_codes = s->d.isotropic ? s->ncodes : 0;
+    if (coded_fraction) *coded_fraction = s->ncell && s->d.isotropic ? (double)s->coded_cells / (double)s->ncell : 0.0;
     return FW_OK;
 }
 

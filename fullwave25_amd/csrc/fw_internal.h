@@ -37,7 +37,7 @@ struct DevSim {
     const float* coef;  // [ndmap][ndim][9], w and e already divided by the axis spacing
     int32_t ndmap;
     int32_t coef_axes_same;  // 1: every axis has the same set for each dcmap value (equal spacings)
-    int32_t isotropic;
+    int32_t isotropic;  // every axis has axis 0's maps (the isotropic model, or per-axis maps that are the same)
     // exponential-attenuation model: no memory variables; v and p are scaled by aexp after
     // their update (aexp == nullptr for the relaxation model)
     const float* aexp;
@@ -428,6 +428,13 @@ struct StreamSet {
     float* w[kMaxStreams];
 };
 hipError_t launch_streams(const StreamSet& a, int nr, int nw, int64_t n, hipStream_t st);
+// pairs of maps to compare bit for bit
+struct MapPairs {
+    const float* a[2 * 5 * (kMaxDim - 1)];
+    const float* b[2 * 5 * (kMaxDim - 1)];
+    int n;
+};
+hipError_t launch_maps_differ(const MapPairs& m, int64_t n, int32_t* differ, hipStream_t st);
 hipError_t launch_code_insert(const CodeMaps& m, int64_t n, unsigned long long* keys, uint32_t nslots, uint32_t* count,
                               int32_t* rep, int32_t* status, hipStream_t st);
 hipError_t launch_code_assign(const CodeMaps& m, int64_t n, const unsigned long long* keys, uint32_t nslots,

@@ -142,7 +142,7 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
     if (f->nshots != 1) return fw::set_error(FW_ERR_UNSUPPORTED, "the adjoint runs single-transmit handles");
     if (checkpoint_every < 0) return fw::set_error(FW_ERR_INVALID, "checkpoint_every must be >= 0");
     Guard g(f->device);
-    int rc = fw::prepare(f);
+    int rc = fw::prepare_untuned(f);  // tape_kernels sets the kernels
     if (rc != FW_OK) return rc;
     tape_kernels(f);
     if ((rc = fw::refit_boundary(f)) != FW_OK) return rc;
@@ -160,7 +160,7 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
         fw_adj_destroy(a);
         return code;
     };
-    auto dalloc = [&](void** p, size_t bytes) -> bool { return hipMalloc(p, bytes ? bytes : 4) == hipSuccess; };
+    auto dalloc = [&](void** p, size_t bytes) -> bool { return fw::device_alloc(f, p, bytes ? bytes : 4) == hipSuccess; };
     if (!dalloc((void**)&a->ckpt, (size_t)(a->nckpt * f->nstate) * 4) ||
         !dalloc((void**)&a->tape, (size_t)(a->every * (nd + 1) * n) * 4) ||
         !dalloc((void**)&a->lam, (size_t)f->nstate * 4) || !dalloc((void**)&a->work, (size_t)((3 * nd + 2) * n) * 4) ||
@@ -352,7 +352,7 @@ int fw_adj_destroy(fw_adj* a) {
     if (a->f->stream) (void)hipStreamSynchronize(a->f->stream);
     for (void* p : {(void*)a->ckpt, (void*)a->tape, (void*)a->lam, (void*)a->work, (void*)a->grec, (void*)a->vox,
                     (void*)a->first, (void*)a->order, (void*)a->vmask, (void*)a->kind, (void*)a->dc8})
-        if (p) (void)hipFree(p);
+        fw::device_free(a->f, p);
     delete a;
     return FW_OK;
 }

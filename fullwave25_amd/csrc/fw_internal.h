@@ -428,6 +428,11 @@ struct StreamSet {
     float* w[kMaxStreams];
 };
 hipError_t launch_streams(const StreamSet& a, int nr, int nw, int64_t n, hipStream_t st);
+// the occupied slots of the hash table (*n counts them; n starts at 0), and codes by slot
+hipError_t launch_code_compact(const unsigned long long* keys, const uint32_t* count, const int32_t* rep, uint32_t nslots,
+                               uint32_t* n, uint32_t* slot, uint32_t* slot_count, int32_t* slot_rep, hipStream_t st);
+hipError_t launch_code_scatter(const uint32_t* slot, int32_t n, uint16_t* slot_code, hipStream_t st);
+hipError_t launch_out_of_range(const int32_t* v, int64_t n, int32_t limit, int32_t* bad, hipStream_t st);
 // pairs of maps to compare bit for bit
 struct MapPairs {
     const float* a[2 * 5 * (kMaxDim - 1)];

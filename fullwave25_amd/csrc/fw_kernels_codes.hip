@@ -157,6 +157,33 @@ __global__ __launch_bounds__(256) void k_code_table(CodeMaps m, int32_t ncodes, 
     rv[6] = rv[7] = rp[6] = rp[7] = 0.f;
 }
 
+// The occupied slots of the hash table, in any order: slot, count and lowest cell of each.
+__global__ __launch_bounds__(256) void k_code_compact(const unsigned long long* keys, const uint32_t* count,
+                                                      const int32_t* rep, uint32_t nslots, uint32_t* n, uint32_t* slot,
+                                                      uint32_t* slot_count, int32_t* slot_rep) {
+    for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < nslots; q += gridDim.x * blockDim.x) {
+        if (!keys[q]) continue;
+        const uint32_t at = atomicAdd(n, 1u);
+        slot[at] = q;
+        slot_count[at] = count[q];
+        slot_rep[at] = rep[q];
+    }
+}
+
+// slot_code[slot[i]] = i for the n slots that get codes (the rest of slot_code holds the escape)
+__global__ __launch_bounds__(256) void k_code_scatter(const uint32_t* slot, int32_t n, uint16_t* slot_code) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) slot_code[slot[i]] = (uint16_t)i;
+}
+
+// *bad = 1 if any of the n values is outside [0, limit)
+__global__ __launch_bounds__(256) void k_out_of_range(const int32_t* v, int64_t n, int32_t limit, int32_t* bad) {
+    bool b = false;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
+        b |= (uint32_t)v[t] >= (uint32_t)limit;
+    if (b) *bad = 1;
+}
+
 // Whether arrays of n words differ: *differ = 1 if any a[k] is not b[k] bit for bit. One read of every
 // array at the copy rate (30 maps of a 400 x 400 x 360 grid: 1.2 ms, once).
 __global__ __launch_bounds__(256) void k_maps_differ(MapPairs m, int64_t n4, int32_t* differ) {
@@ -234,6 +261,24 @@ hipError_t launch_code_table(const CodeMaps& m, int32_t ncodes, const int32_t* r
     if (ncodes <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_code_table, dim3((unsigned)((ncodes + 255) / 256)), dim3(256), 0, st, m, ncodes, rep_of_code,
                        tab_v, tab_p);
+    return hipGetLastError();
+}
+
+hipError_t launch_code_compact(const unsigned long long* keys, const uint32_t* count, const int32_t* rep, uint32_t nslots,
+                               uint32_t* n, uint32_t* slot, uint32_t* slot_count, int32_t* slot_rep, hipStream_t st) {
+    hipLaunchKernelGGL(k_code_compact, code_grid(nslots), dim3(256), 0, st, keys, count, rep, nslots, n, slot, slot_count,
+                       slot_rep);
+    return hipGetLastError();
+}
+
+hipError_t launch_code_scatter(const uint32_t* slot, int32_t n, uint16_t* slot_code, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_code_scatter, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, slot, n, slot_code);
+    return hipGetLastError();
+}
+
+hipError_t launch_out_of_range(const int32_t* v, int64_t n, int32_t limit, int32_t* bad, hipStream_t st) {
+    hipLaunchKernelGGL(k_out_of_range, code_grid(n), dim3(256), 0, st, v, n, limit, bad);
     return hipGetLastError();
 }
 

@@ -45,6 +45,7 @@ struct fw_sim {
     std::vector<fw::GroupBoundary> fbound_h;  // what fbound holds
     bool pinned[2] = {false, false};  // set by fw_sim_set_kernel_config: not autotuned
     fw::LaunchCfg pin[2];
+    bool untuned = false;  // prepare_untuned: the first run's set-up leaves the default kernels
     bool fields_set = false;  // a field was set before the first run: do not tune on it
     bool state_zero = true;   // every wave field is known to be zero (created or reset, not run since)
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -73,6 +74,10 @@ namespace fw {
 // host helpers of fw_api.cpp used by the adjoint
 int set_error(int code, const char* fmt, ...);
 int prepare(fw_sim* s);                    // check inputs, resolve coordinates, pick kernels
+int prepare_untuned(fw_sim* s);            // the same without timing kernels, for a caller that sets them
+// device memory of the handle, ordered on its stream
+hipError_t device_alloc(fw_sim* s, void** p, size_t bytes);
+void device_free(fw_sim* s, void* p);
 int refit_boundary(fw_sim* s);             // the point table again, after a change of the pressure kernel
 int forward_step(fw_sim* s);               // one time step on the handle's stream
 hipError_t grid_to_host(const fw_sim* s, void* dst, const void* src, size_t esize);  // padded -> compact

@@ -879,7 +879,7 @@ def sweep(args) -> int:
     shapes += [f"tile:{c}" for c in (8, 16, 32)]
     if inp.ndim == 3:
         shapes = ["percell"] + [f"{v}:{w}:{c}" for v in ("stream", "pipe", "pipelite") for w in (512, 1024)
-                                for c in (8, 16, 32)]
+                                for c in (8, 16, 32)] + ["brick:32:0", "brick:32:1"]
     if args.sweep_shapes:
         shapes = args.sweep_shapes.split(",")
     upd = updated_cells(inp)

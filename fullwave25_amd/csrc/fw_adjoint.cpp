@@ -116,14 +116,19 @@ int64_t auto_segment(const fw_sim* f, size_t free_bytes) {
     return std::min<int64_t>(nt, std::max<int64_t>(1, (int64_t)std::ceil(c)));
 }
 
-// Kernels that write the tape (the tiled 2D or per-cell families): the tiled ones (8 rows) where
-// the grid takes them, else the per-cell ones; a kernel the caller pinned stays if it writes
-// the tape.
+// Kernels that write the tape (the tiled 2D, brick 3D or per-cell families): the tiled ones (8 rows)
+// or bricks where the grid takes them (136 x 120 x 112: a taped step 85 -> 58 us), else the per-cell
+// ones; a kernel the caller pinned stays if it writes the tape.
 void tape_kernels(fw_sim* f) {
     fw::LaunchCfg t;
     t.variant = 2;
     t.width = 256;
     t.chunk = 8;
+    if (!fw::tape_capable(f->ds, t)) {
+        t.variant = 5;
+        t.width = fw::kBrickZ;
+        t.chunk = 1;
+    }
     if (!fw::tape_capable(f->ds, t)) t.variant = 0;
     for (int kind = 0; kind < 2; ++kind) {
         fw::LaunchCfg& c = kind == 0 ? f->cfg_v : f->cfg_p;

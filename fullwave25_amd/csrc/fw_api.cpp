@@ -422,6 +422,15 @@ int check_cfg(fw_sim* s, const fw::LaunchCfg& c) {
         if (c.chunk < 1 || c.chunk > 4096) return fail(FW_ERR_INVALID, "pipelined kernels: chunk out of range");
         return FW_OK;
     }
+    if (c.variant == 5) {
+        if (!fw::brick_supported(s->ds))
+            return fail(FW_ERR_UNSUPPORTED,
+                        "brick kernels need a 3D grid of fewer than 2^30 cells with equal spacings and at most 16384 "
+                        "coefficient codes, or the exponential model");
+        if (c.width != fw::kBrickZ || c.chunk < 0 || c.chunk > 1)
+            return fail(FW_ERR_INVALID, "brick kernels: width 32, chunk 0 or 1");
+        return FW_OK;
+    }
     if (c.variant == 1) {
         if (!fw::streaming_supported(s->ds)) return fail(FW_ERR_UNSUPPORTED, "this grid needs the per-cell kernels");
         if (s->ndim == 2 && c.width != 64 && c.width != 128 && c.width != 256)
@@ -431,7 +440,7 @@ int check_cfg(fw_sim* s, const fw::LaunchCfg& c) {
         if (c.chunk < 2 || c.chunk > 4096) return fail(FW_ERR_INVALID, "x-marching kernels: chunk out of range");
         return FW_OK;
     }
-    return fail(FW_ERR_INVALID, "kernel variant must be 0 to 4");
+    return fail(FW_ERR_INVALID, "kernel variant must be 0 to 5");
 }
 
 int parse_kernel_env(fw_sim* s, const char* env, fw::LaunchCfg* out) {
@@ -459,6 +468,16 @@ int parse_kernel_env(fw_sim* s, const char* env, fw::LaunchCfg* out) {
         if (n >= 2) c.chunk = ch;
         int rc = check_cfg(s, c);
         if (rc != FW_OK) return rc;
+    } else if (!strncmp(env, "brick", 5)) {
+        c.variant = 5;
+        c.width = fw::kBrickZ;
+        c.chunk = 1;
+        int w = 0, ch = 0;
+        int n = sscanf(env + 5, ":%d:%d", &w, &ch);
+        if (n >= 1) c.width = w;
+        if (n >= 2) c.chunk = ch;
+        int rc = check_cfg(s, c);
+        if (rc != FW_OK) return rc;
     } else if (!strncmp(env, "stream", 6)) {
         if (!stream_ok) return fail(FW_ERR_UNSUPPORTED, "FULLWAVE_HIP_KERNELS=stream: this grid needs the per-cell kernels");
         c.variant = 1;
@@ -470,7 +489,7 @@ int parse_kernel_env(fw_sim* s, const char* env, fw::LaunchCfg* out) {
         if (rc != FW_OK) return rc;
     } else {
         return fail(FW_ERR_INVALID,
-                    "FULLWAVE_HIP_KERNELS must be 'percell', 'stream[:width[:chunk]]', 'tile[:rows]' or 'pipe[:width[:chunk]]'");
+                    "FULLWAVE_HIP_KERNELS must be 'percell', 'stream[:width[:chunk]]', 'tile[:rows]', 'pipe[:width[:chunk]]' or 'brick[:32[:0|1]]'");
     }
     *out = c;
     return FW_OK;
@@ -479,7 +498,8 @@ int parse_kernel_env(fw_sim* s, const char* env, fw::LaunchCfg* out) {
 int choose_kernels_unpinned(fw_sim* s);
 
 // Pick the kernel family and shape of each stencil kernel for this grid.
-// FULLWAVE_HIP_KERNELS overrides both: "percell", "stream[:width[:chunk]]" or "tile[:rows]",
+// FULLWAVE_HIP_KERNELS overrides both: "percell", "stream[:width[:chunk]]", "tile[:rows]",
+// "pipe[:width[:chunk]]", "pipelite[:width[:chunk]]" or "brick[:32[:order]]",
 // or each on its own as "<velocity>/<pressure>" (e.g. "tile:8/stream:256:8").
 // Otherwise every candidate is timed on the handle's own arrays while the wave state is still
 // all zero (the update then leaves it zero, so the timing runs change nothing), and the
@@ -519,9 +539,16 @@ int choose_kernels_unpinned(fw_sim* s) {
     def.variant = stream_ok ? 1 : 0;
     def.width = s->ndim == 3 ? 512 : 256;
     def.chunk = 8;
+    const bool bricks = fw::brick_supported(s->ds);
+    if (bricks) {
+        def.variant = 5;
+        def.width = fw::kBrickZ;
+        def.chunk = 1;
+    }
     s->cfg_v = s->cfg_p = def;
     // a fixed-region handle has no timing events: the default shapes
-    if (s->fields_set || s->fixed_base || s->untuned || !stream_ok || (s->pinned[0] && s->pinned[1])) return FW_OK;
+    if (s->fields_set || s->fixed_base || s->untuned || (!stream_ok && !bricks) || (s->pinned[0] && s->pinned[1]))
+        return FW_OK;
     // Families of candidates whose members differ in the planes (rows) a workgroup takes, ascending: the
     // rest of a family is left out once two in a row are 10 % slower than its best (on small grids more
     // planes a workgroup only make fewer workgroups). The plain 3D marching kernels are behind the
@@ -548,9 +575,10 @@ int choose_kernels_unpinned(fw_sim* s) {
         if (fw::tile2d_supported(s->ds)) family(2, 256, {8, 16, 32});
     } else {
         const bool pipes = s->ncell < ((int64_t)1 << 30);
+        if (bricks) family(5, fw::kBrickZ, {0, 1});
         for (int v : {1, 3, 4})
             for (int w : {512, 1024})
-                if (pipes == (v != 1)) family(v, w, {8, 16, 32, 48, 64, 96, 128});
+                if (stream_ok && pipes == (v != 1)) family(v, w, {8, 16, 32, 48, 64, 96, 128});
     }
     for (int kind = 0; kind < 2; ++kind) {
         if (s->pinned[kind]) continue;
@@ -824,7 +852,9 @@ int setup_fused_boundary(fw_sim* s, const fw::BoundaryLists& bl) {
     const fw::LaunchCfg& c = s->cfg_p;
     std::vector<int32_t> pts;
     fw::PointTable pt;
-    if (c.variant == 0) {
+    if (c.variant == 5) {
+        pt = fw::point_table_bricks(fw::brick_grid(s->ds), s->ds.sx, s->ds.sy, bl, &pts);
+    } else if (c.variant == 0) {
         const int64_t pitch = s->ndim == 2 ? s->ds.sx : s->ds.sy;
         pt = fw::point_table_rows(fw::cell_first_row(s->ds), fw::cell_row_count(s->ds), pitch, fw::cell_tiles_x(s->ds),
                                   fw::kCellTileCols, fw::kCellTileRows, bl, &pts);
@@ -1582,7 +1612,7 @@ int fw_sim_set_kernel_config(fw_sim* s, int32_t kind, int32_t variant, int32_t w
     if (!s) return fail(FW_ERR_INVALID, "null handle");
     if (kind != 0 && kind != 1) return fail(FW_ERR_INVALID, "kind must be 0 (velocity) or 1 (pressure)");
     if (s->ready) return fail(FW_ERR_STATE, "the kernels are fixed at the first run; set them before it");
-    if (variant < 0 || variant > 4) return fail(FW_ERR_INVALID, "kernel variant must be 0 to 4");
+    if (variant < 0 || variant > 5) return fail(FW_ERR_INVALID, "kernel variant must be 0 to 5");
     fw::LaunchCfg c;
     c.variant = variant;
     c.width = width;

@@ -40,20 +40,16 @@ namespace fw {
 
 namespace {
 
-// points_by_tile over contiguous rows [first, first + count) of `pitch` elements
-void points_by_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows,
-                    const std::vector<int64_t>& lin, std::vector<int32_t>* off, std::vector<int32_t>* idx) {
-    const size_t ntiles = (size_t)gx * (size_t)((count + rows - 1) / rows);
+// The points of `lin` grouped by owner(linear index) in [0, ntiles); entries < 0 left out.
+template <class Owner>
+void points_by_owner(size_t ntiles, const Owner& owner_of, const std::vector<int64_t>& lin, std::vector<int32_t>* off,
+                     std::vector<int32_t>* idx) {
     std::vector<int64_t> owner(lin.size(), -1);
     off->assign(ntiles + 1, 0);
     for (size_t q = 0; q < lin.size(); ++q) {
         if (lin[q] < 0) continue;
-        int64_t i = lin[q] / pitch;
-        const int64_t j = lin[q] % pitch;
-        i = i < first ? first : (i > first + count - 1 ? first + count - 1 : i);
-        const int64_t t = ((i - first) / rows) * (int64_t)gx + j / tile_w;
-        owner[q] = t;
-        ++(*off)[(size_t)t + 1];
+        owner[q] = owner_of(lin[q]);
+        ++(*off)[(size_t)owner[q] + 1];
     }
     for (size_t t = 0; t < ntiles; ++t) (*off)[t + 1] += (*off)[t];
     idx->assign((size_t)(*off)[ntiles], 0);
@@ -62,20 +58,19 @@ void points_by_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, in
         if (owner[q] >= 0) (*idx)[(size_t)fill[(size_t)owner[q]]++] = (int32_t)q;
 }
 
-}  // namespace
+int64_t clamped(int64_t v, int64_t lo, int64_t hi) { return v < lo ? lo : v > hi ? hi : v; }
 
-void points_by_tile(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const std::vector<int64_t>& lin,
-                    std::vector<int32_t>* off, std::vector<int32_t>* idx) {
-    points_by_rows(kHalo, nx - 2 * kHalo, ny, gx, tile_w, rows, lin, off, idx);
+// tiles of `tile_w` cells by `rows` contiguous rows of `pitch` elements, from row `first` of `count`; a
+// point outside those rows belongs to the nearest
+auto rows_owner(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows) {
+    return [=](int64_t lin) {
+        return (clamped(lin / pitch, first, first + count - 1) - first) / rows * (int64_t)gx + lin % pitch / tile_w;
+    };
 }
 
-PointTable point_table(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const BoundaryLists& bl,
-                       std::vector<int32_t>* tab) {
-    return point_table_rows(kHalo, nx - 2 * kHalo, ny, gx, tile_w, rows, bl, tab);
-}
-
-PointTable point_table_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows,
-                            const BoundaryLists& bl, std::vector<int32_t>* tab) {
+// The parts of a point table (PointTable) over `ntiles` tiles, appended to `tab`.
+template <class Owner>
+PointTable table_of(size_t ntiles, const Owner& owner_of, const BoundaryLists& bl, std::vector<int32_t>* tab) {
     auto align4 = [&] {
         while (tab->size() % 4) tab->push_back(0);
     };
@@ -85,9 +80,9 @@ PointTable point_table_rows(int64_t first, int64_t count, int64_t pitch, unsigne
     };
     std::vector<int32_t> off[3], idx[3];
     const std::vector<int64_t>* lists[3] = {&bl.src_lin, &bl.zero_lin, &bl.out_lin};
-    for (int k = 0; k < 3; ++k) points_by_rows(first, count, pitch, gx, tile_w, rows, *lists[k], &off[k], &idx[k]);
+    for (int k = 0; k < 3; ++k) points_by_owner(ntiles, owner_of, *lists[k], &off[k], &idx[k]);
     PointTable pt{};
-    pt.ntiles = (int32_t)(off[0].size() - 1);
+    pt.ntiles = (int32_t)ntiles;
     align4();
     pt.off = tab->size();
     for (int k = 0; k < 3; ++k) tab->insert(tab->end(), off[k].begin(), off[k].end());
@@ -108,6 +103,37 @@ PointTable point_table_rows(int64_t first, int64_t count, int64_t pitch, unsigne
         push_lin(bl.out_air[(size_t)q] ? -1 : bl.out_lin[(size_t)q]);
     }
     return pt;
+}
+
+size_t row_tiles(int64_t count, unsigned gx, int rows) { return (size_t)gx * (size_t)((count + rows - 1) / rows); }
+
+}  // namespace
+
+void points_by_tile(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const std::vector<int64_t>& lin,
+                    std::vector<int32_t>* off, std::vector<int32_t>* idx) {
+    const int64_t count = nx - 2 * kHalo;
+    points_by_owner(row_tiles(count, gx, rows), rows_owner(kHalo, count, ny, gx, tile_w, rows), lin, off, idx);
+}
+
+PointTable point_table(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows, const BoundaryLists& bl,
+                       std::vector<int32_t>* tab) {
+    return point_table_rows(kHalo, nx - 2 * kHalo, ny, gx, tile_w, rows, bl, tab);
+}
+
+PointTable point_table_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows,
+                            const BoundaryLists& bl, std::vector<int32_t>* tab) {
+    return table_of(row_tiles(count, gx, rows), rows_owner(first, count, pitch, gx, tile_w, rows), bl, tab);
+}
+
+PointTable point_table_bricks(const BrickGrid& g, int64_t sx, int64_t sy, const BoundaryLists& bl,
+                              std::vector<int32_t>* tab) {
+    auto owner = [=](int64_t lin) {  // points outside the bricks belong to the nearest
+        const int64_t bx = clamped((lin / sx - kHalo) / kBrickX, 0, g.nx - 1);
+        const int64_t by = clamped((lin % sx / sy - kHalo) / kBrickY, 0, g.ny - 1);
+        const int64_t bz = clamped(lin % sy / kBrickZ, 0, g.nz - 1);
+        return (bx * g.ny + by) * g.nz + bz;
+    };
+    return table_of((size_t)(g.nx * g.ny * g.nz), owner, bl, tab);
 }
 
 }  // namespace fw

@@ -374,6 +374,8 @@ enum KernelKind { kVelocity = 0, kPressure = 1, kBoundary = 2, kNumKinds = 3 };
 //   variant 3: 3D x-marching kernels with software pipelining (planes and per-cell operands
 //              loaded one iteration ahead); `width` = workgroup size 512 or 1024
 //   variant 4: as 3, with the per-cell operands loaded at the top of their own iteration
+//   variant 5: 3D brick kernels (brick_supported), workgroups of 256 lanes on bricks of 4 x 8 x 32 cells;
+//              `width` 32, `chunk` 1 where each XCD takes a contiguous run of the bricks, else 0
 struct LaunchCfg {
     int variant = 0;
     int width = 128;
@@ -391,8 +393,17 @@ bool streaming_supported(const DevSim& s);
 bool tile2d_supported(const DevSim& s);
 int tile2d_width(int rows);  // columns of the tile of `rows` rows (8, 16 or 32)
 hipError_t launch_velocity(const DevSim& s, const LaunchCfg& cfg, hipStream_t st);
+// 3D brick kernels (gs as for launch_pressure): bricks of kBrickX x kBrickY x kBrickZ cells from x = y = 8,
+// z = 0, z fastest
+constexpr int kBrickX = 4, kBrickY = 8, kBrickZ = 32;
+struct BrickGrid {
+    int64_t nx, ny, nz;
+};
+bool brick_supported(const DevSim& s);
+BrickGrid brick_grid(const DevSim& s);
+hipError_t launch_brick(const DevSim& s, const LaunchCfg& cfg, bool velocity, const GroupStep& gs, hipStream_t st);
 hipError_t launch_pipe3d(const DevSim& s, const LaunchCfg& cfg, bool velocity, hipStream_t st);
-// gs.g non-null (pressure_fuses_boundary: the per-cell, the 2D marching and the tiled kernels): the
+// gs.g non-null (pressure_fuses_boundary: the per-cell, the brick, the 2D marching and the tiled kernels): the
 // pressure launch also does the step's sources, pressure release and sensors (tile_boundary;
 // gs.g holds one entry per shot, whose points are grouped by the tiles of `cfg`)
 hipError_t launch_pressure(const DevSim& s, const LaunchCfg& cfg, hipStream_t st, const GroupStep& gs = GroupStep{});

@@ -470,17 +470,18 @@ bool tile2d_supported(const DevSim& s);
 hipError_t launch_tile2d(const DevSim& s, const LaunchCfg& cfg, bool velocity, const GroupStep& gs, hipStream_t st);
 
 bool tape_capable(const DevSim& s, const LaunchCfg& cfg) {
-    return cfg.variant == 0 || (cfg.variant == 2 && tile2d_supported(s));
+    return cfg.variant == 0 || (cfg.variant == 2 && tile2d_supported(s)) || (cfg.variant == 5 && brick_supported(s));
 }
 
-// A step that writes the adjoint tape runs the tiled 2D kernels when `cfg` asks for them and the
-// per-cell kernels otherwise (the only families that write it).
+// A step that writes the adjoint tape runs the tiled 2D or the brick kernels when `cfg` asks for them
+// and the per-cell kernels otherwise (the only families that write it).
 hipError_t launch_velocity(const DevSim& s, const LaunchCfg& cfg, hipStream_t st) {
     if (cfg.variant == 2 && tile2d_supported(s)) return launch_tile2d(s, cfg, true, GroupStep{}, st);
+    if (cfg.variant == 5 && brick_supported(s)) return launch_brick(s, cfg, true, GroupStep{}, st);
     if (s.tape_div) return launch_simple(s, true, GroupStep{}, st);
     if ((cfg.variant == 3 || cfg.variant == 4) && s.ndim == 3 && streaming_supported(s))
         return launch_pipe3d(s, cfg, true, st);
-    if (cfg.variant == 0 || !streaming_supported(s)) return launch_simple(s, true, GroupStep{}, st);
+    if (cfg.variant == 0 || cfg.variant == 5 || !streaming_supported(s)) return launch_simple(s, true, GroupStep{}, st);
     if (s.ndim == 3) return launch_velocity_3d(s, cfg, st);
     return launch_2d_any(s, cfg, true, GroupStep{}, st);
 }
@@ -491,6 +492,10 @@ constexpr int64_t kMaxPointTiles = 1 << 18;
 
 bool pressure_fuses_boundary(const DevSim& s, const LaunchCfg& cfg) {
     if (cfg.variant == 0) return cell_tiles(s) <= kMaxPointTiles;
+    if (cfg.variant == 5) {
+        const BrickGrid g = brick_grid(s);
+        return brick_supported(s) && g.nx * g.ny * g.nz <= kMaxPointTiles;
+    }
     if (s.ndim != 2) return false;
     if (cfg.variant == 2) return tile2d_supported(s) && !(s.tape_div && cfg.chunk != 8);  // taped: 8-row tiles
     return cfg.variant == 1 && !s.tape_div && streaming_supported(s);
@@ -499,10 +504,11 @@ bool pressure_fuses_boundary(const DevSim& s, const LaunchCfg& cfg) {
 hipError_t launch_pressure(const DevSim& s, const LaunchCfg& cfg, hipStream_t st, const GroupStep& gs) {
     if (gs.g && !pressure_fuses_boundary(s, cfg)) return hipErrorInvalidValue;
     if (cfg.variant == 2 && tile2d_supported(s)) return launch_tile2d(s, cfg, false, gs, st);
+    if (cfg.variant == 5 && brick_supported(s)) return launch_brick(s, cfg, false, gs, st);
     if (s.tape_div) return launch_simple(s, false, gs, st);
     if ((cfg.variant == 3 || cfg.variant == 4) && s.ndim == 3 && streaming_supported(s))
         return launch_pipe3d(s, cfg, false, st);
-    if (cfg.variant == 0 || !streaming_supported(s)) return launch_simple(s, false, gs, st);
+    if (cfg.variant == 0 || cfg.variant == 5 || !streaming_supported(s)) return launch_simple(s, false, gs, st);
     if (s.ndim == 3) return launch_pressure_3d(s, cfg, st);
     return launch_2d_any(s, cfg, false, gs, st);
 }

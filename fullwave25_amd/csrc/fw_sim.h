@@ -115,6 +115,9 @@ PointTable point_table(int64_t nx, int64_t ny, unsigned gx, int tile_w, int rows
 // of `count` rows (`pitch` elements each).
 PointTable point_table_rows(int64_t first, int64_t count, int64_t pitch, unsigned gx, int tile_w, int rows,
                             const BoundaryLists& bl, std::vector<int32_t>* tab);
+// The same for the 3D brick kernels, on a grid whose rows and planes are sy and sx elements.
+PointTable point_table_bricks(const BrickGrid& g, int64_t sx, int64_t sy, const BoundaryLists& bl,
+                              std::vector<int32_t>* tab);
 // Coefficient table [ndmap][ndim][9] (w_1..w_8, e) from dmap [9][2][ndmap] with each axis's spacing
 // folded in; *axes_same = 1 when every axis has the same set for each sound speed.
 std::vector<float> coefficient_table(const fw_desc& d, const std::vector<float>& dmap, int* axes_same);

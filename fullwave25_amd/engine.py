@@ -38,7 +38,7 @@ EXPORTED_SYMBOLS = (
     "fw_group_run", "fw_group_set_graph_steps", "fw_group_destroy",
     "fw_adj_create", "fw_adj_checkpoint_every", "fw_adj_forward", "fw_adj_backward", "fw_adj_destroy",
 )
-VARIANTS = {"percell": 0, "stream": 1, "tile": 2, "pipe": 3, "pipelite": 4}
+VARIANTS = {"percell": 0, "stream": 1, "tile": 2, "pipe": 3, "pipelite": 4, "brick": 5}
 
 
 class EngineError(RuntimeError):
@@ -284,7 +284,7 @@ class HipSimulation:
         for kind, label in ((0, "velocity"), (1, "pressure")):
             v, w, c = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
             _check(self.lib, self.lib.fw_sim_kernel_config(self._h, kind, ctypes.byref(v), ctypes.byref(w), ctypes.byref(c)))
-            name = {0: "percell", 1: "stream", 2: "tile", 3: "pipe", 4: "pipelite"}.get(v.value, str(v.value))
+            name = {0: "percell", 1: "stream", 2: "tile", 3: "pipe", 4: "pipelite", 5: "brick"}.get(v.value, str(v.value))
             out[label] = {"variant": name, "width": w.value, "chunk": c.value}
         return out
 

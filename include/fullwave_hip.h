@@ -151,11 +151,13 @@ int fw_sim_set_field(fw_sim* sim, const char* name, const float* values, size_t 
  * 2 = 2D tiled kernels with 4-wide vector access (workgroups of `width` = 256 lanes on tiles of
  * `chunk` rows),
  * 3 / 4 = 3D software-pipelined x-marching kernels (workgroups of `width` = 512 or 1024 lanes;
- * per-cell operands loaded one iteration ahead / at the top of their iteration).
+ * per-cell operands loaded one iteration ahead / at the top of their iteration),
+ * 5 = 3D brick kernels (workgroups of 256 lanes on 4 x 8 x 32 cells; `width` 32, `chunk` 1 where
+ * each XCD takes a contiguous run of the bricks, else 0).
  * Chosen on the first run by timing the candidates on the handle's own arrays, separately for
  * the two kernels (or forced for both with
  * the FULLWAVE_HIP_KERNELS environment variable: "percell", "stream[:width[:chunk]]",
- * "tile[:rows]", "pipe[:width[:chunk]]" or "pipelite[:width[:chunk]]", or
+ * "tile[:rows]", "pipe[:width[:chunk]]", "pipelite[:width[:chunk]]" or "brick[:32[:order]]", or
  * "<velocity>/<pressure>" to set each on its own).
  * Calling this before the first run makes that choice. */
 int fw_sim_kernel_config(fw_sim* sim, int32_t kind, int32_t* variant, int32_t* width, int32_t* chunk);

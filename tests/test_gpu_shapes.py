@@ -79,6 +79,60 @@ def test_3d_families_agree_bit_for_bit(monkeypatch, shape, kind):
                 np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("model", ["isotropic", "exponential"])
+@pytest.mark.parametrize("kind", ["one", "patches", "cells"])
+@pytest.mark.parametrize("shape", [(17, 17, 17), (20, 24, 40), (21, 25, 41), (18, 33, 109), (19, 32, 131)])
+def test_3d_bricks_equal_the_per_cell_kernels(monkeypatch, shape, kind, model):
+    """Brick kernels at the edges of bricks (4 x 8 x 32 cells): one cell, whole bricks, one more; shared,
+    per-cell and mixed coefficients; both orders of the bricks; sources, pressure release and sensors on
+    corners, ghost border and brick edges fused into the pressure launch and on their own; two shots; the
+    adjoint's taped run. Bit for bit."""
+    from fullwave25_amd.adjoint import HipAdjoint
+
+    rng = np.random.default_rng(11)
+    corners = np.stack(np.meshgrid(*[[0, n - 1] for n in shape], indexing="ij"), -1).reshape(-1, 3)
+    inside = np.stack([rng.integers(0, n, 30) for n in shape], 1)
+    edge = inside.copy()
+    edge[:, -1] = np.minimum(rng.choice([8, 31, 32, 33], 30), shape[-1] - 1)
+    src, out, air = (np.concatenate([corners, inside[i::3], edge[i::3]]) for i in range(3))
+    nt = 9
+    more = {}
+    if model == "exponential":
+        more = {"a_exp": 0.98 + 0.02 * rng.random(shape)}
+    c = {"one": 1540.0, "patches": np.where(np.arange(shape[0])[:, None, None] < shape[0] // 2, 1500.0, 1560.0) * np.ones(shape),
+         "cells": rng.choice([1500.0, 1523.0, 1580.0], size=shape)}[kind]
+    inp = raw_inputs(shape, c=c, rho=950 + 100 * rng.random(shape), nt=nt, icc=src, modt=2, outc=np.concatenate([out, src[4:], air[:6]]),
+                     icmat=rng.standard_normal((len(src), nt)).astype(np.float32), icczero=air, **more)
+    want = run(inp, "percell", monkeypatch)
+    assert np.abs(want[1]).max() > 0
+    for order in (0, 1):
+        for fused in ("1", "0"):
+            monkeypatch.setenv("FULLWAVE_HIP_FUSED_BOUNDARY", fused)
+            print(f"{shape} {kind} {model}: order {order} fused {fused}", flush=True)
+            for got, ref in zip(run(inp, f"brick:32:{order}", monkeypatch), want):
+                np.testing.assert_array_equal(got, ref)
+    monkeypatch.delenv("FULLWAVE_HIP_FUSED_BOUNDARY")
+    shots = np.stack([inp.icmat, 0.5 * inp.icmat[::-1]])
+    traces = {}
+    for k in ("percell", "brick:32:1"):
+        monkeypatch.setenv("FULLWAVE_HIP_KERNELS", k)
+        with engine.HipSimulation(inp, shots=shots) as sim:
+            sim.run(nt)
+            traces[k] = sim.sensors()
+    np.testing.assert_array_equal(traces["brick:32:1"], traces["percell"])
+    monkeypatch.delenv("FULLWAVE_HIP_KERNELS")
+    weights = rng.standard_normal((inp.n_records, inp.ncoordsout)).astype(np.float32)
+    grads = []
+    for variant, width in (("percell", 0), ("brick", 32)):
+        one = {"variant": variant, "width": width, "chunk": 0}
+        with HipAdjoint(inp, checkpoint_every=4, kernel_config={"velocity": one, "pressure": one}) as adj:
+            assert adj.sim.kernel_config()["velocity"]["variant"] == variant
+            adj.forward()
+            grads.append(adj.backward(weights))
+    for a, b in zip(*grads):
+        np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("model", ["isotropic", "per_axis", "exponential"])
 @pytest.mark.parametrize("shape", [(17, 17), (21, 65), (40, 200), (17, 18, 19), (19, 21, 67)])
 def test_per_cell_boundary_work_matches_boundary_launch(monkeypatch, shape, model):

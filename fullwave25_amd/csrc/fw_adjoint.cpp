@@ -35,8 +35,9 @@ struct fw_adj {
     int32_t* first = nullptr;
     int32_t* order = nullptr;
     int8_t* vmask = nullptr;  // per distinct voxel: 1 pressure release, 2 source point, 0 neither
-    uint8_t* kind = nullptr;  // per device cell (2D): bit 0 pressure release, 1 source point, 2 sensor voxel
-    uint8_t* dc8 = nullptr;   // per device cell: coefficient-set index (grids of the tiled reverse kernels)
+    uint8_t* kind = nullptr;  // per device cell (2D, bricks): bit 0 pressure release, 1 source point, 2 sensor voxel
+    uint8_t* dc8 = nullptr;   // per device cell: coefficient-set index (grids of the tiled and brick reverse kernels)
+    uint32_t* sets = nullptr; // the set of each brick's arms (3D bricks)
     int64_t nvox = 0;
     bool forward_done = false;
 };
@@ -200,7 +201,8 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
     for (size_t t = 0; t < vox.size(); ++t) vmask[t] = zero_set.count(vox[t]) ? 1 : src_set.count(vox[t]) ? 2 : 0;
     // the same per cell, for the reverse kernels that run a step's sparse part cell by cell
     std::vector<uint8_t> kind;
-    if (nd == 2) {
+    const bool bricks = fw::adj_bricks_supported(f->ds) && !fw::adj_percell_gathers();
+    if (nd == 2 || bricks) {
         kind.assign((size_t)n, 0);
         for (int64_t z : zero) kind[(size_t)z] |= 1;
         for (int64_t q : src)
@@ -221,7 +223,11 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
         ok = ok && hipMemcpyAsync(a->kind, kind.data(), kind.size(), hipMemcpyHostToDevice, f->stream) == hipSuccess;
     if (ok && fw::adj_tiles(f->ds)) {
         if (!dalloc((void**)&a->dc8, (size_t)n)) return cleanup(fw::set_error(FW_ERR_NOMEM, "adjoint set-index map"));
-        ok = fw::launch_adj_set_index(f->ds.dcmap, a->dc8, n, f->stream) == hipSuccess;
+    }
+    if (bricks) {
+        const fw::BrickGrid g3 = fw::brick_grid(f->ds);
+        if (!dalloc((void**)&a->dc8, (size_t)n) || !dalloc((void**)&a->sets, (size_t)(g3.nx * g3.ny * g3.nz) * 4))
+            return cleanup(fw::set_error(FW_ERR_NOMEM, "adjoint set-index map"));
     }
     ok = ok && hipMemcpyAsync(a->first, first.data(), first.size() * 4, hipMemcpyHostToDevice, f->stream) == hipSuccess;
     ok = ok && hipStreamSynchronize(f->stream) == hipSuccess;
@@ -272,6 +278,10 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
     hipStream_t st = f->stream;
     const int nd = f->ndim;
     ADJ_HIP(hipMemcpyAsync(a->grec, grad_rec, grad_bytes, hipMemcpyHostToDevice, st));
+    // the set indices, of the map as it is now
+    const bool bricks = a->sets && fw::adj_bricks_supported(f->ds);
+    if (a->dc8) ADJ_HIP(fw::launch_adj_set_index(f->ds.dcmap, a->dc8, n, st));
+    if (bricks) ADJ_HIP(fw::launch_adj_brick_sets(f->ds, a->dc8, a->sets, st));
     ADJ_HIP(hipStreamSynchronize(st));  // grad_rec is the caller's buffer, read during the call only
     ADJ_HIP(hipMemsetAsync(a->lam, 0, (size_t)f->nstate * 4, st));
     ADJ_HIP(hipMemsetAsync(a->work, 0, (size_t)((3 * nd + 2) * n) * 4, st));
@@ -291,6 +301,7 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
     }
     w.gK = a->work + 3 * nd * n;
     w.dc8 = a->dc8;
+    w.sets = bricks ? a->sets : nullptr;
     float* grho = a->work + (3 * nd + 1) * n;
     fw::AdjSparse sp{};
     sp.vox = a->vox;
@@ -307,7 +318,7 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
     auto rec_row = [&](int64_t nn) -> const float* {
         return f->d.modt > 0 && nn % f->d.modt == 0 ? a->grec + (nn / f->d.modt) * nout : nullptr;
     };
-    const bool fuse = fw::adj_fuses_next(f->ds);
+    const bool fuse = fw::adj_fuses_next(f->ds, w);
     bool head_done = false;  // step nn's sparse part and pressure transposed already ran
     int rc;
     for (int64_t k = a->nckpt - 1; k >= 0; --k) {
@@ -356,7 +367,7 @@ int fw_adj_destroy(fw_adj* a) {
     Guard g(a->f->device);
     if (a->f->stream) (void)hipStreamSynchronize(a->f->stream);
     for (void* p : {(void*)a->ckpt, (void*)a->tape, (void*)a->lam, (void*)a->work, (void*)a->grec, (void*)a->vox,
-                    (void*)a->first, (void*)a->order, (void*)a->vmask, (void*)a->kind, (void*)a->dc8})
+                    (void*)a->first, (void*)a->order, (void*)a->vmask, (void*)a->kind, (void*)a->dc8, (void*)a->sets})
         fw::device_free(a->f, p);
     delete a;
     return FW_OK;

@@ -250,7 +250,8 @@ struct AdjView {
     float* lphi[kMaxDim][kNRelax];
     const float* tu[kMaxDim];
     const float* tdiv;
-    const uint8_t* dc8;  // coefficient-set index per device cell (the tiled 2D kernels; ndmap <= 256)
+    const uint8_t* dc8;  // coefficient-set index per device cell (the tiled 2D kernels; ndmap <= 256; bricks)
+    const uint32_t* sets;  // bricks: the set of each brick's arms, or all ones (null: no bricks)
     float* H[kMaxDim];
     float* G[kMaxDim];
     float* gK;               // d/dK, summed over steps
@@ -492,11 +493,37 @@ struct AdjNext {
     const int32_t* order;
     int64_t nvox;
 };
+// lambda_p[c] of the next step after its sparse part (as k_adj_sparse), from lp = lambda_p[c]
+// after this step's gathers and kd = the cell's kind
+__device__ inline float next_mu(const AdjNext& nx, int64_t c, unsigned kd, float lp) {
+    if (!kd) return lp;
+    if ((kd & 1u) || ((kd & 2u) && nx.injecting)) return 0.f;
+    if (!(kd & 4u) || !nx.grow) return lp;
+    int64_t lo = 0, hi = nx.nvox - 1;  // c is one of the sorted voxels
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (nx.vox[mid] < c) lo = mid + 1;
+        else hi = mid;
+    }
+    float acc = 0.f;
+    for (int32_t q = nx.first[lo]; q < nx.first[lo + 1]; ++q) acc += nx.grow[nx.order[q]];
+    return lp + acc;
+}
+
 // One step of the sweep, after launch_adj_sparse: launch_adj_pressure (the pressure transposed),
 // then launch_adj_rest (the rest of the step; with `next` when adj_fuses_next, also the start of
 // the next step, whose launch_adj_sparse and launch_adj_pressure are then skipped).
 bool adj_tiles(const DevSim& s);  // the grid takes the tiled 2D reverse kernels
-bool adj_fuses_next(const DevSim& s);
+bool adj_fuses_next(const DevSim& s, const AdjView& w);
+// FULLWAVE_HIP_ADJ_GATHERS=percell keeps the per-cell kernels (to compare the forms)
+bool adj_percell_gathers();
+// The 3D bricks: which grids take them; the set of each brick's arms (AdjView::sets); the two calls
+// above on them.
+constexpr int kAdjBrickSets = 256;  // sets whose weights LDS holds
+bool adj_bricks_supported(const DevSim& s);
+hipError_t launch_adj_brick_sets(const DevSim& s, const uint8_t* dc8, uint32_t* sets, hipStream_t st);
+hipError_t launch_adj_start_bricks(const DevSim& s, const AdjView& w, hipStream_t st);
+hipError_t launch_adj_rest_bricks(const DevSim& s, const AdjView& w, const AdjNext* next, hipStream_t st);
 // the set-index map the tiled kernels read (AdjView::dc8), from dcmap; only where adj_fuses_next
 hipError_t launch_adj_set_index(const int32_t* dcmap, uint8_t* dc8, int64_t n, hipStream_t st);
 hipError_t launch_adj_pressure(const DevSim& s, const AdjView& w, hipStream_t st);

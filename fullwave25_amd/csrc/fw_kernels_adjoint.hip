@@ -24,8 +24,8 @@
 // collects every active cell whose stencil reads x, with that cell's coefficients. In 2D, steps
 // 3 and 4 run as one tiled kernel (the gather yields nu of its own cell, which step 4 needs
 // alone) and step 5 as another, which also runs steps 1 and 2 of the next (earlier) step for its
-// cells when that step's tape is held (they need lambda_p of the cell alone); elsewhere each step
-// is its own per-cell kernel.
+// cells when that step's tape is held (they need lambda_p of the cell alone); in 3D the same on bricks
+// (fw_kernels_adjoint3d.hip); elsewhere each step is its own per-cell kernel.
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -163,23 +163,6 @@ __global__ __launch_bounds__(256) void k_adj_pressure(DevSim s, AdjView w) {
     pre_load(s, w, c, o);
     pre_decode(s, c, o);
     pre_store<ND, EXPO, CODED, false>(s, w, c, o.lp, o);
-}
-
-// lambda_p[c] of the next step after its sparse part (as k_adj_sparse), from lp = lambda_p[c]
-// after this step's gathers and kd = the cell's kind
-__device__ inline float next_mu(const AdjNext& nx, int64_t c, unsigned kd, float lp) {
-    if (!kd) return lp;
-    if ((kd & 1u) || ((kd & 2u) && nx.injecting)) return 0.f;
-    if (!(kd & 4u) || !nx.grow) return lp;
-    int64_t lo = 0, hi = nx.nvox - 1;  // c is one of the sorted voxels
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (nx.vox[mid] < c) lo = mid + 1;
-        else hi = mid;
-    }
-    float acc = 0.f;
-    for (int32_t q = nx.first[lo]; q < nx.first[lo + 1]; ++q) acc += nx.grow[nx.order[q]];
-    return lp + acc;
 }
 
 // lambda_v_a += (D-_a)^T H_a at active cells
@@ -563,7 +546,7 @@ bool adj_percell_gathers() {
     return e && !strncmp(e, "percell", 7);
 }
 
-bool adj_fuses_next(const DevSim& s) { return adj_tiles(s) && !adj_percell_gathers(); }
+bool adj_fuses_next(const DevSim& s, const AdjView& w) { return w.sets || (adj_tiles(s) && !adj_percell_gathers()); }
 
 hipError_t launch_adj_set_index(const int32_t* dcmap, uint8_t* dc8, int64_t n, hipStream_t st) {
     if (n <= 0) return hipSuccess;
@@ -601,6 +584,7 @@ void launch_rest_nd(const DevSim& s, const AdjView& w, dim3 g, dim3 b, hipStream
 }
 
 hipError_t launch_adj_pressure(const DevSim& s, const AdjView& w, hipStream_t st) {
+    if (w.sets) return launch_adj_start_bricks(s, w, st);
     const dim3 g = adj_grid(s), b(64, 4);
     if (s.ndim == 2) launch_pressure_nd<2>(s, w, g, b, st);
     else launch_pressure_nd<3>(s, w, g, b, st);
@@ -608,7 +592,8 @@ hipError_t launch_adj_pressure(const DevSim& s, const AdjView& w, hipStream_t st
 }
 
 hipError_t launch_adj_rest(const DevSim& s, const AdjView& w, const AdjNext* next, hipStream_t st) {
-    if (adj_fuses_next(s)) {
+    if (w.sets) return launch_adj_rest_bricks(s, w, next, st);
+    if (adj_fuses_next(s, w)) {
         const AdjNext none{};
         if (s.aexp) launch_gather_tile2d<true, true, false, false>(s, w, none, st);
         else if (adj_coded(s)) launch_gather_tile2d<true, false, true, false>(s, w, none, st);

@@ -21,95 +21,11 @@
 // Needs weights that all axes share, and rows with coefficients and weights (DevSim::rwide_v) or the
 // exponential model. A wavefront whose cells share a code (exponential: a weight set) reads its row
 // (weights) with scalar loads; the arithmetic order is the other families'.
-#include "fw_quad.h"
+#include "fw_brick.h"
 
 namespace fw {
 
 namespace {
-
-constexpr int BX = kBrickX, BY = kBrickY, BZ = kBrickZ;
-static_assert(BX == 4 && BY == 8 && BZ == 32, "wavefront = x plane, lane = (row, quad)");
-
-// Where a workgroup's brick and a lane's quad are.
-struct Brick {
-    int i0, j0, k0;      // first cell
-    int wave, row, quad; // the wavefront's x plane, the lane's row and quad within the brick
-    uint32_t c;          // element of the quad
-    int n;               // its updated cells (0: none)
-};
-// Workgroup to brick. With `runs` each XCD takes a contiguous run of bricks, so that neighbours' arms share
-// an L2 (131 x 117 x 109: 53.5 -> 49.0 us a step; 200 x 180 x 160: 160.5 -> 148.2); on large grids eight
-// runs at once read more than the memory-side cache holds (600 x 500 x 200: 1782 -> 1939; 400 x 400 x 360:
-// velocity 838 -> 898, pressure 878 -> 857). The caller times both.
-__device__ __forceinline__ uint32_t brick_number(bool runs) { return runs ? xcd_order(blockIdx.x, gridDim.x) : blockIdx.x; }
-__device__ inline Brick brick_of(const DevSim& s, uint32_t tile, uint32_t ny, uint32_t nz) {
-    Brick b;
-    const uint32_t t = tile / nz, bz = tile - t * nz, bx = t / ny, by = t - bx * ny;
-    b.i0 = kHalo + (int)bx * BX;
-    b.j0 = kHalo + (int)by * BY;
-    b.k0 = (int)bz * BZ;
-    b.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    b.row = (threadIdx.x >> 3) & 7;
-    b.quad = threadIdx.x & 7;
-    const int i = b.i0 + b.wave, j = b.j0 + b.row, k = b.k0 + 4 * b.quad;
-    b.c = (uint32_t)i * (uint32_t)s.sx + (uint32_t)(j * (int)s.sy + k);
-    const int left = (int)s.nz - kHalo - k;
-    b.n = i < (int)s.nx - kHalo && j < (int)s.ny - kHalo && k >= kHalo && left > 0 ? min(left, 4) : 0;
-    return b;
-}
-// plane i0 + dx of a field, and a quad's element within a plane; both clamped into the grid
-__device__ inline const float* plane(const DevSim& s, const Brick& b, const float* f, int dx) {
-    return f + (uint32_t)min(max(b.i0 + dx, 0), (int)s.nx - 1) * (uint64_t)s.sx;
-}
-__device__ inline uint32_t in_plane(const DevSim& s, const Brick& b, int dy, int z) {
-    const int j = min(max(b.j0 + dy, 0), (int)s.ny - 1);
-    return (uint32_t)(j * (int)s.sy + min(max(b.k0 + z, 0), (int)s.sy - 4));
-}
-
-// LDS. X arms: planes from XLO (a multiple of 4 loads), [plane][row][32 columns], so that load l of
-// thread t goes to quad 256 l + t. Row sets: the rows -8 .. 15 of the BX updated planes, then SIDE rows
-// from -1 of the planes -1 and BX, with 4 columns on each side; the z arms' outer quads apart.
-constexpr int kArm = BX + 15, kArmLoads = (kArm + 3) / 4, kArmSize = kArm * BY * BZ;
-constexpr int R = BZ + 8;  // a row of a row set
-template <int LO, int HI, int SIDE>
-struct Rows {
-    static constexpr int N = HI - LO;
-    static constexpr int size = (BX * N + 2 * SIDE) * R;
-    __device__ static int at(int dx) {  // row 0, column 0 of a plane
-        const int row = dx < 0 ? BX * N + 1 : dx < BX ? dx * N - LO : BX * N + SIDE + 1;
-        return row * R + 4;
-    }
-};
-constexpr int kEnds = 8;  // columns -8 .. -5 and BZ + 4 .. BZ + 7 of a row
-__device__ __forceinline__ F4 lds4(const float* p) { return *reinterpret_cast<const F4*>(p); }
-__device__ __forceinline__ void put4(float* p, const F4& v) { *reinterpret_cast<F4*>(p) = v; }
-
-// columns -8 .. 11 from the quad at q (`centre`), whose row's ends are `ends`
-__device__ __forceinline__ void z_arm(const float* q, const float* ends, int quad, const F4& centre, float (&z)[20]) {
-    const F4 x[5] = {lds4(quad > 0 ? q - 8 : ends), lds4(q - 4), centre, lds4(q + 4), lds4(quad < BZ / 4 - 1 ? q + 8 : ends + 4)};
-#pragma unroll
-    for (int i = 0; i < 20; ++i) z[i] = x[i / 4][i % 4];
-}
-// elements beside a quad: [e + 1] with `right` after the last, [e - 1] with `left` before the first
-__device__ __forceinline__ float after(const F4& q, float right, int e) { return e < 3 ? q[e + 1] : right; }
-__device__ __forceinline__ float before(const F4& q, float left, int e) { return e > 0 ? q[e - 1] : left; }
-
-// Store a quad of which the first n cells (1 to 4) are updated.
-template <bool NT>
-__device__ __forceinline__ F4 load_memory(const float* f, uint32_t c) {
-    return NT ? ld4nt(f, c) : ld4(f, c);
-}
-template <bool NT>
-__device__ inline void store_quad(float* f, uint32_t c, const F4& v, int n) {
-    if (n == 4) {
-        if (NT) st4nt(f, c, v);
-        else st4(f, c, v);
-        return;
-    }
-#pragma unroll
-    for (int e = 0; e < 3; ++e)
-        if (e < n) gst32(f, c + e, v[e]);
-}
 
 // Coefficients and weights of a quad's cells. Of a wavefront whose cells share a code (SHARED; scalar
 // registers), of one whose cells share a weight set, of cells that share neither.
@@ -384,96 +300,6 @@ __global__ __launch_bounds__(256) void k_velocity_brick(DevSim batch, uint32_t n
 
 // ---- pressure ---------------------------------------------------------------------------------
 
-// v_x: its x arm, the rows -1 and BY of the planes -1 .. BX - 1, and the columns beside the rows between
-using PyRows = Rows<-8, BY + 8, BY + 1>;  // v_y
-using PzRows = Rows<-1, BY + 1, BY + 1>;  // v_z
-constexpr int kPxLoads = kArmLoads + 1;
-struct PreLds {
-    __attribute__((aligned(16))) float X[kArmSize], F[(BX + 1) * 2 * BZ], Y[PyRows::size], Z[PzRows::size], E[BX * BY * kEnds],
-        G[(BX + 1) * BY * 2];
-};
-
-// the quads of v_x beside its x arm (160), of v_y beside the planes and arms (88), of v_z (24, and 128 ends)
-struct PreSide {
-    int dx, dy, z;
-    bool used;
-};
-__device__ inline PreSide px_side(int t) {
-    if (t < 80) return PreSide{(t >> 4) - 1, t & 8 ? BY : -1, 4 * (t & 7), true};
-    const int q = min(t - 80, 79);
-    return PreSide{(q >> 4) - 1, (q >> 1) & 7, q & 1 ? BZ : -4, t < 160};
-}
-__device__ inline PreSide py_side(int t) {
-    if (t < 16) return PreSide{t & 8 ? BX : -1, -1, 4 * (t & 7), true};
-    const int q = min(t - 16, 71), row = q >> 1;  // the rows -1 .. 7 of the updated planes
-    return PreSide{row / 9, row % 9 - 1, q & 1 ? BZ : -4, t < 88};
-}
-__device__ inline PreSide pz_beside(const Brick& b, int t) {  // rows -1 and BY (wavefront 2), before the rows (3)
-    if (b.wave == 2) return PreSide{b.row >> 1, b.row & 1 ? BY : -1, 4 * b.quad, true};
-    const int q = min(t & 63, 23);
-    return PreSide{q < 8 ? -1 : q < 16 ? BX : (q - 16) >> 1, q < 16 ? q & 7 : q & 1 ? BY : -1, -4, (t & 63) < 24};
-}
-__device__ inline PreSide pz_end(int t) {  // beside the rows of the updated planes
-    const int q = min(t, 127), h = q & 3;
-    return PreSide{q >> 5, (q >> 2) & 7, h < 2 ? 4 * h - 8 : BZ + 4 * h - 8, t < 128};
-}
-__device__ __forceinline__ uint32_t side_element(const DevSim& s, const Brick& b, const PreSide& w) {
-    return (uint32_t)(plane(s, b, s.p, w.dx) - s.p) + in_plane(s, b, w.dy, w.z);
-}
-
-// the quads a lane stages
-struct PreStage {
-    F4 x[kPxLoads], y0, y1, y2, y3, z0, z1, z2;
-};
-__device__ __forceinline__ void pre_load(const DevSim& s, const Brick& b, PreStage& q) {
-    const int t = threadIdx.x;
-    const uint32_t mid = in_plane(s, b, b.row, 4 * b.quad);
-    const uint32_t arm = in_plane(s, b, (b.wave & 1 ? BY : -8) + b.row, 4 * b.quad);
-    // (plane 19 of the x arm isn't used)
-#pragma unroll
-    for (int l = 0; l < kArmLoads; ++l) q.x[l] = ld4(plane(s, b, s.v[0], min(b.wave + 4 * l, kArm - 1) - 8), mid);
-    q.x[kArmLoads] = ld4(s.v[0], side_element(s, b, px_side(t)));
-    q.y0 = ld4(plane(s, b, s.v[1], b.wave), mid);
-    q.y1 = ld4(plane(s, b, s.v[1], b.wave >> 1), arm);
-    q.y2 = ld4(plane(s, b, s.v[1], 2 + (b.wave >> 1)), arm);
-    // wavefronts 0 and 1: the planes -1 and BX of v_y and v_z, and v_z's ends; 2 and 3 what lies beside
-    const uint32_t other = (uint32_t)(plane(s, b, s.p, b.wave & 1 ? BX : -1) - s.p) + mid;
-    const uint32_t beside = side_element(s, b, pz_beside(b, t));
-    q.y3 = ld4(s.v[1], b.wave < 2 ? other : side_element(s, b, py_side(max(t - 128, 0))));
-    q.z0 = ld4(plane(s, b, s.v[2], b.wave), mid);
-    q.z1 = ld4(s.v[2], b.wave < 2 ? other : beside);
-    q.z2 = ld4(s.v[2], side_element(s, b, pz_end(t)));
-}
-__device__ __forceinline__ void pre_put(const Brick& b, const PreStage& q, PreLds& m) {
-    const int t = threadIdx.x, at = b.row * R + 4 * b.quad;
-    const F4 side = q.x[kArmLoads], y3 = q.y3, z1 = q.z1, z2 = q.z2;
-#pragma unroll
-    for (int l = 0; l < kArmLoads; ++l)
-        if (l < kArmLoads - 1 || b.wave + 4 * l < kArm) put4(m.X + 4 * (256 * l + t), q.x[l]);
-    {
-        const PreSide w = px_side(t);
-        const float lo = side.x, hi = side.w;
-        if (t < 80) put4(m.F + 4 * t, side);
-        else if (w.used) m.G[t - 80] = w.z < 0 ? hi : lo;
-    }
-    put4(m.Y + PyRows::at(b.wave) + at, q.y0);
-    put4(m.Y + PyRows::at(b.wave >> 1) + (b.wave & 1 ? BY : -8) * R + at, q.y1);
-    put4(m.Y + PyRows::at(2 + (b.wave >> 1)) + (b.wave & 1 ? BY : -8) * R + at, q.y2);
-    put4(m.Z + PzRows::at(b.wave) + at, q.z0);
-    if (b.wave < 2) {
-        put4(m.Y + PyRows::at(b.wave ? BX : -1) + at, y3);
-        put4(m.Z + PzRows::at(b.wave ? BX : -1) + at, z1);
-        const PreSide w = pz_end(t);
-        const bool end = w.z < -4 || w.z > BZ;
-        put4(end ? m.E + ((w.dx * BY + w.dy) * 2 + (w.z > 0)) * 4 : m.Z + PzRows::at(w.dx) + w.dy * R + w.z, z2);
-    } else {
-        const PreSide w = py_side(t - 128);
-        if (w.used) put4(m.Y + PyRows::at(w.dx) + w.dy * R + w.z, y3);
-        const PreSide v = pz_beside(b, t);
-        if (v.used) put4(m.Z + PzRows::at(v.dx) + v.dy * R + v.z, z1);
-    }
-}
-
 struct PreIn {
     F4 phi[3][2], decay;
 };
@@ -498,75 +324,22 @@ __device__ __forceinline__ void pre_axis(const DevSim& s, const Brick& b, int a,
 }
 
 template <bool EXPO, bool TAPE, bool NT, class Coefs>
-__device__ __forceinline__ void pre_update(const DevSim& s, const Brick& b, const Coefs& k, const PreIn& o, const PreLds& lds) {
-    const int at = b.row * R + 4 * b.quad;
+__device__ __forceinline__ void pre_update(const DevSim& s, const Brick& b, const Coefs& k, const PreIn& o, const Arms<0>& lds) {
     F4 p = ld4(s.p, b.c), div{};
     const F4 K = ld4(s.K, b.c);
     {
-        const float* X = lds.X + 4 * (512 + threadIdx.x);
         F4 D{};
-        const F4 x0 = lds4(X), xm = lds4(X - BY * BZ);
-#pragma unroll
-        for (int m = 1; m <= 8; ++m) {
-            const F4 hi = m == 1 ? x0 : lds4(X + (m - 1) * BY * BZ), lo = m == 1 ? xm : lds4(X - m * BY * BZ);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) D[e] = tap(D[e], k.w(e, m - 1), hi[e], lo[e]);
-        }
-        // rows and columns beside: within the arm, or the fringe
-        const float *F = lds.F + (b.wave + 1) * 2 * BZ + 4 * b.quad, *G = lds.G + ((b.wave + 1) * BY + b.row) * 2;
-        const bool last = b.row == BY - 1, first = b.row == 0, left = b.quad == 0, right = b.quad == BZ / 4 - 1;
-        const F4 u0 = lds4(last ? F + BZ : X + BZ), um = lds4(last ? F - BZ : X - BY * BZ + BZ);
-        const F4 d0 = lds4(first ? F : X - BZ), dm = lds4(first ? F - 2 * BZ : X - BY * BZ - BZ);
-        const float l0 = *(left ? G : X - 1), lm = *(left ? G - 2 * BY : X - BY * BZ - 1);
-        const float r0 = *(right ? G + 1 : X + 4), rm = *(right ? G - 2 * BY + 1 : X - BY * BZ + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float tr = 0.f;
-            tr += (u0[e] - um[e]) + (d0[e] - dm[e]);
-            tr += (after(x0, r0, e) - after(xm, rm, e)) + (before(x0, l0, e) - before(xm, lm, e));
-            D[e] = __builtin_fmaf(k.w(e, 8), tr, D[e]);
-        }
+        derivative<0, 0>(b, lds, k, D);
         pre_axis<EXPO, NT>(s, b, 0, D, k, o, div);
     }
     {
-        const float *Y = lds.Y + PyRows::at(b.wave) + at;
-        const float *Yp = lds.Y + PyRows::at(b.wave + 1) + at, *Ym = lds.Y + PyRows::at(b.wave - 1) + at;
         F4 D{};
-        const F4 y0 = lds4(Y), ym = lds4(Y - R);
-#pragma unroll
-        for (int m = 1; m <= 8; ++m) {
-            const F4 hi = m == 1 ? y0 : lds4(Y + (m - 1) * R), lo = m == 1 ? ym : lds4(Y - m * R);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) D[e] = tap(D[e], k.w(e, m - 1), hi[e], lo[e]);
-        }
-        const F4 u0 = lds4(Yp), um = lds4(Yp - R), d0 = lds4(Ym), dm = lds4(Ym - R);
-        const float l0 = Y[-1], r0 = Y[4], lm = Y[-R - 1], rm = Y[-R + 4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float tr = 0.f;
-            tr += (u0[e] - um[e]) + (d0[e] - dm[e]);
-            tr += (after(y0, r0, e) - after(ym, rm, e)) + (before(y0, l0, e) - before(ym, lm, e));
-            D[e] = __builtin_fmaf(k.w(e, 8), tr, D[e]);
-        }
+        derivative<1, 0>(b, lds, k, D);
         pre_axis<EXPO, NT>(s, b, 1, D, k, o, div);
     }
     {
-        const float *Z = lds.Z + PzRows::at(b.wave) + at;
-        const float *Zp = lds.Z + PzRows::at(b.wave + 1) + at, *Zm = lds.Z + PzRows::at(b.wave - 1) + at;
-        float z[20];
-        z_arm(Z, lds.E + (b.wave * BY + b.row) * kEnds, b.quad, lds4(Z), z);
-        const F4 xp = lds4(Zp), xm = lds4(Zm), yp = lds4(Z + R), ym = lds4(Z - R);
-        const float xp_l = Zp[-1], xm_l = Zm[-1], yp_l = Z[R - 1], ym_l = Z[-R - 1];
         F4 D{};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-#pragma unroll
-            for (int m = 1; m <= 8; ++m) D[e] = tap(D[e], k.w(e, m - 1), z[8 + e + m - 1], z[8 + e - m]);
-            float tr = 0.f;
-            tr += (xp[e] - before(xp, xp_l, e)) + (xm[e] - before(xm, xm_l, e));
-            tr += (yp[e] - before(yp, yp_l, e)) + (ym[e] - before(ym, ym_l, e));
-            D[e] = __builtin_fmaf(k.w(e, 8), tr, D[e]);
-        }
+        derivative<2, 0>(b, lds, k, D);
         pre_axis<EXPO, NT>(s, b, 2, D, k, o, div);
     }
 #pragma unroll
@@ -582,7 +355,7 @@ __device__ __forceinline__ void pre_update(const DevSim& s, const Brick& b, cons
 // its brick, for shot blockIdx.y
 template <bool EXPO, bool TAPE, bool NT>
 __global__ __launch_bounds__(256) void k_pressure_brick(DevSim batch, uint32_t nby, uint32_t nbz, bool runs, GroupStep gs) {
-    __shared__ PreLds lds;
+    __shared__ Arms<0> lds;
     TileWork w{};
     if (gs.g) {
         const GroupBoundary& e = gs.g[blockIdx.y];
@@ -592,8 +365,8 @@ __global__ __launch_bounds__(256) void k_pressure_brick(DevSim batch, uint32_t n
     const Brick b = brick_of(s, brick_number(runs), nby, nbz);
     BrickCoef<false, EXPO> kc;
     if (b.n > 0) kc.head(s, b);
-    PreStage q;
-    pre_load(s, b, q);
+    ArmQuads q;
+    load_arms<0>(s, b, [&](int a, uint64_t c0, uint32_t c) { return ld4(s.v[a] + c0, c); }, q);
     PreIn o;
     if (b.n > 0) {
 #pragma unroll
@@ -605,7 +378,7 @@ __global__ __launch_bounds__(256) void k_pressure_brick(DevSim batch, uint32_t n
         if (EXPO) o.decay = ld4(s.aexp, b.c);
         kc.rows(s, b);
     }
-    pre_put(b, q, lds);
+    put_arms<0>(b, q, lds);
     __syncthreads();
     if (b.n > 0) kc.with(s, [&](const auto& k) { pre_update<EXPO, TAPE, NT>(s, b, k, o, lds); });
     if (!gs.g) return;

@@ -133,6 +133,43 @@ def test_3d_bricks_equal_the_per_cell_kernels(monkeypatch, shape, kind, model):
         np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("model", ["isotropic", "exponential"])
+@pytest.mark.parametrize("kind", ["one", "patches", "cells"])
+@pytest.mark.parametrize("shape", [(19, 21, 22), (20, 24, 40), (21, 25, 41), (30, 33, 109)])
+def test_3d_reverse_bricks_meet_the_per_cell_gathers(monkeypatch, shape, kind, model):
+    """The reverse step on bricks: gradients as the per-cell kernels' (the same terms summed in another
+    order: sums of 60 terms with unit roundoff 6e-8, 3.6e-6 a gather, over 9 steps of two gathers: 6.5e-5
+    of the largest value), the same bit for bit for any checkpoint spacing (the fused start of a step and
+    the start on its own), with records on source and release points and brick edges."""
+    from fullwave25_amd.adjoint import HipAdjoint
+
+    rng = np.random.default_rng(12)
+    nt = 9
+    pts = np.stack([rng.integers(8, n - 8, 60) for n in shape], 1)
+    pts[:12, -1] = np.minimum(rng.choice([8, 31, 32, 33], 12), shape[-1] - 9)
+    src, air = pts[:16], pts[16:24]
+    out = np.concatenate([pts[24:], src[:6], air[:4], pts[30:36]])
+    c = {"one": 1540.0, "patches": np.where(np.arange(shape[0])[:, None, None] < shape[0] // 2, 1500.0, 1560.0) * np.ones(shape),
+         "cells": rng.choice([1500.0, 1523.0, 1580.0], size=shape)}[kind]
+    more = {"a_exp": 0.98 + 0.02 * rng.random(shape)} if model == "exponential" else {}
+    inp = raw_inputs(shape, c=c, rho=950 + 100 * rng.random(shape), nt=nt, icc=src, outc=out, icczero=air,
+                     icmat=rng.standard_normal((len(src), nt - 3)).astype(np.float32), **more)
+    weights = rng.standard_normal((inp.n_records, inp.ncoordsout)).astype(np.float32)
+    got = {}
+    for mode, every in (("percell", nt), ("bricks", nt), ("bricks", 4), ("bricks", 1)):
+        monkeypatch.setenv("FULLWAVE_HIP_ADJ_GATHERS", mode)
+        print(f"{shape} {kind} {model}: {mode} every {every}", flush=True)
+        with HipAdjoint(inp, checkpoint_every=every) as adj:
+            adj.forward()
+            got[mode, every] = adj.backward(weights)
+    for k in range(2):
+        ref, new = got["percell", nt][k], got["bricks", nt][k]
+        assert np.abs(ref).max() > 0
+        assert np.abs(new - ref).max() <= 6.5e-5 * np.abs(ref).max()
+        for every in (4, 1):
+            np.testing.assert_array_equal(got["bricks", every][k], new)
+
+
 @pytest.mark.parametrize("model", ["isotropic", "per_axis", "exponential"])
 @pytest.mark.parametrize("shape", [(17, 17), (21, 65), (40, 200), (17, 18, 19), (19, 21, 67)])
 def test_per_cell_boundary_work_matches_boundary_launch(monkeypatch, shape, model):

@@ -37,7 +37,7 @@ struct fw_adj {
     int8_t* vmask = nullptr;  // per distinct voxel: 1 pressure release, 2 source point, 0 neither
     uint8_t* kind = nullptr;  // per device cell (2D, bricks): bit 0 pressure release, 1 source point, 2 sensor voxel
     uint8_t* dc8 = nullptr;   // per device cell: coefficient-set index (grids of the tiled and brick reverse kernels)
-    uint32_t* sets = nullptr; // the set of each brick's arms (3D bricks)
+    uint32_t* sets = nullptr; // the set of each tile's (2D) or brick's (3D) arms
     int64_t nvox = 0;
     bool forward_done = false;
 };
@@ -222,7 +222,8 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
     if (!kind.empty())
         ok = ok && hipMemcpyAsync(a->kind, kind.data(), kind.size(), hipMemcpyHostToDevice, f->stream) == hipSuccess;
     if (ok && fw::adj_tiles(f->ds)) {
-        if (!dalloc((void**)&a->dc8, (size_t)n)) return cleanup(fw::set_error(FW_ERR_NOMEM, "adjoint set-index map"));
+        if (!dalloc((void**)&a->dc8, (size_t)n) || !dalloc((void**)&a->sets, fw::adj_tile_count(f->ds) * 4))
+            return cleanup(fw::set_error(FW_ERR_NOMEM, "adjoint set-index map"));
     }
     if (bricks) {
         const fw::BrickGrid g3 = fw::brick_grid(f->ds);
@@ -281,6 +282,7 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
     // the set indices, of the map as it is now
     const bool bricks = a->sets && fw::adj_bricks_supported(f->ds);
     if (a->dc8) ADJ_HIP(fw::launch_adj_set_index(f->ds.dcmap, a->dc8, n, st));
+    if (a->dc8 && nd == 2) ADJ_HIP(fw::launch_adj_tile_sets(f->ds, a->dc8, a->sets, st));
     if (bricks) ADJ_HIP(fw::launch_adj_brick_sets(f->ds, a->dc8, a->sets, st));
     ADJ_HIP(hipStreamSynchronize(st));  // grad_rec is the caller's buffer, read during the call only
     ADJ_HIP(hipMemsetAsync(a->lam, 0, (size_t)f->nstate * 4, st));
@@ -301,6 +303,7 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
     }
     w.gK = a->work + 3 * nd * n;
     w.dc8 = a->dc8;
+    w.tile_sets = nd == 2 ? a->sets : nullptr;
     w.sets = bricks ? a->sets : nullptr;
     float* grho = a->work + (3 * nd + 1) * n;
     fw::AdjSparse sp{};

@@ -251,6 +251,7 @@ struct AdjView {
     const float* tu[kMaxDim];
     const float* tdiv;
     const uint8_t* dc8;  // coefficient-set index per device cell (the tiled 2D kernels; ndmap <= 256; bricks)
+    const uint32_t* tile_sets;  // tiled 2D kernels: the set of each tile's arms, or all ones
     const uint32_t* sets;  // bricks: the set of each brick's arms, or all ones (null: no bricks)
     float* H[kMaxDim];
     float* G[kMaxDim];
@@ -526,6 +527,9 @@ hipError_t launch_adj_start_bricks(const DevSim& s, const AdjView& w, hipStream_
 hipError_t launch_adj_rest_bricks(const DevSim& s, const AdjView& w, const AdjNext* next, hipStream_t st);
 // the set-index map the tiled kernels read (AdjView::dc8), from dcmap; only where adj_fuses_next
 hipError_t launch_adj_set_index(const int32_t* dcmap, uint8_t* dc8, int64_t n, hipStream_t st);
+// the tiles of a 2D grid, and the set of each one's arms (AdjView::tile_sets)
+size_t adj_tile_count(const DevSim& s);
+hipError_t launch_adj_tile_sets(const DevSim& s, const uint8_t* dc8, uint32_t* sets, hipStream_t st);
 hipError_t launch_adj_pressure(const DevSim& s, const AdjView& w, hipStream_t st);
 hipError_t launch_adj_rest(const DevSim& s, const AdjView& w, const AdjNext* next, hipStream_t st);
 // the forward kernels that write a tape (DevSim::tape_div set): the per-cell kernels, and the

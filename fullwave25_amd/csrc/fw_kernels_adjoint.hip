@@ -308,76 +308,87 @@ __global__ __launch_bounds__(256) void k_adj_dplus_t(DevSim s, AdjView w) {
     w.lp[x] += acc;
 }
 
-// The transposed gathers of a 2D step on tiles, with the gathered field (H or G), the
-// coefficient-set index of every cell it comes from and the coefficient table staged in LDS (the
-// per-cell kernels above read each neighbour's index and weights from global memory). A
+// The transposed gathers of a 2D step on tiles, with the gathered field (H or G) staged in LDS. A
 // workgroup of 256 lanes owns a tile of ATX rows (x) by ATY columns (y); lane (r, j) updates
 // rows r, r + 4, ... of column j. Axis x's field is staged over rows [i0 - 8, i0 + ATX + 8) and
 // columns [j0 - 1, j0 + ATY + 1), axis y's over rows [i0 - 1, i0 + ATX + 1) and columns
 // [j0 - 8, j0 + ATY + 8): every offset either gather reads (along its axis -8..+8, across it
-// -1..+1). Cells outside the grid stage 0 (H and G are 0 off the updated cells anyway). Every
-// lane issues all of its staging loads before it stores any of them, so one memory latency
-// covers the staging. The coefficient table takes the handle's sets only (dynamic LDS). The
-// arithmetic and its order are the per-cell kernels', so the results are the same bit for bit.
-constexpr int ATX = 16, ATY = 64, kAdjLanes = 256;
+// -1..+1). Quads outside the grid stage the ghost border's values (H and G are 0 off the updated
+// cells). Every lane issues all of its staging loads before it stores any of them, so one memory
+// latency covers the staging. A gather weighs each neighbour by the neighbour's own coefficient
+// set: where the arms of a tile hold one set (AdjView::tile_sets) its weights are scalar
+// registers; a tile of several sets also stages the cells' set indices and the handle's weights
+// (dynamic LDS), two dependent LDS reads a neighbour. The arithmetic and its order are the
+// per-cell kernels', so the results are the same bit for bit.
+constexpr int ATX = 8, ATY = 64, kAdjLanes = 256;
 constexpr int AXR = ATX + 16, AXC = ATY + 2;  // axis-x staged region
 constexpr int AYR = ATX + 2, AYC = ATY + 16;  // axis-y staged region
-constexpr int NSX = (AXR * AXC + kAdjLanes - 1) / kAdjLanes;  // staged elements per lane
-constexpr int NSY = (AYR * AYC + kAdjLanes - 1) / kAdjLanes;
 constexpr int kAdjLdsSets = 256;  // coefficient sets staged (ndmap beyond: per-cell kernels)
-constexpr uint32_t kXcds = 8;     // XCDs of an MI355X (the tile order is a bijection for any value)
-constexpr int NCT = (kAdjLdsSets * 2 * kNCoef + kAdjLanes - 1) / kAdjLanes;
+constexpr uint32_t kMixedSets = 0xffffffffu;
 
-template <bool UNI>
-__device__ inline void stage_gather(const DevSim& s, const uint8_t* dc8, const float* fx, const float* fy, int64_t i0,
-                                    int64_t j0, float* FX, float* FY, uint8_t* DX, uint8_t* DY, float* CT) {
-    const int nct = (UNI ? 1 : s.ndmap) * 2 * kNCoef;
-    float vx[NSX], vy[NSY], vc[NCT];
-    int32_t dx[NSX], dy[NSY];
+// Stage R x C cells of `f` from row i, column j, with MIXED their set indices too; load first, put after.
+template <int R, int C, bool MIXED>
+struct GatherStage {
+    static constexpr int N = (R * C + kAdjLanes - 1) / kAdjLanes;
+    float v[N];
+    uint8_t d[MIXED ? N : 1];
+    __device__ __forceinline__ void load(const DevSim& s, const float* f, const uint8_t* dc8, int i, int j) {
 #pragma unroll
-    for (int q = 0; q < NSX; ++q) {
-        const int t = threadIdx.x + q * kAdjLanes;
-        const int r = t / AXC, cc = t - r * AXC;
-        const int64_t i = i0 - 8 + r, j = j0 - 1 + cc;
-        const bool in = t < AXR * AXC && i >= 0 && i < s.nx && j >= 0 && j < s.ny;
-        vx[q] = in ? fx[i * s.sx + j] : 0.f;
-        if (!UNI) dx[q] = in ? dc8[i * s.sx + j] : 0;
-    }
-#pragma unroll
-    for (int q = 0; q < NSY; ++q) {
-        const int t = threadIdx.x + q * kAdjLanes;
-        const int r = t / AYC, cc = t - r * AYC;
-        const int64_t i = i0 - 1 + r, j = j0 - 8 + cc;
-        const bool in = t < AYR * AYC && i >= 0 && i < s.nx && j >= 0 && j < s.ny;
-        vy[q] = in ? fy[i * s.sx + j] : 0.f;
-        if (!UNI) dy[q] = in ? dc8[i * s.sx + j] : 0;
-    }
-#pragma unroll
-    for (int q = 0; q < NCT; ++q) {
-        const int t = threadIdx.x + q * kAdjLanes;
-        vc[q] = t < nct ? s.coef[t] : 0.f;
-    }
-#pragma unroll
-    for (int q = 0; q < NSX; ++q) {
-        const int t = threadIdx.x + q * kAdjLanes;
-        if (t < AXR * AXC) {
-            FX[t] = vx[q];
-            if (!UNI) DX[t] = (uint8_t)dx[q];
+        for (int q = 0; q < N; ++q) {
+            const int t = min((int)threadIdx.x + q * kAdjLanes, R * C - 1);
+            const int r = t / C, cc = t - r * C;
+            const uint32_t c = (uint32_t)(min(max(i + r, 0), (int)s.nx - 1) * (int)s.ny + min(max(j + cc, 0), (int)s.ny - 1));
+            v[q] = gld32(f, c);
+            if (MIXED) d[q] = dc8[c];
         }
     }
+    __device__ __forceinline__ void put(float* F, uint8_t* D) const {
 #pragma unroll
-    for (int q = 0; q < NSY; ++q) {
-        const int t = threadIdx.x + q * kAdjLanes;
-        if (t < AYR * AYC) {
-            FY[t] = vy[q];
-            if (!UNI) DY[t] = (uint8_t)dy[q];
+        for (int q = 0; q < N; ++q) {
+            const int t = threadIdx.x + q * kAdjLanes;
+            if (t >= R * C) continue;
+            F[t] = v[q];
+            if (MIXED) D[t] = d[q];
         }
     }
-#pragma unroll
-    for (int q = 0; q < NCT; ++q) {
-        const int t = threadIdx.x + q * kAdjLanes;
-        if (t < nct) CT[t] = vc[q];
+};
+template <bool MIXED>
+__device__ __forceinline__ void stage_gather(const DevSim& s, const uint8_t* dc8, const float* fx, const float* fy, int i0, int j0,
+                                             float* FX, float* FY, uint8_t* DX, uint8_t* DY, float* CT) {
+    GatherStage<AXR, AXC, MIXED> x;
+    GatherStage<AYR, AYC, MIXED> y;
+    x.load(s, fx, dc8, i0 - 8, j0 - 1);
+    y.load(s, fy, dc8, i0 - 1, j0 - 8);
+    if (MIXED)
+        for (int t = threadIdx.x; t < s.ndmap * 2 * kNCoef; t += kAdjLanes) CT[t] = s.coef[t];
+    x.put(FX, DX);
+    y.put(FY, DY);
+}
+
+// The set of the updated cells in each tile's arms, or kMixedSets.
+__global__ __launch_bounds__(kAdjLanes) void k_adj_tile_sets(DevSim s, const uint8_t* dc8, uint32_t* sets) {
+    __shared__ uint32_t least, most;
+    const int i0 = kHalo + (int)blockIdx.y * ATX, j0 = kHalo + (int)blockIdx.x * ATY;
+    if (threadIdx.x == 0) {
+        least = 255;
+        most = 0;
     }
+    __syncthreads();
+    uint32_t lo = 255, hi = 0;
+    for (int a = 0; a < 2; ++a) {
+        const int ei = a ? 1 : 8, ej = a ? 8 : 1, cols = ATY + 2 * ej, n = (ATX + 2 * ei) * cols;
+        for (int t = threadIdx.x; t < n; t += kAdjLanes) {
+            const int i = i0 - ei + t / cols, j = j0 - ej + t % cols;
+            if (i < kHalo || i >= (int)s.nx - kHalo || j < kHalo || j >= (int)s.ny - kHalo) continue;
+            const uint32_t set = dc8[(uint32_t)(i * (int)s.ny + j)];
+            lo = min(lo, set);
+            hi = max(hi, set);
+        }
+    }
+    atomicMin(&least, lo);
+    atomicMax(&most, hi);
+    __syncthreads();
+    if (threadIdx.x == 0) sets[blockIdx.x + blockIdx.y * gridDim.x] = least == most ? least : kMixedSets;
 }
 
 // DMINUS: lambda_v_a += (D-_a)^T H_a, then the velocity transposed of the cell (EXPO, CODED as
@@ -385,6 +396,13 @@ __device__ inline void stage_gather(const DevSim& s, const uint8_t* dc8, const f
 // part and pressure transposed of the cell (EXPO, CODED as k_adj_pressure; w.tdiv is then the
 // next step's tape). Each lane loads the operands of its first row before the staging and those
 // of row m + 1 before the gathers of row m, so their memory latency overlaps other work.
+//
+// What bounds it: the latencies of a workgroup's load, gather and store phases (small grids have few
+// workgroups a CU), the memory traffic on large ones. us a reverse step with 6 sound speeds, tiles of 16
+// rows that always looked weights up -> these with 16 rows -> with 8 rows: 240 x 256 22.6 -> 20.0 -> 14.5;
+// 640 x 640 30.9 -> 27.4 -> 26.0; 1184 x 1184 71.4 -> 70.7 -> 65.9; 1700 x 1700 152.6 -> 150.4 -> 147.7.
+// One sound speed, 640 x 640: 24.1 -> 23.0 -> 21.3; exponential model 27.6 -> 25.1 -> 23.9. Measured and left
+// out: both rows' operands and table rows before the staging (640 x 640: 28.3).
 template <bool UNI, bool DMINUS, bool EXPO, bool CODED, bool NEXT>
 __global__ __launch_bounds__(kAdjLanes) void k_adj_gather_tile2d(DevSim s, AdjView w, AdjNext nx) {
     __shared__ float FX[AXR * AXC];
@@ -393,13 +411,10 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_gather_tile2d(DevSim s, AdjVi
     __shared__ uint8_t DY[UNI ? 1 : AYR * AYC];
     extern __shared__ float CT[];  // [set][axis][9], the handle's sets
     constexpr int NR = ATX / 4;    // rows per lane: rl, rl + 4, ...
-    // Workgroup b runs on XCD b % 8 (round-robin dispatch). XCD k takes the tiles
-    // [k q + min(k, r), ...) in row-major order, so that neighbouring tiles, which stage the same
-    // halo cells, share an L2: the fetch from memory drops by 40 % (the halos are 3.5 staged
-    // values a cell) and the kernels run 17 % faster than with the tiles in launch order.
-    const uint32_t nb = gridDim.x * gridDim.y, b = blockIdx.x + blockIdx.y * gridDim.x;
-    const uint32_t xcd = b % kXcds, k = b / kXcds, q = nb / kXcds, r = nb % kXcds;
-    const uint32_t tile = xcd * q + (xcd < r ? xcd : r) + k;
+    // Each XCD takes a contiguous run of tiles, so that neighbouring tiles, which stage the same halo
+    // cells, share an L2: the fetch from memory drops by 40 % and the kernels run 17 % faster than with
+    // the tiles in launch order.
+    const uint32_t tile = xcd_order(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
     const uint32_t bx = tile % gridDim.x, by = tile / gridDim.x;
     const int64_t i0 = kHalo + (int64_t)by * ATX, j0 = kHalo + (int64_t)bx * ATY;
     const int jl = threadIdx.x % ATY, rl = threadIdx.x / ATY;
@@ -421,75 +436,92 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_gather_tile2d(DevSim s, AdjVi
         }
     };
     if (nrows > 0) load(0, ops[0]);
-    stage_gather<UNI>(s, w.dc8, DMINUS ? w.H[0] : w.G[0], DMINUS ? w.H[1] : w.G[1], i0, j0, FX, FY, DX, DY, CT);
+    const uint32_t set = UNI ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(w.tile_sets[tile]);
+    const float *fx = DMINUS ? w.H[0] : w.G[0], *fy = DMINUS ? w.H[1] : w.G[1];
+    if (UNI || set != kMixedSets) stage_gather<false>(s, w.dc8, fx, fy, (int)i0, (int)j0, FX, FY, DX, DY, CT);
+    else stage_gather<true>(s, w.dc8, fx, fy, (int)i0, (int)j0, FX, FY, DX, DY, CT);
     __syncthreads();
     // staged element at (di, dj) from cell (il, jl) of the tile, for axis x's and axis y's field
     auto ex = [&](int il, int di, int dj) { return (il + 8 + di) * AXC + (jl + 1 + dj); };
     auto ey = [&](int il, int di, int dj) { return (il + 1 + di) * AYC + (jl + 8 + dj); };
-    auto wx = [&](int e, int k) { return CT[(UNI ? 0 : (int)DX[e] * 2) * kNCoef + k]; };             // axis 0 set
-    auto wy = [&](int e, int k) { return CT[(UNI ? kNCoef : ((int)DY[e] * 2 + 1) * kNCoef) + k]; };  // axis 1 set
+    // wx, wy: weight k of the staged element e, of axis x's and axis y's field
+    auto rows = [&](const auto& wx, const auto& wy) {
 #pragma unroll
-    for (int m = 0; m < NR; ++m) {
-        if (m >= nrows) break;
-        Ops& o = ops[m & 1];
-        const int il = rl + 4 * m;
-        const int64_t x = (i0 + il) * s.sx + j;
-        if constexpr (DMINUS) vel_decode(s, x, o);
-        else if constexpr (NEXT) pre_decode(s, x, o);
-        if (m + 1 < nrows) load(m + 1, ops[(m + 1) & 1]);
-        if constexpr (DMINUS) {
-            // axis x: c1 = x - (m-1) e_x, c2 = x + m e_x; transverse c1 = x -+ e_y, c2 = x + e_x -+ e_y
-            float acc = 0.f;
+        for (int m = 0; m < NR; ++m) {
+            if (m >= nrows) break;
+            Ops& o = ops[m & 1];
+            const int il = rl + 4 * m;
+            const int64_t x = (i0 + il) * s.sx + j;
+            if constexpr (DMINUS) vel_decode(s, x, o);
+            else if constexpr (NEXT) pre_decode(s, x, o);
+            if (m + 1 < nrows) load(m + 1, ops[(m + 1) & 1]);
+            if constexpr (DMINUS) {
+                // axis x: c1 = x - (m-1) e_x, c2 = x + m e_x; transverse c1 = x -+ e_y, c2 = x + e_x -+ e_y
+                float acc = 0.f;
 #pragma unroll
-            for (int q = 1; q <= 8; ++q) {
-                const int e1 = ex(il, -(q - 1), 0), e2 = ex(il, q, 0);
-                acc += wx(e1, q - 1) * FX[e1] - wx(e2, q - 1) * FX[e2];
+                for (int q = 1; q <= 8; ++q) {
+                    const int e1 = ex(il, -(q - 1), 0), e2 = ex(il, q, 0);
+                    acc += wx(e1, q - 1) * FX[e1] - wx(e2, q - 1) * FX[e2];
+                }
+#pragma unroll
+                for (int sg = -1; sg <= 1; sg += 2) {
+                    const int e1 = ex(il, 0, -sg), e2 = ex(il, 1, -sg);
+                    acc += wx(e1, 8) * FX[e1] - wx(e2, 8) * FX[e2];
+                }
+                o.nu[0] = o.nu[0] + acc;
+                acc = 0.f;
+#pragma unroll
+                for (int q = 1; q <= 8; ++q) {
+                    const int e1 = ey(il, 0, -(q - 1)), e2 = ey(il, 0, q);
+                    acc += wy(e1, q - 1) * FY[e1] - wy(e2, q - 1) * FY[e2];
+                }
+#pragma unroll
+                for (int sg = -1; sg <= 1; sg += 2) {
+                    const int e1 = ey(il, -sg, 0), e2 = ey(il, -sg, 1);
+                    acc += wy(e1, 8) * FY[e1] - wy(e2, 8) * FY[e2];
+                }
+                o.nu[1] = o.nu[1] + acc;
+                vel_store<2, EXPO, CODED, true>(s, w, x, o);
+            } else {
+                // axis x: c1 = x - m e_x, c2 = x + (m-1) e_x; transverse c1 = x - e_x -+ e_y, c2 = x -+ e_y
+                float acc = 0.f;
+#pragma unroll
+                for (int q = 1; q <= 8; ++q) {
+                    const int e1 = ex(il, -q, 0), e2 = ex(il, q - 1, 0);
+                    acc += wx(e1, q - 1) * FX[e1] - wx(e2, q - 1) * FX[e2];
+                }
+#pragma unroll
+                for (int sg = -1; sg <= 1; sg += 2) {
+                    const int e1 = ex(il, -1, -sg), e2 = ex(il, 0, -sg);
+                    acc += wx(e1, 8) * FX[e1] - wx(e2, 8) * FX[e2];
+                }
+#pragma unroll
+                for (int q = 1; q <= 8; ++q) {
+                    const int e1 = ey(il, 0, -q), e2 = ey(il, 0, q - 1);
+                    acc += wy(e1, q - 1) * FY[e1] - wy(e2, q - 1) * FY[e2];
+                }
+#pragma unroll
+                for (int sg = -1; sg <= 1; sg += 2) {
+                    const int e1 = ey(il, -sg, -1), e2 = ey(il, -sg, 0);
+                    acc += wy(e1, 8) * FY[e1] - wy(e2, 8) * FY[e2];
+                }
+                if constexpr (NEXT) pre_store<2, EXPO, CODED, true>(s, w, x, next_mu(nx, x, o.kind, o.lp + acc), o);
+                else w.lp[x] = o.lp + acc;
             }
-#pragma unroll
-            for (int sg = -1; sg <= 1; sg += 2) {
-                const int e1 = ex(il, 0, -sg), e2 = ex(il, 1, -sg);
-                acc += wx(e1, 8) * FX[e1] - wx(e2, 8) * FX[e2];
-            }
-            o.nu[0] = o.nu[0] + acc;
-            acc = 0.f;
-#pragma unroll
-            for (int q = 1; q <= 8; ++q) {
-                const int e1 = ey(il, 0, -(q - 1)), e2 = ey(il, 0, q);
-                acc += wy(e1, q - 1) * FY[e1] - wy(e2, q - 1) * FY[e2];
-            }
-#pragma unroll
-            for (int sg = -1; sg <= 1; sg += 2) {
-                const int e1 = ey(il, -sg, 0), e2 = ey(il, -sg, 1);
-                acc += wy(e1, 8) * FY[e1] - wy(e2, 8) * FY[e2];
-            }
-            o.nu[1] = o.nu[1] + acc;
-            vel_store<2, EXPO, CODED, true>(s, w, x, o);
-        } else {
-            // axis x: c1 = x - m e_x, c2 = x + (m-1) e_x; transverse c1 = x - e_x -+ e_y, c2 = x -+ e_y
-            float acc = 0.f;
-#pragma unroll
-            for (int q = 1; q <= 8; ++q) {
-                const int e1 = ex(il, -q, 0), e2 = ex(il, q - 1, 0);
-                acc += wx(e1, q - 1) * FX[e1] - wx(e2, q - 1) * FX[e2];
-            }
-#pragma unroll
-            for (int sg = -1; sg <= 1; sg += 2) {
-                const int e1 = ex(il, -1, -sg), e2 = ex(il, 0, -sg);
-                acc += wx(e1, 8) * FX[e1] - wx(e2, 8) * FX[e2];
-            }
-#pragma unroll
-            for (int q = 1; q <= 8; ++q) {
-                const int e1 = ey(il, 0, -q), e2 = ey(il, 0, q - 1);
-                acc += wy(e1, q - 1) * FY[e1] - wy(e2, q - 1) * FY[e2];
-            }
-#pragma unroll
-            for (int sg = -1; sg <= 1; sg += 2) {
-                const int e1 = ey(il, -sg, -1), e2 = ey(il, -sg, 0);
-                acc += wy(e1, 8) * FY[e1] - wy(e2, 8) * FY[e2];
-            }
-            if constexpr (NEXT) pre_store<2, EXPO, CODED, true>(s, w, x, next_mu(nx, x, o.kind, o.lp + acc), o);
-            else w.lp[x] = o.lp + acc;
         }
+    };
+    if (UNI || set != kMixedSets) {
+        float kx[kNCoef], ky[kNCoef];
+        const scalar_ptr c = as_scalar(s.coef) + set * 2 * kNCoef;
+#pragma unroll
+        for (int k = 0; k < kNCoef; ++k) {
+            kx[k] = c[k];
+            ky[k] = c[kNCoef + k];
+        }
+        rows([&](int, int k) { return kx[k]; }, [&](int, int k) { return ky[k]; });
+    } else {
+        rows([&](int e, int k) { return CT[(int)DX[e] * 2 * kNCoef + k]; },
+             [&](int e, int k) { return CT[((int)DY[e] * 2 + 1) * kNCoef + k]; });
     }
 }
 
@@ -538,7 +570,7 @@ hipError_t launch_adj_sparse(float* lp, const float* grow, const AdjSparse& sp, 
 
 // the transposed gathers on LDS tiles: 2D grids of at most kAdjLdsSets coefficient sets (the
 // staged set indices are 16-bit)
-bool adj_tiles(const DevSim& s) { return s.ndim == 2 && s.ndmap <= kAdjLdsSets; }
+bool adj_tiles(const DevSim& s) { return s.ndim == 2 && s.ndmap <= kAdjLdsSets && s.nx * s.ny < ((int64_t)1 << 30) && s.nx < ATX * (int64_t)65535; }
 
 // FULLWAVE_HIP_ADJ_GATHERS=percell keeps the per-cell kernels (to compare the two forms)
 bool adj_percell_gathers() {
@@ -554,15 +586,29 @@ hipError_t launch_adj_set_index(const int32_t* dcmap, uint8_t* dc8, int64_t n, h
     return hipGetLastError();
 }
 
+static dim3 adj_tile_grid(const DevSim& s) {
+    return dim3((unsigned)((s.ny - 2 * kHalo + ATY - 1) / ATY), (unsigned)((s.nx - 2 * kHalo + ATX - 1) / ATX));
+}
+
+size_t adj_tile_count(const DevSim& s) {
+    const dim3 g = adj_tile_grid(s);
+    return (size_t)g.x * g.y;
+}
+
+hipError_t launch_adj_tile_sets(const DevSim& s, const uint8_t* dc8, uint32_t* sets, hipStream_t st) {
+    hipLaunchKernelGGL(k_adj_tile_sets, adj_tile_grid(s), dim3(kAdjLanes), 0, st, s, dc8, sets);
+    return hipGetLastError();
+}
+
 template <bool DMINUS, bool EXPO, bool CODED, bool NEXT>
 void launch_gather_tile2d(const DevSim& s, const AdjView& w, const AdjNext& nx, hipStream_t st) {
-    const dim3 g((unsigned)((s.ny - 2 * kHalo + ATY - 1) / ATY), (unsigned)((s.nx - 2 * kHalo + ATX - 1) / ATX));
-    const bool uni = s.ndmap == 1;
-    const size_t lds = (size_t)(uni ? 1 : s.ndmap) * 2 * kNCoef * sizeof(float);
-    if (uni)
-        hipLaunchKernelGGL((k_adj_gather_tile2d<true, DMINUS, EXPO, CODED, NEXT>), g, dim3(kAdjLanes), lds, st, s, w, nx);
-    else
-        hipLaunchKernelGGL((k_adj_gather_tile2d<false, DMINUS, EXPO, CODED, NEXT>), g, dim3(kAdjLanes), lds, st, s, w, nx);
+    const dim3 g = adj_tile_grid(s);
+    if (s.ndmap == 1) {
+        hipLaunchKernelGGL((k_adj_gather_tile2d<true, DMINUS, EXPO, CODED, NEXT>), g, dim3(kAdjLanes), 0, st, s, w, nx);
+        return;
+    }
+    const size_t lds = (size_t)s.ndmap * 2 * kNCoef * sizeof(float);
+    hipLaunchKernelGGL((k_adj_gather_tile2d<false, DMINUS, EXPO, CODED, NEXT>), g, dim3(kAdjLanes), lds, st, s, w, nx);
 }
 
 static bool adj_coded(const DevSim& s) { return !s.aexp && s.isotropic && s.rcode; }

@@ -171,6 +171,42 @@ def test_3d_reverse_bricks_meet_the_per_cell_gathers(monkeypatch, shape, kind, m
 
 
 @pytest.mark.parametrize("model", ["isotropic", "per_axis", "exponential"])
+@pytest.mark.parametrize("kind", ["one", "patches", "cells"])
+@pytest.mark.parametrize("shape", [(21, 26), (24, 80), (25, 81), (40, 150), (67, 211)])
+def test_2d_reverse_tiles_equal_the_per_cell_gathers(monkeypatch, shape, kind, model):
+    """The reverse step on tiles of 8 x 64 cells, at the edges of tiles (part of one, whole tiles, one more),
+    with tiles of one coefficient set, of several, and of both kinds side by side (patches), equal to the
+    per-cell kernels bit for bit, for any checkpoint spacing."""
+    from fullwave25_amd.adjoint import HipAdjoint
+
+    rng = np.random.default_rng(14)
+    nt = 9
+    pts = np.stack([rng.integers(8, n - 8, 60) for n in shape], 1)
+    pts[:12, -1] = np.minimum(rng.choice([8, 71, 72, 73], 12), shape[-1] - 9)
+    src, air = pts[:16], pts[16:24]
+    out = np.concatenate([pts[24:], src[:6], air[:4], pts[30:36]])
+    c = {"one": 1540.0, "patches": np.where(np.arange(shape[0])[:, None] < shape[0] // 2, 1500.0, 1560.0) * np.ones(shape),
+         "cells": rng.choice([1500.0, 1523.0, 1580.0], size=shape)}[kind]
+    more = {"a_exp": 0.98 + 0.02 * rng.random(shape)} if model == "exponential" else {"isotropic": model == "isotropic"}
+    inp = raw_inputs(shape, c=c, rho=950 + 100 * rng.random(shape), nt=nt, icc=src, outc=out, icczero=air,
+                     icmat=rng.standard_normal((len(src), nt - 3)).astype(np.float32), **more)
+    if kind == "patches":
+        inp = dataclasses.replace(inp, dy=inp.dx * 1.25)
+    weights = rng.standard_normal((inp.n_records, inp.ncoordsout)).astype(np.float32)
+    got = []
+    for mode, every in (("percell", nt), ("tiles", nt), ("tiles", 4)):
+        monkeypatch.setenv("FULLWAVE_HIP_ADJ_GATHERS", mode)
+        print(f"{shape} {kind} {model}: {mode} every {every}", flush=True)
+        with HipAdjoint(inp, checkpoint_every=every) as adj:
+            adj.forward()
+            got.append(adj.backward(weights))
+    assert np.abs(got[0][0]).max() > 0
+    for new in got[1:]:
+        for g, ref in zip(new, got[0]):
+            np.testing.assert_array_equal(g, ref)
+
+
+@pytest.mark.parametrize("model", ["isotropic", "per_axis", "exponential"])
 @pytest.mark.parametrize("shape", [(17, 17), (21, 65), (40, 200), (17, 18, 19), (19, 21, 67)])
 def test_per_cell_boundary_work_matches_boundary_launch(monkeypatch, shape, model):
     """The per-cell pressure kernels do the step's sources, pressure release and sensors for the points

@@ -569,7 +569,7 @@ hipError_t launch_adj_sparse(float* lp, const float* grow, const AdjSparse& sp, 
 }
 
 // the transposed gathers on LDS tiles: 2D grids of at most kAdjLdsSets coefficient sets (the
-// staged set indices are 16-bit)
+// staged set indices are bytes)
 bool adj_tiles(const DevSim& s) { return s.ndim == 2 && s.ndmap <= kAdjLdsSets && s.nx * s.ny < ((int64_t)1 << 30) && s.nx < ATX * (int64_t)65535; }
 
 // FULLWAVE_HIP_ADJ_GATHERS=percell keeps the per-cell kernels (to compare the two forms)

@@ -401,7 +401,8 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_tile_sets(DevSim s, const uin
 // workgroups a CU), the memory traffic on large ones. us a reverse step with 6 sound speeds, tiles of 16
 // rows that always looked weights up -> these with 16 rows -> with 8 rows: 240 x 256 22.6 -> 20.0 -> 14.5;
 // 640 x 640 30.9 -> 27.4 -> 26.0; 1184 x 1184 71.4 -> 70.7 -> 65.9; 1700 x 1700 152.6 -> 150.4 -> 147.7.
-// One sound speed, 640 x 640: 24.1 -> 23.0 -> 21.3; exponential model 27.6 -> 25.1 -> 23.9. Measured and left
+// One sound speed, 640 x 640: 24.1 -> 23.0 -> 21.3; exponential model 27.6 -> 25.1 -> 23.9. 130 sound speeds on
+// 1152 x 1152 (every tile looks its weights up): 55.6 -> 55.5 us of kernels. Measured and left
 // out: both rows' operands and table rows before the staging (640 x 640: 28.3).
 template <bool UNI, bool DMINUS, bool EXPO, bool CODED, bool NEXT>
 __global__ __launch_bounds__(kAdjLanes) void k_adj_gather_tile2d(DevSim s, AdjView w, AdjNext nx) {

@@ -618,6 +618,16 @@ void drop(fw_sim* s, const char* name) {
     s->dev.erase(it);
 }
 
+// The captured steps hold the addresses of the handle's tables (codes, points): forget them before one is
+// freed; the next run captures again.
+int drop_graph(fw_sim* s) {
+    if (!s->graph) return FW_OK;
+    FW_HIP(hipStreamSynchronize(s->stream));
+    (void)hipGraphExecDestroy(s->graph);
+    s->graph = nullptr;
+    return FW_OK;
+}
+
 void drop_codes(fw_sim* s) {
     for (const char* name : {"_rcode", "_rtab_v", "_rtab_p", "_rwide_v", "_rwide_p"}) drop(s, name);
     s->ds.rcode = nullptr;
@@ -806,14 +816,11 @@ int encode_relaxation(fw_sim* s) {
     return rc;
 }
 
-// New codes for a handle that has run: a captured graph holds the old table addresses.
+// New codes for a handle that has run.
 int recode(fw_sim* s) {
     FW_HIP(hipStreamSynchronize(s->stream));
-    if (s->graph) {
-        (void)hipGraphExecDestroy(s->graph);
-        s->graph = nullptr;
-    }
-    const int rc = match_axes(s);
+    int rc = drop_graph(s);
+    if (rc == FW_OK) rc = match_axes(s);
     return rc != FW_OK ? rc : encode_relaxation(s);
 }
 
@@ -842,7 +849,10 @@ std::vector<fw::GroupBoundary> fused_entries(const fw_sim* s, const fw::GroupBou
 constexpr size_t kMaxFusedPoints = size_t(1) << 18;
 
 int setup_fused_boundary(fw_sim* s, const fw::BoundaryLists& bl) {
+    int rc = drop_graph(s);
+    if (rc != FW_OK) return rc;
     s->fused_boundary = false;
+    s->fbound = nullptr;
     drop(s, "_fpoints");
     drop(s, "_fbound");
     if (s->fixed_base || !fw::pressure_fuses_boundary(s->ds, s->cfg_p)) return FW_OK;
@@ -865,7 +875,6 @@ int setup_fused_boundary(fw_sim* s, const fw::BoundaryLists& bl) {
         pt = fw::point_table(s->ds.nx, s->ds.ny, gx, tile_w, rows, bl, &pts);
     }
     void* p;
-    int rc;
     if ((rc = alloc(s, "_fpoints", pts.size() * 4, &p)) != FW_OK) return rc;
     FW_HIP(copy_sync(s, p, pts.data(), pts.size() * 4, hipMemcpyHostToDevice));
     const int32_t* base = (const int32_t*)p;
@@ -1578,11 +1587,8 @@ int fw_sim_set_graph_steps(fw_sim* s, int64_t steps) {
     if (!s) return fail(FW_ERR_INVALID, "null handle");
     if (steps < 0 || steps > 100000) return fail(FW_ERR_INVALID, "graph steps must be in [0, 100000]");
     DeviceGuard g(s->device);
-    if (s->graph) {
-        FW_HIP(hipStreamSynchronize(s->stream));
-        (void)hipGraphExecDestroy(s->graph);
-        s->graph = nullptr;
-    }
+    const int rc = drop_graph(s);
+    if (rc != FW_OK) return rc;
     s->graph_steps = steps;
     return FW_OK;
 }

@@ -1,0 +1,142 @@
+// What a handle keeps alive, and for how long: the engine's host code on a stand-in runtime
+// (host_runtime.h), under AddressSanitizer. Built and run by tests/test_host_runtime.py, one check a run:
+// host_runtime_check <check>.
+#include <cmath>
+#include <random>
+
+#include "host_runtime.h"
+
+namespace {
+
+using rt::Launch;
+
+// Inputs of a small run: isotropic, per-axis or exponential; every source point is also a sensor, so that
+// the records hold the signals whatever the stencils do.
+struct Inputs {
+    fw_desc d{};
+    std::map<std::string, std::vector<float>> f;
+    std::map<std::string, std::vector<int32_t>> i;
+    int64_t cells() const { return d.nx * d.ny * d.nz; }
+};
+
+Inputs inputs(int ndim, int64_t nx, int64_t ny, int64_t nz, int64_t nt, int isotropic = 1, int model = 0, int sound_speeds = 3) {
+    Inputs in;
+    fw_desc& d = in.d;
+    d.abi_version = FW_ABI_VERSION;
+    d.ndim = ndim;
+    d.isotropic = isotropic;
+    d.attenuation_model = model;
+    d.n_relax = 2;
+    d.nx = nx, d.ny = ny, d.nz = ndim == 3 ? nz : 1;
+    d.nt = nt;
+    d.dx = d.dy = d.dz = 4.3e-5;
+    d.dt = 1.1e-8;
+    d.c0 = 1540;
+    d.modt = 2;
+    d.ndmap = sound_speeds;
+    const int64_t n = in.cells();
+    std::mt19937 rng(5);
+    auto map = [&](const std::string& name, float lo, float step) {  // a few values in patches
+        std::vector<float> v((size_t)n);
+        for (int64_t c = 0; c < n; ++c) v[(size_t)c] = lo + step * (float)(c * 3 / n);
+        in.f[name] = v;
+    };
+    map("K", 2e9f, 1e8f);
+    map("rho", 1000.f, 10.f);
+    const char *av[3] = {"u", "w", "v"}, *ap[3] = {"x", "y", "z"};
+    if (model == 1) map("a_exp", 0.9f, 0.01f);
+    for (int a = 0; a < (isotropic ? 1 : ndim) && model == 0; ++a)
+        for (const char* x : {av[a], ap[a]}) {
+            map(std::string("kappa") + x, 1.f, 0.1f);
+            for (const char* nu : {"1", "2"}) {
+                map(std::string("apml") + x + nu, -0.1f, 0.01f);
+                map(std::string("bpml") + x + nu, 0.8f, 0.01f);
+            }
+        }
+    in.f["dmap"].assign((size_t)(18 * d.ndmap), 0.1f);
+    auto& dc = in.i["dcmap"];
+    for (int64_t c = 0; c < n; ++c) dc.push_back((int32_t)(c * sound_speeds / n));
+    auto& src = in.i["icc"];
+    const int64_t dims[3] = {nx, ny, nz};
+    d.ncoords = 9;
+    for (int64_t q = 0; q < d.ncoords; ++q)
+        for (int a = 0; a < ndim; ++a) src.push_back((int32_t)(a == 0 ? 8 + q % (nx - 16) : 8 + (7 * q) % (dims[a] - 16)));
+    in.i["outc"] = src;
+    d.ncoordsout = d.ncoords;
+    d.ntic = nt;
+    auto& sig = in.f["icmat"];
+    for (int64_t k = 0; k < d.ncoords * d.ntic; ++k) sig.push_back((float)(rng() % 1000) + 1.f);
+    return in;
+}
+
+fw_sim* make(const Inputs& in) {
+    fw_sim* s = nullptr;
+    CHECK(fw_sim_create(&in.d, 0, &s) == FW_OK);
+    for (const auto& m : in.f) CHECK(fw_sim_upload(s, m.first.c_str(), m.second.data(), m.second.size() * 4) == FW_OK);
+    for (const auto& m : in.i) CHECK(fw_sim_upload(s, m.first.c_str(), m.second.data(), m.second.size() * 4) == FW_OK);
+    return s;
+}
+
+void pin(fw_sim* s, int variant, int width, int chunk) {
+    for (int kind = 0; kind < 2; ++kind) CHECK(fw_sim_set_kernel_config(s, kind, variant, width, chunk) == FW_OK);
+}
+
+// run `steps` from rest; the records are the signals
+void run_and_check(fw_sim* s, const Inputs& in, int64_t steps) {
+    CHECK(fw_sim_reset(s) == FW_OK);
+    const int rc = fw_sim_run(s, steps);
+    CHECK(rc == FW_OK);
+    if (rc != FW_OK) {
+        std::fprintf(stderr, "run: %s\n", fw_last_error());
+        return;
+    }
+    const int64_t rows = (steps + in.d.modt - 1) / in.d.modt;
+    std::vector<float> rec((size_t)(rows * in.d.ncoordsout));
+    CHECK(fw_sim_download_sensors(s, rec.data(), rec.size() * 4) == FW_OK);
+    for (int64_t r = 0; r < rows; ++r)
+        for (int64_t q = 0; q < in.d.ncoordsout; ++q)
+            CHECK(rec[(size_t)(r * in.d.ncoordsout + q)] == in.f.at("icmat")[(size_t)(q * in.d.ntic + r * in.d.modt)]);
+}
+
+// An adjoint made on a handle that has run from a captured graph: the graph's launches hold the address of
+// the point table that the adjoint's kernels replace.
+void graph_then_adjoint() {
+    struct Pin {
+        int ndim, variant, width, chunk;
+    };
+    for (const Pin& p : {Pin{2, 1, 64, 5}, Pin{2, 2, 256, 32}, Pin{2, 0, 0, 0}, Pin{3, 0, 0, 0}, Pin{3, 5, 32, 1}}) {
+        const Inputs in = inputs(p.ndim, 40, 36, 44, 24);
+        fw_sim* s = make(in);
+        pin(s, p.variant, p.width, p.chunk);
+        CHECK(fw_sim_set_graph_steps(s, 4) == FW_OK);
+        run_and_check(s, in, 10);
+        fw_adj* a = nullptr;
+        CHECK(fw_adj_create(s, 8, &a) == FW_OK);
+        run_and_check(s, in, 10);
+        run_and_check(s, in, 24);
+        CHECK(fw_adj_destroy(a) == FW_OK && fw_sim_destroy(s) == FW_OK);
+    }
+}
+
+struct Check {
+    const char* name;
+    void (*run)();
+};
+const Check checks[] = {
+    {"graph_then_adjoint", graph_then_adjoint},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const size_t before = rt::live.size();
+    for (const Check& c : checks)
+        if (argc > 1 && !strcmp(argv[1], c.name)) {
+            c.run();
+            CHECK(rt::live.size() == before && rt::streams.empty() && rt::graphs.empty());  // all given back
+            std::printf("%s: %s (%d failures)\n", c.name, rt::failures ? "FAILED" : "ok", rt::failures);
+            return rt::failures ? 1 : 0;
+        }
+    std::fprintf(stderr, "no such check\n");
+    return 2;
+}

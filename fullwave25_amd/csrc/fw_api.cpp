@@ -380,6 +380,7 @@ int check_coords(const fw_desc& d, int64_t sx, int64_t sy, const std::vector<int
 int time_config(fw_sim* s, const fw::LaunchCfg& cfg, bool velocity, float best, float* ms) {
     fw::DevBoundary none = s->db;
     none.ntic = 0;
+    if (!s->rec_cap) none.nout = 0;  // no steps, no records to write
     const bool apart = !velocity && !fw::pressure_fuses_boundary(s->ds, cfg);
     auto launch = [&] {
         if (velocity) return fw::launch_velocity(s->ds, cfg, s->stream);

@@ -118,12 +118,26 @@ void graph_then_adjoint() {
     }
 }
 
+// A handle of no steps has no records: choosing its kernels writes none.
+void no_records() {
+    for (int ndim : {2, 3}) {
+        Inputs in = inputs(ndim, 40, 36, 44, 6);
+        in.d.nt = 0;
+        fw_sim* s = make(in);
+        int32_t v, w, c;
+        CHECK(fw_sim_kernel_config(s, 1, &v, &w, &c) == FW_OK);
+        CHECK(fw_sim_run(s, 0) == FW_OK && fw_sim_run(s, 1) == FW_ERR_INVALID);
+        CHECK(fw_sim_destroy(s) == FW_OK);
+    }
+}
+
 struct Check {
     const char* name;
     void (*run)();
 };
 const Check checks[] = {
     {"graph_then_adjoint", graph_then_adjoint},
+    {"no_records", no_records},
 };
 
 }  // namespace

@@ -57,3 +57,7 @@ def check(driver, name, **env):
 
 def test_adjoint_on_a_handle_with_a_captured_graph(driver):
     check(driver, "graph_then_adjoint")
+
+
+def test_kernels_of_a_handle_without_steps(driver):
+    check(driver, "no_records")

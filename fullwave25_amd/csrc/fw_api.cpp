@@ -994,6 +994,10 @@ int finalize(fw_sim* s) {
     return FW_OK;
 }
 
+// Whether a step's pressure launch does the boundary work: the points are grouped for it, and the kernel that
+// runs takes them (a taped step's may be another, and so may one whose grid lost its codes).
+bool step_fuses_boundary(const fw_sim* s) { return s->fused_boundary && fw::pressure_fuses_boundary(s->ds, s->cfg_p); }
+
 int launch_step(fw_sim* s, bool timed, double* ms) {
     hipError_t e;
     auto timed_launch = [&](int kind, auto&& fn) -> int {
@@ -1012,8 +1016,7 @@ int launch_step(fw_sim* s, bool timed, double* ms) {
     int rc;
     rc = timed_launch(fw::kVelocity, [&] { return fw::launch_velocity(s->ds, s->cfg_v, s->stream); });
     if (rc != FW_OK) return rc;
-    // the pressure launch does the boundary work where its kernel can (a taped step's may be another)
-    if (s->fused_boundary && fw::pressure_fuses_boundary(s->ds, s->cfg_p)) {
+    if (step_fuses_boundary(s)) {
         const fw::GroupStep gs{s->fbound, nullptr, s->step};
         rc = timed_launch(fw::kPressure, [&] { return fw::launch_pressure(s->ds, s->cfg_p, s->stream, gs); });
         if (rc != FW_OK) return rc;
@@ -1038,7 +1041,7 @@ int capture_graph(fw_sim* s) {
     hipError_t e = hipSuccess;
     for (int64_t it = 0; it < s->graph_steps && e == hipSuccess; ++it) {
         e = fw::launch_velocity(s->ds, s->cfg_v, s->stream);
-        if (e == hipSuccess && s->fused_boundary) {
+        if (e == hipSuccess && step_fuses_boundary(s)) {
             e = fw::launch_pressure(s->ds, s->cfg_p, s->stream, fw::GroupStep{s->fbound, s->step_dev, 0});
         } else {
             if (e == hipSuccess) e = fw::launch_pressure(s->ds, s->cfg_p, s->stream);

@@ -131,6 +131,36 @@ void no_records() {
     }
 }
 
+// Bricks need codes: a brick handle that replays captured steps runs on after its codes are gone (switched
+// off; one axis with a map of its own), and with bricks again when they are back.
+void graph_without_codes() {
+    for (int isotropic : {1, 0}) {
+        const Inputs in = inputs(3, 24, 26, 44, 24, isotropic);
+        fw_sim* s = make(in);
+        pin(s, 5, 32, 1);
+        CHECK(fw_sim_set_graph_steps(s, 4) == FW_OK);
+        run_and_check(s, in, 10);
+        CHECK(fw_sim_set_relaxation_codes(s, 0) == FW_OK);
+        run_and_check(s, in, 10);
+        CHECK(fw_sim_set_relaxation_codes(s, 1) == FW_OK);
+        run_and_check(s, in, 10);
+        const char* last = isotropic ? "bpmlx2" : "bpmlz2";
+        std::vector<float> own = in.f.at(last);
+        for (size_t c = 0; c < own.size(); ++c) own[c] = isotropic ? 1e-6f * (float)c : own[c] * 0.5f;  // too many codes
+        CHECK(fw_sim_upload(s, last, own.data(), own.size() * 4) == FW_OK);
+        run_and_check(s, in, 10);
+        CHECK(fw_sim_upload(s, last, in.f.at(last).data(), own.size() * 4) == FW_OK);
+        rt::log.clear();
+        rt::keep_log = true;
+        run_and_check(s, in, 10);
+        rt::keep_log = false;
+        int bricks = 0;
+        for (const Launch& l : rt::log) bricks += l.is("k_pressure_brick");
+        CHECK(bricks == 10);
+        CHECK(fw_sim_destroy(s) == FW_OK);
+    }
+}
+
 struct Check {
     const char* name;
     void (*run)();
@@ -138,6 +168,7 @@ struct Check {
 const Check checks[] = {
     {"graph_then_adjoint", graph_then_adjoint},
     {"no_records", no_records},
+    {"graph_without_codes", graph_without_codes},
 };
 
 }  // namespace

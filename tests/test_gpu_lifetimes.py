@@ -49,3 +49,41 @@ def test_adjoint_on_a_handle_with_captured_steps(monkeypatch, kernels):
                 np.testing.assert_array_equal(sim.field("p"), want[1])
         finally:
             sim.lib.fw_adj_destroy(adj)
+
+
+@pytest.mark.parametrize("graph_steps", [0, 4])
+@pytest.mark.parametrize("isotropic", [True, False])
+def test_bricks_whose_codes_go_and_come_back(monkeypatch, isotropic, graph_steps):
+    """Brick kernels need relaxation codes: codes switched off and on, one axis map that differs and the
+    old one again, between runs of one handle."""
+    monkeypatch.delenv("FULLWAVE_HIP_KERNELS", raising=False)
+    relax = {"v": {"kappa": 1.05, "d": (9e3, 4e5), "alpha": (3e6, 9e7)}, "p": {"kappa": 1.02, "d": (3e4, 5e5), "alpha": (1.5e7, 1.1e8)}}
+    inp = inputs((24, 26, 44), isotropic=isotropic, relax=relax)
+    want = fresh(inp)
+    name = "bpmlx2" if isotropic else "bpmlz2"
+    own = inp.maps[name] * np.linspace(0.2, 1.0, inp.maps[name].size, dtype=np.float32).reshape(inp.shape)
+    changed = inputs((24, 26, 44), isotropic=isotropic, relax=relax)
+    changed.maps[name] = own
+    other = fresh(changed)
+    assert (other[1] != want[1]).any()
+    brick = {"variant": "brick", "width": 32, "chunk": 1}
+    with engine.HipSimulation(inp) as sim:
+        sim.set_kernel_config({"velocity": brick, "pressure": brick})
+        sim.set_graph_steps(graph_steps)
+
+        def again(ref):
+            for _ in range(2):
+                sim.reset()
+                sim.run(inp.nt)
+                np.testing.assert_array_equal(sim.sensors(), ref[0])
+                np.testing.assert_array_equal(sim.field("p"), ref[1])
+
+        again(want)
+        sim.set_relaxation_codes(False)
+        again(want)
+        sim.set_relaxation_codes(True)
+        again(want)
+        sim.upload(name, own)
+        again(other)
+        sim.upload(name, inp.maps[name])
+        again(want)

@@ -61,3 +61,7 @@ def test_adjoint_on_a_handle_with_a_captured_graph(driver):
 
 def test_kernels_of_a_handle_without_steps(driver):
     check(driver, "no_records")
+
+
+def test_captured_steps_of_bricks_that_lose_their_codes(driver):
+    check(driver, "graph_without_codes")

@@ -132,9 +132,9 @@ void tape_kernels(fw_sim* f) {
     }
     if (!fw::tape_capable(f->ds, t)) t.variant = 0;
     for (int kind = 0; kind < 2; ++kind) {
-        fw::LaunchCfg& c = kind == 0 ? f->cfg_v : f->cfg_p;
-        if (f->pinned[kind] && fw::tape_capable(f->ds, c)) continue;
-        c = t;
+        fw::LaunchCfg& c = f->chosen[kind];
+        if (!(f->pinned[kind] && fw::tape_capable(f->ds, c))) c = t;
+        f->spare[kind] = fw::LaunchCfg{};  // the per-cell kernels
     }
 }
 
@@ -151,7 +151,7 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
     int rc = fw::prepare_untuned(f);  // tape_kernels sets the kernels
     if (rc != FW_OK) return rc;
     tape_kernels(f);
-    if ((rc = fw::refit_boundary(f)) != FW_OK) return rc;
+    if ((rc = fw::fit_kernels(f)) != FW_OK) return rc;
     size_t free_b = 0, total_b = 0;
     if (checkpoint_every == 0) ADJ_HIP(hipMemGetInfo(&free_b, &total_b));
     fw_adj* a = new fw_adj();

@@ -38,7 +38,10 @@ struct fw_sim {
     int64_t step = 0;
     int64_t rec_cap = 0;
     fw::LaunchCfg cfg_v, cfg_p;  // velocity and pressure kernels, chosen independently
-    // per-cell, 2D marching or tiled pressure kernels: the step's sources, pressure release and sensors
+    // what was chosen for each kind, and what runs in its place while the grid has no codes for chosen
+    // bricks (fit_kernels)
+    fw::LaunchCfg chosen[2], spare[2];
+    // per-cell, brick, 2D marching or tiled pressure kernels: the step's sources, pressure release and sensors
     // run inside the pressure launch (one entry per shot, points grouped by the kernel's tiles)
     bool fused_boundary = false;
     fw::GroupBoundary* fbound = nullptr;
@@ -78,7 +81,8 @@ int prepare_untuned(fw_sim* s);            // the same without timing kernels, f
 // device memory of the handle, ordered on its stream
 hipError_t device_alloc(fw_sim* s, void** p, size_t bytes);
 void device_free(fw_sim* s, void* p);
-int refit_boundary(fw_sim* s);             // the point table again, after a change of the pressure kernel
+// the handle's kernels and its point table from fw_sim::chosen and spare, after a change of these or of the codes
+int fit_kernels(fw_sim* s);
 int forward_step(fw_sim* s);               // one time step on the handle's stream
 hipError_t grid_to_host(const fw_sim* s, void* dst, const void* src, size_t esize);  // padded -> compact
 // Host-side set-up of a handle, without device access.

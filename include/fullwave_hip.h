@@ -159,7 +159,9 @@ int fw_sim_set_field(fw_sim* sim, const char* name, const float* values, size_t 
  * the FULLWAVE_HIP_KERNELS environment variable: "percell", "stream[:width[:chunk]]",
  * "tile[:rows]", "pipe[:width[:chunk]]", "pipelite[:width[:chunk]]" or "brick[:32[:order]]", or
  * "<velocity>/<pressure>" to set each on its own).
- * Calling this before the first run makes that choice. */
+ * Calling this before the first run makes that choice. While the grid of a handle that chose brick kernels has
+ * no codes (fw_sim_set_relaxation_codes), it runs the fastest of the other families (stream:512:8 where they
+ * were not timed), and reports it. */
 int fw_sim_kernel_config(fw_sim* sim, int32_t kind, int32_t* variant, int32_t* width, int32_t* chunk);
 /* Fix the kernel family and shape of `kind` (values as fw_sim_kernel_config reports them)
  * before the first run, instead of timing the candidates; it overrides FULLWAVE_HIP_KERNELS.

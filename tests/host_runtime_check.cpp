@@ -161,6 +161,53 @@ void graph_without_codes() {
     }
 }
 
+std::string config(fw_sim* s, int kind) {
+    int32_t v = -1, w = 0, c = 0;
+    CHECK(fw_sim_kernel_config(s, kind, &v, &w, &c) == FW_OK);
+    return std::to_string(v) + ":" + std::to_string(w) + ":" + std::to_string(c);
+}
+
+// The kernels of a brick handle whose codes go away: the fastest of the others where they were timed, the
+// stated default where they were not, the per-cell ones (which write the tape) for an adjoint; the bricks
+// again with the codes.
+void kernels_without_codes() {
+    rt::cost = [](const Launch& l) {
+        if (l.is("k_velocity_brick") || l.is("k_pressure_brick")) return 10.0;
+        if (l.is("k_velocity_pipe3d")) return 20.0 + std::abs(l.arg<int>(1) - 48) + (l.name.find("<16, ") != std::string::npos ? 3 : 0);
+        if (l.is("k_pressure_pipe3d")) return 20.0 + std::abs(l.arg<int>(1) - 16) + (l.name.find("<16, ") != std::string::npos ? 0 : 3);
+        return l.is("k_boundary") ? 1.0 : 100.0;
+    };
+    const Inputs in = inputs(3, 24, 26, 44, 24);
+    const std::vector<float> zero((size_t)in.cells(), 0.f);
+    for (int how = 0; how < 3; ++how) {  // timed, a field set before the first run, bound to an adjoint
+        fw_sim* s = make(in);
+        if (how == 1) CHECK(fw_sim_set_field(s, "p", zero.data(), zero.size() * 4) == FW_OK);
+        fw_adj* a = nullptr;
+        if (how == 2) CHECK(fw_adj_create(s, 8, &a) == FW_OK);
+        for (int round = 0; round < 2; ++round) {
+            run_and_check(s, in, 10);
+            for (int kind = 0; kind < 2; ++kind) CHECK(config(s, kind).compare(0, 5, "5:32:") == 0);
+            CHECK(fw_sim_set_relaxation_codes(s, 0) == FW_OK);
+            rt::log.clear();
+            rt::keep_log = true;
+            run_and_check(s, in, 10);
+            rt::keep_log = false;
+            int march = 0, cell = 0;
+            for (const Launch& l : rt::log) {
+                march += l.is("k_velocity_pipe3d") || l.is("k_pressure_pipe3d") || l.is("k_velocity_3d") || l.is("k_pressure_3d");
+                cell += l.is("k_velocity_cell") || l.is("k_pressure_cell");
+            }
+            CHECK(march == (how == 2 ? 0 : 20) && cell == (how == 2 ? 20 : 0));
+            const std::string v = config(s, 0), p = config(s, 1);
+            if (how == 0) CHECK((v == "3:512:48" || v == "4:512:48") && (p == "3:1024:16" || p == "4:1024:16"));
+            if (how == 1) CHECK(v == "1:512:8" && p == "1:512:8");
+            if (how == 2) CHECK(v[0] == '0' && p[0] == '0');
+            CHECK(fw_sim_set_relaxation_codes(s, 1) == FW_OK);
+        }
+        CHECK(fw_adj_destroy(a) == FW_OK && fw_sim_destroy(s) == FW_OK);
+    }
+}
+
 struct Check {
     const char* name;
     void (*run)();
@@ -169,6 +216,7 @@ const Check checks[] = {
     {"graph_then_adjoint", graph_then_adjoint},
     {"no_records", no_records},
     {"graph_without_codes", graph_without_codes},
+    {"kernels_without_codes", kernels_without_codes},
 };
 
 }  // namespace

@@ -65,3 +65,7 @@ def test_kernels_of_a_handle_without_steps(driver):
 
 def test_captured_steps_of_bricks_that_lose_their_codes(driver):
     check(driver, "graph_without_codes")
+
+
+def test_kernels_of_bricks_that_lose_their_codes(driver):
+    check(driver, "kernels_without_codes")

@@ -391,6 +391,8 @@ unsigned cell_tiles_x(const DevSim& s);
 int64_t cell_tiles(const DevSim& s);
 int64_t cell_first_row(const DevSim& s);
 int64_t cell_row_count(const DevSim& s);
+// load the code of a family (LaunchCfg::variant) on the current device, as its first launch would
+hipError_t load_family(const DevSim& s, int variant);
 bool streaming_supported(const DevSim& s);
 bool tile2d_supported(const DevSim& s);
 int tile2d_width(int rows);  // columns of the tile of `rows` rows (8, 16 or 32)

@@ -414,6 +414,11 @@ bool brick_supported(const DevSim& s) {
     return g.nx * g.ny * g.nz < ((int64_t)1 << 31);
 }
 
+hipError_t load_brick_code() {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_velocity_brick<true, false, false>));
+}
+
 hipError_t launch_brick(const DevSim& s, const LaunchCfg& cfg, bool velocity, const GroupStep& gs, hipStream_t st) {
     const bool runs = cfg.chunk == 1;
     const bool nt = memory_streams(s);

@@ -615,6 +615,11 @@ void launch_pipe(bool velocity, const DevSim& s, int chunk, hipStream_t st) {
 
 // cfg.width is the workgroup size: 512 (tiles of 8 rows in y) or 1024 (16 rows); variant 3
 // loads the per-cell operands one iteration ahead, variant 4 at the top of their iteration
+hipError_t load_pipe3d_code() {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_velocity_pipe3d<8, true, true, true, true, true>));
+}
+
 hipError_t launch_pipe3d(const DevSim& s, const LaunchCfg& cfg, bool velocity, hipStream_t st) {
     const int chunk = cfg.chunk < 1 ? 1 : cfg.chunk;
     const bool ahead = cfg.variant == 3;

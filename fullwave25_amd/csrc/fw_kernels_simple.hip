@@ -471,6 +471,11 @@ hipError_t launch_simple(const DevSim& s, bool velocity, const GroupStep& gs, hi
     return s.ndim == 2 ? launch_cell_nd<2>(s, velocity, gs, st) : launch_cell_nd<3>(s, velocity, gs, st);
 }
 
+hipError_t load_cell_code() {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_reciprocal));
+}
+
 hipError_t launch_boundary(const DevSim& s, const DevBoundary& b, int64_t step, int64_t modt,
                            hipStream_t st) {
     // lanes for what this step does: a step between two records of the whole domain injects a few

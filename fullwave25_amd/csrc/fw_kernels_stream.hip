@@ -469,6 +469,28 @@ bool streaming_supported(const DevSim& s) {
 bool tile2d_supported(const DevSim& s);
 hipError_t launch_tile2d(const DevSim& s, const LaunchCfg& cfg, bool velocity, const GroupStep& gs, hipStream_t st);
 
+hipError_t load_stream2d_code() {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_velocity_2d_group<64>));
+}
+
+hipError_t load_cell_code();
+hipError_t load_brick_code();
+hipError_t load_tile2d_code();
+hipError_t load_pipe3d_code();
+hipError_t load_stream3d_code();
+
+hipError_t load_family(const DevSim& s, int variant) {
+    switch (variant) {
+        case 1: return s.ndim == 3 ? load_stream3d_code() : load_stream2d_code();
+        case 2: return load_tile2d_code();
+        case 3:
+        case 4: return load_pipe3d_code();
+        case 5: return load_brick_code();
+        default: return load_cell_code();
+    }
+}
+
 bool tape_capable(const DevSim& s, const LaunchCfg& cfg) {
     return cfg.variant == 0 || (cfg.variant == 2 && tile2d_supported(s)) || (cfg.variant == 5 && brick_supported(s));
 }

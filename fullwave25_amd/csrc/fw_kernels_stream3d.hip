@@ -288,6 +288,11 @@ void launch_3d(bool velocity, const DevSim& s, int lds, int chunk, hipStream_t s
 }
 
 // cfg.width is the workgroup size: 512 (tiles of 8 rows in y) or 1024 (16 rows)
+hipError_t load_stream3d_code() {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_velocity_3d<8, true, true>));
+}
+
 hipError_t launch_velocity_3d(const DevSim& s, const LaunchCfg& cfg, hipStream_t st) {
     const int chunk = cfg.chunk < 1 ? 1 : cfg.chunk;
     if (cfg.width == 1024) launch_3d<16>(true, s, coef_lds_bytes_3d(s), chunk, st);

@@ -680,6 +680,11 @@ hipError_t launch_group_tile2d(const GroupTile* t, int n, uint32_t blocks, int r
     }
 }
 
+hipError_t load_tile2d_code() {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_velocity_tile_group<Tile8, true>));
+}
+
 hipError_t launch_tile2d(const DevSim& s, const LaunchCfg& cfg, bool velocity, const GroupStep& gs, hipStream_t st) {
     if (s.tape_div) return launch_tile<Tile8, true>(s, velocity, gs, st);  // taped steps: 8-row tiles
     switch (cfg.chunk) {

@@ -208,6 +208,77 @@ void kernels_without_codes() {
     }
 }
 
+// A process whose launches cost what `us` says; the code of each of the engine's source files takes 3 ms
+// to load, at the first use of one of its kernels.
+template <class F>
+void launch_costs(std::set<std::string>* loaded, const F& us) {
+    loaded->clear();
+    rt::load = [loaded](const std::string& n) {
+        const char* files[] = {"brick", "pipe3d", "_tile", "_2d", "_3d", "code"};
+        std::string file = "cell";
+        for (const char* f : files)
+            if (n.find(f) != std::string::npos) {
+                file = f;
+                break;
+            }
+        return loaded->insert(file).second ? 3000.0 : 0.0;
+    };
+    rt::cost = us;
+}
+
+// The kernels that timing keeps are the fastest of the candidates, whatever a first launch costs.
+void timing() {
+    std::set<std::string> loaded;
+    const Inputs in = inputs(3, 24, 26, 44, 4);
+    auto kernels = [&](const Inputs& i) {
+        fw_sim* s = make(i);
+        const std::string c = config(s, 0) + " " + config(s, 1);
+        CHECK(fw_sim_destroy(s) == FW_OK);
+        return c;
+    };
+    // long kernels: the bricks' first order, and the last of the marching families
+    launch_costs(&loaded, [](const Launch& l) {
+        if (l.is("k_velocity_brick")) return l.arg<bool>(3) ? 900.0 : 835.0;
+        if (l.is("k_pressure_brick")) return l.arg<bool>(3) ? 857.0 : 880.0;
+        if (l.is("k_velocity_pipe3d")) return 893.0 + std::abs(l.arg<int>(1) - 48);
+        if (l.is("k_pressure_pipe3d")) return l.name.find("<16, ") != std::string::npos && l.arg<int>(1) == 8 ? 839.0 : 950.0;
+        return l.is("k_boundary") ? 4.0 : 2000.0;
+    });
+    CHECK(kernels(in) == "5:32:0 3:1024:8");
+    CHECK(kernels(in) == "5:32:0 3:1024:8");  // a later handle of the process
+    // short ones
+    launch_costs(&loaded, [](const Launch& l) {
+        if (l.is("k_velocity_brick")) return l.arg<bool>(3) ? 21.0 : 22.0;
+        if (l.is("k_pressure_brick")) return l.arg<bool>(3) ? 23.0 : 22.0;
+        return l.is("k_boundary") ? 4.0 : 25.0;
+    });
+    CHECK(kernels(in) == "5:32:1 5:32:0");
+    // a long kernel whose first timed launch is short by 5 %: the fastest two are launched again
+    std::map<std::string, int> seen;
+    launch_costs(&loaded, [&seen](const Launch& l) {
+        const bool v = l.is("k_velocity_brick"), p = l.is("k_pressure_brick");
+        if (!v && !p) return l.is("k_boundary") ? 4.0 : 3000.0;
+        const bool order = l.arg<bool>(3), slow = order == p;
+        const bool odd = slow && ++seen[l.name] == 1;
+        return slow ? odd ? 965.0 : 1015.0 : 1000.0;
+    });
+    CHECK(kernels(in) == "5:32:1 5:32:0");
+    // points that no pressure launch takes: every family makes a boundary launch, and none is charged for it
+    Inputs many = in;
+    many.i["outc"].clear();
+    many.d.ncoordsout = (int64_t(1) << 18) + 1;
+    for (int64_t q = 0; q < 3 * many.d.ncoordsout; ++q) many.i["outc"].push_back(9);
+    auto marching = [](const Launch& l) {
+        if (l.is("k_velocity_brick") || l.is("k_pressure_brick")) return 103.0;
+        if (l.is("k_velocity_pipe3d") || l.is("k_pressure_pipe3d")) return l.arg<int>(1) == 16 ? 100.0 : 110.0;
+        return l.is("k_boundary") ? 10.0 : 200.0;
+    };
+    launch_costs(&loaded, marching);
+    CHECK(kernels(many) == "3:512:16 3:512:16");
+    launch_costs(&loaded, marching);
+    CHECK(kernels(in) == "3:512:16 5:32:0");  // points that a pressure launch takes
+}
+
 struct Check {
     const char* name;
     void (*run)();
@@ -217,6 +288,7 @@ const Check checks[] = {
     {"no_records", no_records},
     {"graph_without_codes", graph_without_codes},
     {"kernels_without_codes", kernels_without_codes},
+    {"timing", timing},
 };
 
 }  // namespace

@@ -69,3 +69,7 @@ def test_captured_steps_of_bricks_that_lose_their_codes(driver):
 
 def test_kernels_of_bricks_that_lose_their_codes(driver):
     check(driver, "kernels_without_codes")
+
+
+def test_timing_keeps_the_fastest_kernels(driver):
+    check(driver, "timing")

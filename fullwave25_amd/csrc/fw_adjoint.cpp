@@ -248,7 +248,8 @@ int fw_adj_forward(fw_adj* a) {
     fw_sim* f = a->f;
     f->state_zero = false;
     Guard g(f->device);
-    int rc = fw_sim_reset(f);
+    int rc = fw::settle(f);
+    if (rc == FW_OK) rc = fw_sim_reset(f);
     if (rc != FW_OK) return rc;
     a->tape_seg = -1;
     const int64_t last = a->nckpt - 1, s_last = last * a->every;

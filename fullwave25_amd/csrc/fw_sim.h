@@ -62,6 +62,9 @@ struct fw_sim {
     // ncodes = codes in use (0: the marching kernels read the per-cell maps), covering
     // coded_cells of the ncell device cells (the others read the per-cell maps)
     int codes_mode = -1;
+    // per-axis handles: a map was uploaded after the first run. Until settle() compares and codes the maps
+    // again, the handle runs per axis, without codes.
+    bool maps_new = false;
     int32_t ncodes = 0;
     int64_t coded_cells = 0;
     // fixed-region handle (fw_run_dir_noalloc): every device array is carved out of
@@ -76,7 +79,8 @@ struct fw_sim {
 namespace fw {
 // host helpers of fw_api.cpp used by the adjoint
 int set_error(int code, const char* fmt, ...);
-int prepare(fw_sim* s);                    // check inputs, resolve coordinates, pick kernels
+int prepare(fw_sim* s);                    // check inputs, resolve coordinates, pick kernels; settle()
+int settle(fw_sim* s);                     // codes and kernels of the maps as they are now
 int prepare_untuned(fw_sim* s);            // the same without timing kernels, for a caller that sets them
 // device memory of the handle, ordered on its stream
 hipError_t device_alloc(fw_sim* s, void** p, size_t bytes);

@@ -187,7 +187,8 @@ int fw_sim_set_graph_steps(fw_sim* sim, int64_t steps);
  * the cells. fw_sim_set_relaxation_codes(sim, 0) keeps the per-cell maps (as does
  * FULLWAVE_HIP_CODES=0 in the environment); called after the first run it re-codes at once.
  * Uploading a relaxation map or dcmap after the first run re-codes too.
- * Per-axis handles whose axes have the same maps, bit for bit, run as isotropic ones, with codes.
+ * Per-axis handles whose axes have the same maps, bit for bit, run as isotropic ones, with codes (after
+ * uploads to one that has run, from its next run on).
  * fw_sim_relaxation_codes returns the number of codes in use (0: per-cell maps, or a per-axis
  * handle) and, if
  * coded_fraction is not NULL, the fraction of device cells that carry a code (3D device rows

@@ -279,6 +279,53 @@ void timing() {
     CHECK(kernels(in) == "3:512:16 5:32:0");  // points that a pressure launch takes
 }
 
+// A set of per-axis maps uploaded again: the maps are compared and coded once, by the next run, and until then
+// nothing of the old codes is used. One axis with a map of its own is found, also by an adjoint's run.
+void per_axis_uploads() {
+    for (int ndim : {2, 3}) {
+        const Inputs in = inputs(ndim, 24, 28, 44, 24, 0);
+        fw_sim* s = make(in);
+        auto again = [&](const char* own) {
+            for (const auto& m : in.f) {
+                const bool map = m.first.compare(0, 5, "kappa") == 0 || m.first.compare(1, 3, "pml") == 0;
+                if (!map) continue;
+                std::vector<float> v = m.second;
+                for (size_t c = 0; own && m.first == own && c < v.size(); ++c) v[c] *= 0.5f;
+                CHECK(fw_sim_upload(s, m.first.c_str(), v.data(), v.size() * 4) == FW_OK);
+            }
+        };
+        auto count = [&](const char* kernel) {
+            int n = 0;
+            for (const Launch& l : rt::log) n += l.is(kernel) && !l.is("k_maps_differ_tail");
+            return n;
+        };
+        CHECK(fw_sim_set_graph_steps(s, 4) == FW_OK);
+        run_and_check(s, in, 10);
+        fw_adj* a = nullptr;
+        const std::vector<float> w(in.d.ncoordsout * 12, 1.f);
+        std::vector<float> gk((size_t)in.cells()), gr((size_t)in.cells());
+        auto gradient = [&] {
+            CHECK(fw_adj_forward(a) == FW_OK);
+            CHECK(fw_adj_backward(a, w.data(), w.size() * 4, gk.data(), gr.data(), gk.size() * 4) == FW_OK);
+        };
+        for (const char* own : {(const char*)nullptr, ndim == 2 ? "bpmly2" : "bpmlz2", (const char*)nullptr}) {
+            rt::log.clear();
+            rt::keep_log = true;
+            again(own);
+            CHECK(count("k_maps_differ") == 0 && count("k_code_insert") == 0);
+            if (a) gradient();
+            run_and_check(s, in, 10);
+            rt::keep_log = false;
+            CHECK(count("k_maps_differ") == 1 && count("k_code_insert") == (own ? 0 : 1));
+            if (!a) CHECK(fw_adj_create(s, 8, &a) == FW_OK);
+            gradient();
+            again(nullptr);
+            CHECK(fw_adj_backward(a, w.data(), w.size() * 4, gk.data(), gr.data(), gk.size() * 4) == FW_OK);
+        }
+        CHECK(fw_adj_destroy(a) == FW_OK && fw_sim_destroy(s) == FW_OK);
+    }
+}
+
 struct Check {
     const char* name;
     void (*run)();
@@ -289,6 +336,7 @@ const Check checks[] = {
     {"graph_without_codes", graph_without_codes},
     {"kernels_without_codes", kernels_without_codes},
     {"timing", timing},
+    {"per_axis_uploads", per_axis_uploads},
 };
 
 }  // namespace

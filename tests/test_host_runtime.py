@@ -73,3 +73,7 @@ def test_kernels_of_bricks_that_lose_their_codes(driver):
 
 def test_timing_keeps_the_fastest_kernels(driver):
     check(driver, "timing")
+
+
+def test_per_axis_maps_uploaded_again(driver):
+    check(driver, "per_axis_uploads")

@@ -156,6 +156,7 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
     if (checkpoint_every == 0) ADJ_HIP(hipMemGetInfo(&free_b, &total_b));
     fw_adj* a = new fw_adj();
     a->f = f;
+    f->adjoints.insert(a);
     a->every = checkpoint_every ? std::min<int64_t>(checkpoint_every, std::max<int64_t>(f->d.nt, 1))
                                 : auto_segment(f, free_b);
     a->nckpt = (f->d.nt + a->every - 1) / a->every;
@@ -246,6 +247,7 @@ int fw_adj_checkpoint_every(const fw_adj* a, int64_t* every) {
 int fw_adj_forward(fw_adj* a) {
     if (!a) return fw::set_error(FW_ERR_INVALID, "null handle");
     fw_sim* f = a->f;
+    if (!f) return fw::set_error(FW_ERR_STATE, "the adjoint's simulation has been destroyed");
     f->state_zero = false;
     Guard g(f->device);
     int rc = fw::settle(f);
@@ -268,6 +270,7 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
                     size_t grid_bytes) {
     if (!a || !grad_rec || !grad_k || !grad_rho) return fw::set_error(FW_ERR_INVALID, "null argument");
     fw_sim* f = a->f;
+    if (!f) return fw::set_error(FW_ERR_STATE, "the adjoint's simulation has been destroyed");
     f->state_zero = false;
     if (!a->forward_done) return fw::set_error(FW_ERR_STATE, "run fw_adj_forward first");
     const int64_t nrec = f->rec_cap, nout = f->d.ncoordsout, n = f->ncell, nt = f->d.nt;
@@ -368,13 +371,23 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
 
 int fw_adj_destroy(fw_adj* a) {
     if (!a) return FW_OK;
-    Guard g(a->f->device);
-    if (a->f->stream) (void)hipStreamSynchronize(a->f->stream);
-    for (void* p : {(void*)a->ckpt, (void*)a->tape, (void*)a->lam, (void*)a->work, (void*)a->grec, (void*)a->vox,
-                    (void*)a->first, (void*)a->order, (void*)a->vmask, (void*)a->kind, (void*)a->dc8, (void*)a->sets})
-        fw::device_free(a->f, p);
+    if (a->f) fw::unbind(a);
     delete a;
     return FW_OK;
 }
 
 }  // extern "C"
+
+namespace fw {
+
+void unbind(fw_adj* a) {
+    Guard g(a->f->device);
+    if (a->f->stream) (void)hipStreamSynchronize(a->f->stream);
+    for (void* p : {(void*)a->ckpt, (void*)a->tape, (void*)a->lam, (void*)a->work, (void*)a->grec, (void*)a->vox,
+                    (void*)a->first, (void*)a->order, (void*)a->vmask, (void*)a->kind, (void*)a->dc8, (void*)a->sets})
+        device_free(a->f, p);
+    a->f->adjoints.erase(a);
+    a->f = nullptr;
+}
+
+}  // namespace fw

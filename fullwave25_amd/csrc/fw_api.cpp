@@ -1692,6 +1692,7 @@ int fw_sim_destroy(fw_sim* s) {
     if (!s) return FW_OK;
     DeviceGuard g(s->device);
     if (s->stream) (void)hipStreamSynchronize(s->stream);
+    while (!s->adjoints.empty()) fw::unbind(*s->adjoints.begin());
     if (s->graph) (void)hipGraphExecDestroy(s->graph);
     dev_free(s, s->step_dev);
     for (auto& kv : s->dev)

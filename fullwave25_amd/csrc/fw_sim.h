@@ -67,6 +67,8 @@ struct fw_sim {
     bool maps_new = false;
     int32_t ncodes = 0;
     int64_t coded_cells = 0;
+    // adjoints bound to this handle, which gives back their device memory when it is destroyed before them
+    std::set<struct fw_adj*> adjoints;
     // fixed-region handle (fw_run_dir_noalloc): every device array is carved out of
     // [fixed_base, fixed_base + fixed_size) in order and nothing is freed; no device allocation,
     // pinned host buffer, stream or event is created (the handle runs on the per-thread stream)
@@ -88,6 +90,7 @@ void device_free(fw_sim* s, void* p);
 // the handle's kernels and its point table from fw_sim::chosen and spare, after a change of these or of the codes
 int fit_kernels(fw_sim* s);
 int forward_step(fw_sim* s);               // one time step on the handle's stream
+void unbind(struct fw_adj* a);              // give back an adjoint's device memory and part it from its handle
 hipError_t grid_to_host(const fw_sim* s, void* dst, const void* src, size_t esize);  // padded -> compact
 // Host-side set-up of a handle, without device access.
 // Source, pressure-release and sensor points as one time step applies them.

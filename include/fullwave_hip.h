@@ -261,6 +261,8 @@ int fw_adj_forward(fw_adj* adj);
  * [nx, ny(, nz)] (grid_bytes each) receiving dJ/dK and dJ/drho. */
 int fw_adj_backward(fw_adj* adj, const float* grad_rec, size_t grad_bytes, float* grad_k, float* grad_rho,
                     size_t grid_bytes);
+/* Before or after the simulation's handle: destroying that first gives back the adjoint's device memory, and
+ * fw_adj_forward and fw_adj_backward then fail with FW_ERR_STATE. */
 int fw_adj_destroy(fw_adj* adj);
 
 #ifdef __cplusplus

@@ -326,6 +326,60 @@ void per_axis_uploads() {
     }
 }
 
+// Gradients with every list that an adjoint builds (sensors on planes, on sources, on release points and
+// twice on a voxel), destroyed after its simulation's handle, before it, and with the runtime's ordinary
+// allocations in place of the stream-ordered ones.
+void adjoint_lifetimes() {
+    struct Case {
+        int ndim, model, isotropic;
+        int64_t nx, ny, nz, nt, every;
+    };
+    for (const Case& c : {Case{3, 0, 1, 136, 120, 112, 4, 4}, Case{3, 0, 1, 21, 25, 41, 9, 4}, Case{3, 1, 1, 18, 33, 43, 9, 0},
+                          Case{3, 0, 0, 21, 25, 41, 9, 9}, Case{2, 0, 1, 25, 81, 1, 9, 4}, Case{2, 0, 0, 67, 212, 1, 9, 0},
+                          Case{2, 1, 1, 21, 26, 1, 9, 1}}) {
+        Inputs in = inputs(c.ndim, c.nx, c.ny, c.nz, c.nt, c.isotropic, c.model);
+        auto& out = in.i["outc"];
+        auto& air = in.i["icczero"];
+        const int64_t dims[3] = {c.nx, c.ny, in.d.nz};
+        auto plane = [&](int axis) {
+            for (int64_t i = 0; i < dims[0]; ++i)
+                for (int64_t j = 0; j < dims[1]; ++j)
+                    for (int64_t k = 0; k < dims[2]; ++k) {
+                        const int64_t x[3] = {i, j, k};
+                        if (x[axis] != dims[axis] / 2) continue;
+                        for (int a = 0; a < c.ndim; ++a) out.push_back((int32_t)x[a]);
+                    }
+        };
+        for (int a = 0; a < c.ndim; ++a) plane(a);
+        for (int q = 0; q < 12 * c.ndim; ++q) air.push_back((int32_t)(q % c.ndim == 0 ? q % 2 ? dims[0] - 1 : 3 : 0));  // corners
+        for (int q = 0; q < 3 * c.ndim; ++q) air.push_back(in.i["icc"][(size_t)q]);
+        in.d.ncoordszero = (int64_t)air.size() / c.ndim;
+        in.d.ncoordsout = (int64_t)out.size() / c.ndim;
+        for (int order = 0; order < 3; ++order) {
+            rt::async_fails = order == 2;
+            fw_sim* s = make(in);
+            fw_adj* a = nullptr;
+            CHECK(fw_adj_create(s, c.every, &a) == FW_OK);
+            const std::vector<float> w((size_t)(in.d.ncoordsout * ((c.nt + 1) / 2)), 1.f);
+            std::vector<float> gk((size_t)in.cells()), gr((size_t)in.cells());
+            for (int pass = 0; pass < 2; ++pass) {
+                CHECK(fw_adj_forward(a) == FW_OK);
+                CHECK(fw_adj_backward(a, w.data(), w.size() * 4, gk.data(), gr.data(), gk.size() * 4) == FW_OK);
+            }
+            if (order == 1) {
+                CHECK(fw_sim_destroy(s) == FW_OK);
+                CHECK(fw_adj_forward(a) == FW_ERR_STATE);
+                CHECK(fw_adj_backward(a, w.data(), w.size() * 4, gk.data(), gr.data(), gk.size() * 4) == FW_ERR_STATE);
+                CHECK(fw_adj_destroy(a) == FW_OK);
+            } else {
+                CHECK(fw_adj_destroy(a) == FW_OK);
+                CHECK(fw_sim_destroy(s) == FW_OK);
+            }
+            rt::async_fails = false;
+        }
+    }
+}
+
 struct Check {
     const char* name;
     void (*run)();
@@ -337,6 +391,7 @@ const Check checks[] = {
     {"kernels_without_codes", kernels_without_codes},
     {"timing", timing},
     {"per_axis_uploads", per_axis_uploads},
+    {"adjoint_lifetimes", adjoint_lifetimes},
 };
 
 }  // namespace

@@ -87,3 +87,20 @@ def test_bricks_whose_codes_go_and_come_back(monkeypatch, isotropic, graph_steps
         again(other)
         sim.upload(name, inp.maps[name])
         again(want)
+
+
+def test_adjoint_outlives_its_simulation():
+    """Closing the simulation first leaves an adjoint that refuses to run and closes like any other."""
+    from fullwave25_amd.adjoint import HipAdjoint
+
+    inp = inputs((24, 26, 44))
+    adj = HipAdjoint(inp, checkpoint_every=8)
+    adj.forward()
+    weights = np.ones((inp.n_records, inp.ncoordsout), np.float32)
+    assert np.abs(adj.backward(weights)[0]).max() > 0
+    adj.sim.close()
+    with pytest.raises(engine.EngineError, match="destroyed"):
+        adj.forward()
+    with pytest.raises(engine.EngineError, match="destroyed"):
+        adj.backward(weights)
+    adj.close()

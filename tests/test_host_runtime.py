@@ -77,3 +77,7 @@ def test_timing_keeps_the_fastest_kernels(driver):
 
 def test_per_axis_maps_uploaded_again(driver):
     check(driver, "per_axis_uploads")
+
+
+def test_adjoint_destroyed_before_and_after_its_simulation(driver):
+    check(driver, "adjoint_lifetimes")

@@ -37,7 +37,7 @@ struct fw_adj {
     int8_t* vmask = nullptr;  // per distinct voxel: 1 pressure release, 2 source point, 0 neither
     uint8_t* kind = nullptr;  // per device cell (2D, bricks): bit 0 pressure release, 1 source point, 2 sensor voxel
     uint8_t* dc8 = nullptr;   // per device cell: coefficient-set index (grids of the tiled and brick reverse kernels)
-    uint32_t* sets = nullptr; // the set of each tile's (2D) or brick's (3D) arms
+    uint32_t* sets = nullptr; // the sets of each tile's (2D: short, then tall ones) or brick's (3D) arms
     int64_t nvox = 0;
     bool forward_done = false;
 };
@@ -223,7 +223,8 @@ int fw_adj_create(fw_sim* f, int64_t checkpoint_every, fw_adj** out) {
     if (!kind.empty())
         ok = ok && hipMemcpyAsync(a->kind, kind.data(), kind.size(), hipMemcpyHostToDevice, f->stream) == hipSuccess;
     if (ok && fw::adj_tiles(f->ds)) {
-        if (!dalloc((void**)&a->dc8, (size_t)n) || !dalloc((void**)&a->sets, fw::adj_tile_count(f->ds) * 4))
+        const size_t tiles = fw::adj_tile_count(f->ds, false) + fw::adj_tile_count(f->ds, true);
+        if (!dalloc((void**)&a->dc8, (size_t)n) || !dalloc((void**)&a->sets, tiles * 4))
             return cleanup(fw::set_error(FW_ERR_NOMEM, "adjoint set-index map"));
     }
     if (bricks) {
@@ -286,7 +287,21 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
     // the set indices, of the map as it is now
     const bool bricks = a->sets && fw::adj_bricks_supported(f->ds);
     if (a->dc8) ADJ_HIP(fw::launch_adj_set_index(f->ds.dcmap, a->dc8, n, st));
-    if (a->dc8 && nd == 2) ADJ_HIP(fw::launch_adj_tile_sets(f->ds, a->dc8, a->sets, st));
+    const size_t n_short = a->dc8 && nd == 2 ? fw::adj_tile_count(f->ds, false) : 0;
+    if (n_short) ADJ_HIP(fw::launch_adj_tile_sets(f->ds, a->dc8, false, a->sets, st));
+    uint32_t tall_span = 0;
+    if (n_short && fw::adj_may_take_tall_tiles(f->ds)) {
+        std::vector<uint32_t> words(n_short);
+        ADJ_HIP(hipMemcpyAsync(words.data(), a->sets, n_short * 4, hipMemcpyDeviceToHost, st));
+        ADJ_HIP(hipStreamSynchronize(st));
+        if (fw::adj_takes_tall_tiles(f->ds, words)) {
+            words.resize(fw::adj_tile_count(f->ds, true));
+            ADJ_HIP(fw::launch_adj_tile_sets(f->ds, a->dc8, true, a->sets + n_short, st));
+            ADJ_HIP(hipMemcpyAsync(words.data(), a->sets + n_short, words.size() * 4, hipMemcpyDeviceToHost, st));
+            ADJ_HIP(hipStreamSynchronize(st));
+            tall_span = fw::adj_tile_span(words);
+        }
+    }
     if (bricks) ADJ_HIP(fw::launch_adj_brick_sets(f->ds, a->dc8, a->sets, st));
     ADJ_HIP(hipStreamSynchronize(st));  // grad_rec is the caller's buffer, read during the call only
     ADJ_HIP(hipMemsetAsync(a->lam, 0, (size_t)f->nstate * 4, st));
@@ -307,7 +322,8 @@ int fw_adj_backward(fw_adj* a, const float* grad_rec, size_t grad_bytes, float* 
     }
     w.gK = a->work + 3 * nd * n;
     w.dc8 = a->dc8;
-    w.tile_sets = nd == 2 ? a->sets : nullptr;
+    w.tall_span = tall_span;
+    w.tile_sets = nd == 2 ? a->sets + (tall_span ? n_short : 0) : nullptr;
     w.sets = bricks ? a->sets : nullptr;
     float* grho = a->work + (3 * nd + 1) * n;
     fw::AdjSparse sp{};

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace fw {
 
 constexpr int kHalo = 8;      // axial stencil half-width == ghost border width
@@ -251,7 +253,8 @@ struct AdjView {
     const float* tu[kMaxDim];
     const float* tdiv;
     const uint8_t* dc8;  // coefficient-set index per device cell (the tiled 2D kernels; ndmap <= 256; bricks)
-    const uint32_t* tile_sets;  // tiled 2D kernels: the set of each tile's arms, or all ones
+    const uint32_t* tile_sets;  // tiled 2D kernels: the sets of each tile's arms
+    uint32_t tall_span;         // tall tiles: the most sets of one's arms; short tiles: 0
     const uint32_t* sets;  // bricks: the set of each brick's arms, or all ones (null: no bricks)
     float* H[kMaxDim];
     float* G[kMaxDim];
@@ -529,9 +532,15 @@ hipError_t launch_adj_start_bricks(const DevSim& s, const AdjView& w, hipStream_
 hipError_t launch_adj_rest_bricks(const DevSim& s, const AdjView& w, const AdjNext* next, hipStream_t st);
 // the set-index map the tiled kernels read (AdjView::dc8), from dcmap; only where adj_fuses_next
 hipError_t launch_adj_set_index(const int32_t* dcmap, uint8_t* dc8, int64_t n, hipStream_t st);
-// the tiles of a 2D grid, and the set of each one's arms (AdjView::tile_sets)
-size_t adj_tile_count(const DevSim& s);
-hipError_t launch_adj_tile_sets(const DevSim& s, const uint8_t* dc8, uint32_t* sets, hipStream_t st);
+// the tiles of a 2D grid, short ones of 8 rows or tall ones of 16, and the sets of each one's arms
+// (AdjView::tile_sets)
+size_t adj_tile_count(const DevSim& s, bool tall);
+hipError_t launch_adj_tile_sets(const DevSim& s, const uint8_t* dc8, bool tall, uint32_t* sets, hipStream_t st);
+// whether the reverse kernels take tall tiles, by the grid alone and by the short tiles' words; the most sets
+// that one of these words holds
+bool adj_may_take_tall_tiles(const DevSim& s);
+bool adj_takes_tall_tiles(const DevSim& s, const std::vector<uint32_t>& words);
+uint32_t adj_tile_span(const std::vector<uint32_t>& words);
 hipError_t launch_adj_pressure(const DevSim& s, const AdjView& w, hipStream_t st);
 hipError_t launch_adj_rest(const DevSim& s, const AdjView& w, const AdjNext* next, hipStream_t st);
 // the forward kernels that write a tape (DevSim::tape_div set): the per-cell kernels, and the

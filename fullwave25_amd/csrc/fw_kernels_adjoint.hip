@@ -26,6 +26,7 @@
 // alone) and step 5 as another, which also runs steps 1 and 2 of the next (earlier) step for its
 // cells when that step's tape is held (they need lambda_p of the cell alone); in 3D the same on bricks
 // (fw_kernels_adjoint3d.hip); elsewhere each step is its own per-cell kernel.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -317,29 +318,35 @@ __global__ __launch_bounds__(256) void k_adj_dplus_t(DevSim s, AdjView w) {
 // cells). Every lane issues all of its staging loads before it stores any of them, so one memory
 // latency covers the staging. A gather weighs each neighbour by the neighbour's own coefficient
 // set: where the arms of a tile hold one set (AdjView::tile_sets) its weights are scalar
-// registers; a tile of several sets also stages the cells' set indices and the handle's weights
-// (dynamic LDS), two dependent LDS reads a neighbour. The arithmetic and its order are the
+// registers; a tile of several sets also stages the cells' set indices and the weights of the handle's sets
+// (tall tiles: of its own) in dynamic LDS, two dependent LDS reads a neighbour. The arithmetic and its order are the
 // per-cell kernels', so the results are the same bit for bit.
-constexpr int ATX = 8, ATY = 64, kAdjLanes = 256;
-constexpr int AXR = ATX + 16, AXC = ATY + 2;  // axis-x staged region
-constexpr int AYR = ATX + 2, AYC = ATY + 16;  // axis-y staged region
+constexpr int ATY = 64, kAdjLanes = 256;
+constexpr int kShortTile = 8, kTallTile = 16;  // ATX
+constexpr int AXC = ATY + 2, AYC = ATY + 16;   // columns of the staged regions
+// How a launch weighs: the grid has one set; tiles of one set and tiles that look theirs up in the whole
+// table; tiles that all look up, in a table of their own sets.
+enum { kOneSet = 0, kAnySets = 1, kLookUp = 2 };
 constexpr int kAdjLdsSets = 256;  // coefficient sets staged (ndmap beyond: per-cell kernels)
-constexpr uint32_t kMixedSets = 0xffffffffu;
+// A tile's word in AdjView::tile_sets: the lowest set of its arms, and how many from there.
+__device__ __forceinline__ uint32_t lowest_set(uint32_t word) { return word & 0xffu; }
+__device__ __forceinline__ uint32_t set_span(uint32_t word) { return word >> 8; }
 
-// Stage R x C cells of `f` from row i, column j, with MIXED their set indices too; load first, put after.
+// Stage R x C cells of `f` from row i, column j, with MIXED their set indices (above `lowest`) too; load
+// first, put after.
 template <int R, int C, bool MIXED>
 struct GatherStage {
     static constexpr int N = (R * C + kAdjLanes - 1) / kAdjLanes;
     float v[N];
     uint8_t d[MIXED ? N : 1];
-    __device__ __forceinline__ void load(const DevSim& s, const float* f, const uint8_t* dc8, int i, int j) {
+    __device__ __forceinline__ void load(const DevSim& s, const float* f, const uint8_t* dc8, uint32_t lowest, int i, int j) {
 #pragma unroll
         for (int q = 0; q < N; ++q) {
             const int t = min((int)threadIdx.x + q * kAdjLanes, R * C - 1);
             const int r = t / C, cc = t - r * C;
             const uint32_t c = (uint32_t)(min(max(i + r, 0), (int)s.nx - 1) * (int)s.ny + min(max(j + cc, 0), (int)s.ny - 1));
             v[q] = gld32(f, c);
-            if (MIXED) d[q] = dc8[c];
+            if (MIXED) d[q] = (uint8_t)(dc8[c] - lowest);
         }
     }
     __device__ __forceinline__ void put(float* F, uint8_t* D) const {
@@ -352,22 +359,46 @@ struct GatherStage {
         }
     }
 };
-template <bool MIXED>
-__device__ __forceinline__ void stage_gather(const DevSim& s, const uint8_t* dc8, const float* fx, const float* fy, int i0, int j0,
-                                             float* FX, float* FY, uint8_t* DX, uint8_t* DY, float* CT) {
-    GatherStage<AXR, AXC, MIXED> x;
-    GatherStage<AYR, AYC, MIXED> y;
-    x.load(s, fx, dc8, i0 - 8, j0 - 1);
-    y.load(s, fy, dc8, i0 - 1, j0 - 8);
-    if (MIXED)
+// The weights of `n` sets from `lowest`, as pairs (9 a set), five loads in flight a lane.
+__device__ __forceinline__ void stage_weights(const DevSim& s, uint32_t lowest, int sets, float* CT) {
+    const int n = sets * kNCoef;
+    const float2* from = reinterpret_cast<const float2*>(s.coef) + lowest * kNCoef;
+    float2* to = reinterpret_cast<float2*>(CT);
+    if (n <= 2 * kAdjLanes) {
+        for (int t = threadIdx.x; t < n; t += kAdjLanes) to[t] = from[t];
+        return;
+    }
+    constexpr int K = 5;
+    for (int t0 = threadIdx.x; t0 < n; t0 += K * kAdjLanes) {
+        float2 v[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) v[k] = from[min(t0 + k * kAdjLanes, n - 1)];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (t0 + k * kAdjLanes < n) to[t0 + k * kAdjLanes] = v[k];
+    }
+}
+// word: the tile's, with OWN table of its sets; else the handle's table.
+template <int ATX, bool MIXED, bool OWN>
+__device__ __forceinline__ void stage_gather(const DevSim& s, const uint8_t* dc8, uint32_t word, const float* fx, const float* fy,
+                                             int i0, int j0, float* FX, float* FY, uint8_t* DX, uint8_t* DY, float* CT) {
+    GatherStage<ATX + 16, AXC, MIXED> x;
+    GatherStage<ATX + 2, AYC, MIXED> y;
+    x.load(s, fx, dc8, OWN ? lowest_set(word) : 0u, i0 - 8, j0 - 1);
+    y.load(s, fy, dc8, OWN ? lowest_set(word) : 0u, i0 - 1, j0 - 8);
+    if (MIXED && OWN) stage_weights(s, lowest_set(word), (int)set_span(word), CT);
+    if (MIXED && !OWN)
         for (int t = threadIdx.x; t < s.ndmap * 2 * kNCoef; t += kAdjLanes) CT[t] = s.coef[t];
     x.put(FX, DX);
     y.put(FY, DY);
 }
 
-// The set of the updated cells in each tile's arms, or kMixedSets.
+// Each tile's word: of the updated cells in its arms (the fields are 0 elsewhere); of tall tiles, whose tables
+// hold no other sets, every cell of the grid in its arms.
+template <int ATX>
 __global__ __launch_bounds__(kAdjLanes) void k_adj_tile_sets(DevSim s, const uint8_t* dc8, uint32_t* sets) {
     __shared__ uint32_t least, most;
+    constexpr int edge = ATX == kTallTile ? 0 : kHalo;
     const int i0 = kHalo + (int)blockIdx.y * ATX, j0 = kHalo + (int)blockIdx.x * ATY;
     if (threadIdx.x == 0) {
         least = 255;
@@ -379,7 +410,7 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_tile_sets(DevSim s, const uin
         const int ei = a ? 1 : 8, ej = a ? 8 : 1, cols = ATY + 2 * ej, n = (ATX + 2 * ei) * cols;
         for (int t = threadIdx.x; t < n; t += kAdjLanes) {
             const int i = i0 - ei + t / cols, j = j0 - ej + t % cols;
-            if (i < kHalo || i >= (int)s.nx - kHalo || j < kHalo || j >= (int)s.ny - kHalo) continue;
+            if (i < edge || i >= (int)s.nx - edge || j < edge || j >= (int)s.ny - edge) continue;
             const uint32_t set = dc8[(uint32_t)(i * (int)s.ny + j)];
             lo = min(lo, set);
             hi = max(hi, set);
@@ -388,7 +419,7 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_tile_sets(DevSim s, const uin
     atomicMin(&least, lo);
     atomicMax(&most, hi);
     __syncthreads();
-    if (threadIdx.x == 0) sets[blockIdx.x + blockIdx.y * gridDim.x] = least == most ? least : kMixedSets;
+    if (threadIdx.x == 0) sets[blockIdx.x + blockIdx.y * gridDim.x] = (most - least + 1) << 8 | least;
 }
 
 // DMINUS: lambda_v_a += (D-_a)^T H_a, then the velocity transposed of the cell (EXPO, CODED as
@@ -401,16 +432,18 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_tile_sets(DevSim s, const uin
 // workgroups a CU), the memory traffic on large ones. us a reverse step with 6 sound speeds, tiles of 16
 // rows that always looked weights up -> these with 16 rows -> with 8 rows: 240 x 256 22.6 -> 20.0 -> 14.5;
 // 640 x 640 30.9 -> 27.4 -> 26.0; 1184 x 1184 71.4 -> 70.7 -> 65.9; 1700 x 1700 152.6 -> 150.4 -> 147.7.
-// One sound speed, 640 x 640: 24.1 -> 23.0 -> 21.3; exponential model 27.6 -> 25.1 -> 23.9. 130 sound speeds on
-// 1152 x 1152 (every tile looks its weights up): 55.6 -> 55.5 us of kernels. Measured and left
-// out: both rows' operands and table rows before the staging (640 x 640: 28.3).
-template <bool UNI, bool DMINUS, bool EXPO, bool CODED, bool NEXT>
+// One sound speed, 640 x 640: 24.1 -> 23.0 -> 21.3; exponential model 27.6 -> 25.1 -> 23.9. Many sets on large
+// grids: tiles of 16 rows that all look up, in a table of the sets that they hold (adj_may_take_tall_tiles).
+// Measured and left out: both rows' operands and table rows before the staging (640 x 640: 28.3); in the
+// short tiles the tile's own table (640 x 640, 6 sets: 25.8 -> 26.1; 1152 x 1152, 31 sets: 63.2 -> 63.7).
+template <int ATX, int SETS, bool DMINUS, bool EXPO, bool CODED, bool NEXT>
 __global__ __launch_bounds__(kAdjLanes) void k_adj_gather_tile2d(DevSim s, AdjView w, AdjNext nx) {
+    constexpr int AXR = ATX + 16, AYR = ATX + 2;  // rows of the staged regions
     __shared__ float FX[AXR * AXC];
     __shared__ float FY[AYR * AYC];
-    __shared__ uint8_t DX[UNI ? 1 : AXR * AXC];
-    __shared__ uint8_t DY[UNI ? 1 : AYR * AYC];
-    extern __shared__ float CT[];  // [set][axis][9], the handle's sets
+    __shared__ uint8_t DX[SETS == kOneSet ? 1 : AXR * AXC];
+    __shared__ uint8_t DY[SETS == kOneSet ? 1 : AYR * AYC];
+    extern __shared__ __attribute__((aligned(8))) float CT[];  // [set][axis][9], the handle's sets or the tile's
     constexpr int NR = ATX / 4;    // rows per lane: rl, rl + 4, ...
     // Each XCD takes a contiguous run of tiles, so that neighbouring tiles, which stage the same halo
     // cells, share an L2: the fetch from memory drops by 40 % and the kernels run 17 % faster than with
@@ -437,10 +470,11 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_gather_tile2d(DevSim s, AdjVi
         }
     };
     if (nrows > 0) load(0, ops[0]);
-    const uint32_t set = UNI ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(w.tile_sets[tile]);
+    const uint32_t word = SETS == kOneSet ? 1u << 8 : (uint32_t)__builtin_amdgcn_readfirstlane(w.tile_sets[tile]);
+    const bool one = SETS == kOneSet || (SETS == kAnySets && set_span(word) == 1);
     const float *fx = DMINUS ? w.H[0] : w.G[0], *fy = DMINUS ? w.H[1] : w.G[1];
-    if (UNI || set != kMixedSets) stage_gather<false>(s, w.dc8, fx, fy, (int)i0, (int)j0, FX, FY, DX, DY, CT);
-    else stage_gather<true>(s, w.dc8, fx, fy, (int)i0, (int)j0, FX, FY, DX, DY, CT);
+    if (one) stage_gather<ATX, false, false>(s, w.dc8, word, fx, fy, (int)i0, (int)j0, FX, FY, DX, DY, CT);
+    else stage_gather<ATX, true, SETS == kLookUp>(s, w.dc8, word, fx, fy, (int)i0, (int)j0, FX, FY, DX, DY, CT);
     __syncthreads();
     // staged element at (di, dj) from cell (il, jl) of the tile, for axis x's and axis y's field
     auto ex = [&](int il, int di, int dj) { return (il + 8 + di) * AXC + (jl + 1 + dj); };
@@ -511,9 +545,9 @@ __global__ __launch_bounds__(kAdjLanes) void k_adj_gather_tile2d(DevSim s, AdjVi
             }
         }
     };
-    if (UNI || set != kMixedSets) {
+    if (one) {
         float kx[kNCoef], ky[kNCoef];
-        const scalar_ptr c = as_scalar(s.coef) + set * 2 * kNCoef;
+        const scalar_ptr c = as_scalar(s.coef) + lowest_set(word) * 2 * kNCoef;
 #pragma unroll
         for (int k = 0; k < kNCoef; ++k) {
             kx[k] = c[k];
@@ -571,7 +605,7 @@ hipError_t launch_adj_sparse(float* lp, const float* grow, const AdjSparse& sp, 
 
 // the transposed gathers on LDS tiles: 2D grids of at most kAdjLdsSets coefficient sets (the
 // staged set indices are bytes)
-bool adj_tiles(const DevSim& s) { return s.ndim == 2 && s.ndmap <= kAdjLdsSets && s.nx * s.ny < ((int64_t)1 << 30) && s.nx < ATX * (int64_t)65535; }
+bool adj_tiles(const DevSim& s) { return s.ndim == 2 && s.ndmap <= kAdjLdsSets && s.nx * s.ny < ((int64_t)1 << 30) && s.nx < kShortTile * (int64_t)65535; }
 
 // FULLWAVE_HIP_ADJ_GATHERS=percell keeps the per-cell kernels (to compare the two forms)
 bool adj_percell_gathers() {
@@ -587,29 +621,54 @@ hipError_t launch_adj_set_index(const int32_t* dcmap, uint8_t* dc8, int64_t n, h
     return hipGetLastError();
 }
 
-static dim3 adj_tile_grid(const DevSim& s) {
-    return dim3((unsigned)((s.ny - 2 * kHalo + ATY - 1) / ATY), (unsigned)((s.nx - 2 * kHalo + ATX - 1) / ATX));
+static dim3 adj_tile_grid(const DevSim& s, bool tall) {
+    const int rows = tall ? kTallTile : kShortTile;
+    return dim3((unsigned)((s.ny - 2 * kHalo + ATY - 1) / ATY), (unsigned)((s.nx - 2 * kHalo + rows - 1) / rows));
 }
 
-size_t adj_tile_count(const DevSim& s) {
-    const dim3 g = adj_tile_grid(s);
+size_t adj_tile_count(const DevSim& s, bool tall) {
+    const dim3 g = adj_tile_grid(s, tall);
     return (size_t)g.x * g.y;
 }
 
-hipError_t launch_adj_tile_sets(const DevSim& s, const uint8_t* dc8, uint32_t* sets, hipStream_t st) {
-    hipLaunchKernelGGL(k_adj_tile_sets, adj_tile_grid(s), dim3(kAdjLanes), 0, st, s, dc8, sets);
+// Tall tiles stage fewer halo cells a cell (3.5 against 4.7); short ones have twice as many workgroups, weigh
+// tiles of one set with scalars, and stage the whole table in the others. us a reverse step, short -> tall, of
+// media whose tiles mostly hold several sets, smooth / random cells (short tiles in brackets):
+//   sets   640 x 640 (780)               900 x 900 (1554)             1152 x 1152 (2556)
+//     6    27.5 -> 31.5 / 27.1 -> 30.1   39.8 -> 42.8 / 42.6 -> 43.4   56.3 -> 56.8 / 60.4 -> 58.7
+//    30    27.8 -> 30.0 / 29.9 -> 31.6   43.3 -> 42.8 / 45.5 -> 46.3   60.6 -> 56.9 / 64.7 -> 61.5
+//   130    29.4 -> 30.2 / 34.9 -> 34.2   46.4 -> 43.1 / 52.5 -> 52.7   64.8 -> 57.7 / 75.1 -> 67.9
+// So tall from 32 sets and 1280 short tiles (five workgroups a CU, the most that run at once), where the
+// part of the short tiles that hold several sets makes up for the others: at 130 sets on 1152 x 1152 with
+// 38 % of them 60.6 -> 57.7, with 13 % left short at 56.4 (tall: 57.5).
+bool adj_may_take_tall_tiles(const DevSim& s) { return s.ndmap >= 32 && adj_tile_count(s, false) >= 1280; }
+
+bool adj_takes_tall_tiles(const DevSim& s, const std::vector<uint32_t>& words) {
+    size_t several = 0;
+    for (uint32_t w : words) several += (w >> 8) > 1;
+    return (double)several >= (0.2 + 16.0 / s.ndmap) * (double)words.size();
+}
+
+uint32_t adj_tile_span(const std::vector<uint32_t>& words) {
+    uint32_t span = 1;
+    for (uint32_t w : words) span = std::max(span, w >> 8);
+    return span;
+}
+
+hipError_t launch_adj_tile_sets(const DevSim& s, const uint8_t* dc8, bool tall, uint32_t* sets, hipStream_t st) {
+    const dim3 g = adj_tile_grid(s, tall);
+    if (tall) hipLaunchKernelGGL(k_adj_tile_sets<kTallTile>, g, dim3(kAdjLanes), 0, st, s, dc8, sets);
+    else hipLaunchKernelGGL(k_adj_tile_sets<kShortTile>, g, dim3(kAdjLanes), 0, st, s, dc8, sets);
     return hipGetLastError();
 }
 
 template <bool DMINUS, bool EXPO, bool CODED, bool NEXT>
 void launch_gather_tile2d(const DevSim& s, const AdjView& w, const AdjNext& nx, hipStream_t st) {
-    const dim3 g = adj_tile_grid(s);
-    if (s.ndmap == 1) {
-        hipLaunchKernelGGL((k_adj_gather_tile2d<true, DMINUS, EXPO, CODED, NEXT>), g, dim3(kAdjLanes), 0, st, s, w, nx);
-        return;
-    }
-    const size_t lds = (size_t)s.ndmap * 2 * kNCoef * sizeof(float);
-    hipLaunchKernelGGL((k_adj_gather_tile2d<false, DMINUS, EXPO, CODED, NEXT>), g, dim3(kAdjLanes), lds, st, s, w, nx);
+    const dim3 g = adj_tile_grid(s, w.tall_span != 0), b(kAdjLanes);
+    const size_t lds = (size_t)(w.tall_span ? w.tall_span : (uint32_t)s.ndmap) * 2 * kNCoef * sizeof(float);
+    if (s.ndmap == 1) hipLaunchKernelGGL((k_adj_gather_tile2d<kShortTile, kOneSet, DMINUS, EXPO, CODED, NEXT>), g, b, 0, st, s, w, nx);
+    else if (w.tall_span) hipLaunchKernelGGL((k_adj_gather_tile2d<kTallTile, kLookUp, DMINUS, EXPO, CODED, NEXT>), g, b, lds, st, s, w, nx);
+    else hipLaunchKernelGGL((k_adj_gather_tile2d<kShortTile, kAnySets, DMINUS, EXPO, CODED, NEXT>), g, b, lds, st, s, w, nx);
 }
 
 static bool adj_coded(const DevSim& s) { return !s.aexp && s.isotropic && s.rcode; }

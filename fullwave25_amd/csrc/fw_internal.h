@@ -181,10 +181,11 @@ __device__ __forceinline__ float corrected(float D, float ik, float q1, float q2
 #pragma clang fp contract(off)
     return __builtin_fmaf(D, ik, q1 + q2);
 }
-// v - dt / rho_bar u, rho_bar the mean of the two voxels' densities
+// v - dt / rho_bar u, rho_bar the mean of the two voxels' densities (the sign on u: on the quotient the 2D
+// marching kernels take 4 registers more and lose a wavefront a SIMD, 4256 x 2208 cells 103 -> 150 us)
 __device__ __forceinline__ float velocity_step(float v, float dt, float rho0, float rho1, float u) {
 #pragma clang fp contract(off)
-    return __builtin_fmaf(-(dt / (0.5f * (rho0 + rho1))), u, v);
+    return __builtin_fmaf(dt / (0.5f * (rho0 + rho1)), -u, v);
 }
 // p - dt K div
 __device__ __forceinline__ float pressure_step(float p, float dt, float K, float div) {

@@ -66,11 +66,18 @@ __device__ inline bool cell_of_lane(const DevSim& s, unsigned tile, unsigned gx,
 // offset where the grid has fewer than 2^30 cells
 __device__ __forceinline__ float at(const float* f, int64_t base, uint32_t c) { return gld32(f + base, c); }
 __device__ __forceinline__ float at(const float* f, int64_t base, int64_t c) { return f[base + c]; }
-__device__ __forceinline__ float at_nt(const float* f, uint32_t c) { return gldnt(f, c); }
+template <bool NT>
+__device__ __forceinline__ float at_nt(const float* f, uint32_t c) { return NT ? gldnt(f, c) : gld32(f, c); }
+template <bool NT>
 __device__ __forceinline__ float at_nt(const float* f, int64_t c) { return f[c]; }
 __device__ __forceinline__ void put(float* f, uint32_t c, float v) { gst32(f, c, v); }
 __device__ __forceinline__ void put(float* f, int64_t c, float v) { f[c] = v; }
-__device__ __forceinline__ void put_nt(float* f, uint32_t c, float v) { gstnt(f, c, v); }
+template <bool NT>
+__device__ __forceinline__ void put_nt(float* f, uint32_t c, float v) {
+    if (NT) gstnt(f, c, v);
+    else gst32(f, c, v);
+}
+template <bool NT>
 __device__ __forceinline__ void put_nt(float* f, int64_t c, float v) { f[c] = v; }
 
 // The coefficients of a cell: one set for all axes, or (kCellAxes) one per axis; the weights of axis 0.
@@ -163,7 +170,7 @@ __device__ inline void coef_tail(CellCoef<ND, MODEL>& k, const DevSim& s, Idx c)
 }
 
 // TAPE: also write the adjoint tape of the step (DevSim::tape_u, tape_div)
-template <int ND, int MODEL, bool TAPE, class Idx>
+template <int ND, int MODEL, bool TAPE, bool NT, class Idx>
 __global__ __launch_bounds__(256) void k_velocity_cell(DevSim batch, unsigned gx) {
     const DevSim s = shot_view(batch, blockIdx.y);
     Idx c;
@@ -189,8 +196,8 @@ __global__ __launch_bounds__(256) void k_velocity_cell(DevSim batch, unsigned gx
         rho_n[a] = at(s.rho, sa, c);
         v[a] = at(s.v[a], 0, c);
         if (MODEL != kCellExpo) {
-            psi[a][0] = at_nt(s.psi[a][0], c);
-            psi[a][1] = at_nt(s.psi[a][1], c);
+            psi[a][0] = at_nt<NT>(s.psi[a][0], c);
+            psi[a][1] = at_nt<NT>(s.psi[a][1], c);
         }
     }
     rho_c = at(s.rho, 0, c);
@@ -218,15 +225,15 @@ __global__ __launch_bounds__(256) void k_velocity_cell(DevSim batch, unsigned gx
         constexpr bool axes = MODEL == kCellAxes;
         const float q1 = memory_step(k.b[axes ? a : 0][0], psi[a][0], k.a[axes ? a : 0][0], D);
         const float q2 = memory_step(k.b[axes ? a : 0][1], psi[a][1], k.a[axes ? a : 0][1], D);
-        put_nt(s.psi[a][0], c, q1);
-        put_nt(s.psi[a][1], c, q2);
+        put_nt<NT>(s.psi[a][0], c, q1);
+        put_nt<NT>(s.psi[a][1], c, q2);
         const float u = corrected(D, k.ik[axes ? a : 0], q1, q2);
         put(s.v[a], c, velocity_step(v[a], s.dt, rho_c, rho_n[a], u));
         if (TAPE) put(s.tape_u[a], c, u);
     }
 }
 
-template <int ND, int MODEL, bool TAPE, class Idx>
+template <int ND, int MODEL, bool TAPE, bool NT, class Idx>
 __device__ inline void pressure_cell(const DevSim& s, Idx c) {
     CellCoef<ND, MODEL> k;
     coef_head(k, s, c);
@@ -251,8 +258,8 @@ __device__ inline void pressure_cell(const DevSim& s, Idx c) {
             side[a][b][3] = at(va, -sa - sb, c);
         }
         if (MODEL != kCellExpo) {
-            phi[a][0] = at_nt(s.phi[a][0], c);
-            phi[a][1] = at_nt(s.phi[a][1], c);
+            phi[a][0] = at_nt<NT>(s.phi[a][0], c);
+            phi[a][1] = at_nt<NT>(s.phi[a][1], c);
         }
     }
     const float p = at(s.p, 0, c), K = at(s.K, 0, c);
@@ -279,8 +286,8 @@ __device__ inline void pressure_cell(const DevSim& s, Idx c) {
         constexpr bool axes = MODEL == kCellAxes;
         const float q1 = memory_step(k.b[axes ? a : 0][0], phi[a][0], k.a[axes ? a : 0][0], D);
         const float q2 = memory_step(k.b[axes ? a : 0][1], phi[a][1], k.a[axes ? a : 0][1], D);
-        put_nt(s.phi[a][0], c, q1);
-        put_nt(s.phi[a][1], c, q2);
+        put_nt<NT>(s.phi[a][0], c, q1);
+        put_nt<NT>(s.phi[a][1], c, q2);
         div += corrected(D, k.ik[axes ? a : 0], q1, q2);
     }
     const float out = pressure_step(p, s.dt, K, div);
@@ -290,7 +297,7 @@ __device__ inline void pressure_cell(const DevSim& s, Idx c) {
 
 // gs.g non-null: each workgroup then also does the step's source, pressure-release and sensor work of
 // its tile (tile blockIdx.x of shot blockIdx.y)
-template <int ND, int MODEL, bool TAPE, class Idx>
+template <int ND, int MODEL, bool TAPE, bool NT, class Idx>
 __global__ __launch_bounds__(256) void k_pressure_cell(DevSim batch, unsigned gx, GroupStep gs) {
     TileWork w{};
     if (gs.g) {
@@ -299,7 +306,7 @@ __global__ __launch_bounds__(256) void k_pressure_cell(DevSim batch, unsigned gx
     }
     const DevSim s = shot_view(batch, blockIdx.y);
     Idx c;
-    if (cell_of_lane<ND, Idx>(s, cell_tile<ND>(), gx, c)) pressure_cell<ND, MODEL, TAPE, Idx>(s, c);
+    if (cell_of_lane<ND, Idx>(s, cell_tile<ND>(), gx, c)) pressure_cell<ND, MODEL, TAPE, NT, Idx>(s, c);
     if (!gs.g) return;
     __syncthreads();
     tile_boundary(w);
@@ -438,25 +445,40 @@ int64_t cell_tiles(const DevSim& s) {
 int64_t cell_first_row(const DevSim& s) { return cell_rows(s).first; }
 int64_t cell_row_count(const DevSim& s) { return cell_rows(s).count; }
 
-template <int ND, int MODEL, bool TAPE, class Idx>
+template <int ND, int MODEL, bool TAPE, bool NT, class Idx>
 static hipError_t launch_cell(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st) {
     const int64_t tiles = cell_tiles(s);
     if (tiles > 0x7fffffff) return hipErrorInvalidValue;
     const dim3 g((unsigned)tiles, (unsigned)s.nshots), b(kCellTileCols * kCellTileRows);
-    if (velocity) hipLaunchKernelGGL((k_velocity_cell<ND, MODEL, TAPE, Idx>), g, b, 0, st, s, cell_tiles_x(s));
-    else hipLaunchKernelGGL((k_pressure_cell<ND, MODEL, TAPE, Idx>), g, b, 0, st, s, cell_tiles_x(s), gs);
+    if (velocity) hipLaunchKernelGGL((k_velocity_cell<ND, MODEL, TAPE, NT, Idx>), g, b, 0, st, s, cell_tiles_x(s));
+    else hipLaunchKernelGGL((k_pressure_cell<ND, MODEL, TAPE, NT, Idx>), g, b, 0, st, s, cell_tiles_x(s), gs);
     return hipGetLastError();
 }
 
-// 32-bit offsets where the grid (with the row padding of its last plane) has fewer than 2^30 cells
+// Whether the memory variables go past the caches (non-temporal): in 3D where the arrays of a step (so many
+// of 4 bytes a cell) exceed the memory-side cache of 256 MB by a third or more anyway; 2D grids of any
+// size. us a step, past the caches / through them:
+//   codes  112 x 120 x 100  59 / 47   128 x 136 x 128  77 / 61   180 x 170 x 180  212 / 234
+//   maps   112 x 120 x 100  62 / 53   128 x 136 x 128  81 / 71   150 x 140 x 150  134 / 148
+//   axes   112 x 120 x 100  64 / 60   128 x 136 x 128  96 / 101  150 x 160 x 170  207 / 217
+static bool cell_memory_streams(const DevSim& s, int model) {
+    return s.nx * s.sx * (int64_t)s.nshots * (model == kCellCoded ? 20 : model == kCellMaps ? 29 : 49) >= ((int64_t)20 << 22);
+}
+
+template <int ND, int MODEL, bool TAPE>
+static hipError_t launch_cell_tape(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st) {
+    // 32-bit offsets where the grid (with the row padding of its last plane) has fewer than 2^30 cells
+    if (s.nx * s.sx >= ((int64_t)1 << 30)) return launch_cell<ND, MODEL, TAPE, true, int64_t>(s, velocity, gs, st);
+    if constexpr (ND == 3 && MODEL != kCellExpo) {  // (the exponential model has no memory variables)
+        if (!cell_memory_streams(s, MODEL)) return launch_cell<ND, MODEL, TAPE, false, uint32_t>(s, velocity, gs, st);
+    }
+    return launch_cell<ND, MODEL, TAPE, true, uint32_t>(s, velocity, gs, st);
+}
+
 template <int ND, int MODEL>
 static hipError_t launch_cell_model(const DevSim& s, bool velocity, const GroupStep& gs, hipStream_t st) {
-    const bool small = s.nx * s.sx < ((int64_t)1 << 30);
-    if (s.tape_div)
-        return small ? launch_cell<ND, MODEL, true, uint32_t>(s, velocity, gs, st)
-                     : launch_cell<ND, MODEL, true, int64_t>(s, velocity, gs, st);
-    return small ? launch_cell<ND, MODEL, false, uint32_t>(s, velocity, gs, st)
-                 : launch_cell<ND, MODEL, false, int64_t>(s, velocity, gs, st);
+    return s.tape_div ? launch_cell_tape<ND, MODEL, true>(s, velocity, gs, st)
+                      : launch_cell_tape<ND, MODEL, false>(s, velocity, gs, st);
 }
 
 template <int ND>

@@ -118,8 +118,11 @@ int64_t auto_segment(const fw_sim* f, size_t free_bytes) {
 }
 
 // Kernels that write the tape (the tiled 2D, brick 3D or per-cell families): the tiled ones (8 rows)
-// or bricks where the grid takes them (136 x 120 x 112: a taped step 85 -> 58 us), else the per-cell
-// ones; a kernel the caller pinned stays if it writes the tape.
+// or bricks where the grid takes them, else the per-cell ones; a kernel the caller pinned stays if it writes
+// the tape. A grid of few bricks leaves most of the chip idle: us a taped step, per-cell / bricks, relaxation and
+// exponential model: 24 x 26 x 44 (8 bricks) 8.6 / 15.9 and 8.7 / 14.8; 64 x 64 x 64 (144) 13.6 / 16.7 and 11.9 / 12.6; 68 x
+// 66 x 64 (182) 15.6 / 16.6 and 14.1 / 12.6; 72 x 72 x 72 (196) 21.5 / 17.9 and 19.0 / 13.9.
+constexpr int64_t kMinTapeBricks = 160;
 void tape_kernels(fw_sim* f) {
     fw::LaunchCfg t;
     t.variant = 2;
@@ -130,7 +133,8 @@ void tape_kernels(fw_sim* f) {
         t.width = fw::kBrickZ;
         t.chunk = 1;
     }
-    if (!fw::tape_capable(f->ds, t)) t.variant = 0;
+    const fw::BrickGrid g = fw::brick_grid(f->ds);
+    if (!fw::tape_capable(f->ds, t) || (t.variant == 5 && g.nx * g.ny * g.nz < kMinTapeBricks)) t.variant = 0;
     for (int kind = 0; kind < 2; ++kind) {
         fw::LaunchCfg& c = f->chosen[kind];
         if (!(f->pinned[kind] && fw::tape_capable(f->ds, c))) c = t;

@@ -183,6 +183,7 @@ void kernels_without_codes() {
         fw_sim* s = make(in);
         if (how == 1) CHECK(fw_sim_set_field(s, "p", zero.data(), zero.size() * 4) == FW_OK);
         fw_adj* a = nullptr;
+        if (how == 2) pin(s, 5, 32, 1);  // (few bricks: not the adjoint's own choice)
         if (how == 2) CHECK(fw_adj_create(s, 8, &a) == FW_OK);
         for (int round = 0; round < 2; ++round) {
             run_and_check(s, in, 10);
@@ -380,6 +381,28 @@ void adjoint_lifetimes() {
     }
 }
 
+// The kernels of an adjoint's taped steps: bricks from 160 of them on, else the per-cell kernels; a pinned
+// family that writes the tape stays.
+void taped_kernels() {
+    struct Case {
+        int64_t nx, ny, nz;
+        int variant;
+    };
+    for (int model : {0, 1})
+        for (const Case& c : {Case{24, 26, 44, 0}, Case{64, 64, 64, 0}, Case{68, 66, 64, 5}})
+            for (bool pinned : {false, true}) {
+                const Inputs in = inputs(3, c.nx, c.ny, c.nz, 4, 1, model);
+                fw_sim* s = make(in);
+                if (pinned) pin(s, 5, 32, 0);
+                fw_adj* a = nullptr;
+                CHECK(fw_adj_create(s, 2, &a) == FW_OK);
+                const int want = pinned ? 5 : c.variant;
+                for (int kind = 0; kind < 2; ++kind) CHECK(config(s, kind)[0] == '0' + want);
+                CHECK(fw_adj_forward(a) == FW_OK);
+                CHECK(fw_adj_destroy(a) == FW_OK && fw_sim_destroy(s) == FW_OK);
+            }
+}
+
 struct Check {
     const char* name;
     void (*run)();
@@ -392,6 +415,7 @@ const Check checks[] = {
     {"timing", timing},
     {"per_axis_uploads", per_axis_uploads},
     {"adjoint_lifetimes", adjoint_lifetimes},
+    {"taped_kernels", taped_kernels},
 };
 
 }  // namespace

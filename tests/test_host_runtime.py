@@ -81,3 +81,7 @@ def test_per_axis_maps_uploaded_again(driver):
 
 def test_adjoint_destroyed_before_and_after_its_simulation(driver):
     check(driver, "adjoint_lifetimes")
+
+
+def test_kernels_of_taped_steps(driver):
+    check(driver, "taped_kernels")

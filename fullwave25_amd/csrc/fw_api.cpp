@@ -837,7 +837,10 @@ int encode_relaxation(fw_sim* s) {
         s->ds.rtab_p = (const float*)tp;
         s->ncodes = n;
         s->coded_cells = covered;
-        if (n <= fw::kMaxWideCodes && s->ds.coef_axes_same) {  // rows with weights for the per-cell kernels
+        // rows with weights for the per-cell and brick kernels, which take it that no cell escapes: only tuples
+        // beyond kMaxCodes get no code
+        static_assert(fw::kMaxWideCodes < fw::kMaxCodes, "grids with wide rows code every cell");
+        if (n <= fw::kMaxWideCodes && covered == s->ncell && s->ds.coef_axes_same) {
             void *wv, *wp;
             if ((r = alloc(s, "_rwide_v", (size_t)n * fw::kWideStride * 4, &wv)) != FW_OK) return r;
             if ((r = alloc(s, "_rwide_p", (size_t)n * fw::kWideStride * 4, &wp)) != FW_OK) return r;

@@ -58,8 +58,8 @@ struct DevSim {
     const float* rtab_v;
     const float* rtab_p;
     // the same rows with the stencil weights of the row's set, kWideStride floats {1/kappa, a1, a2, b1,
-    // b2, w_1..w_8, e, 0, 0}, for the per-cell kernels (null: more than kMaxWideCodes codes, or axes
-    // with weights of their own)
+    // b2, w_1..w_8, e, 0, 0}, for the per-cell and brick kernels (null: more than kMaxWideCodes codes, or axes
+    // with weights of their own). A grid that has them has a code for every cell, none escapes.
     const float* rwide_v;
     const float* rwide_p;
 

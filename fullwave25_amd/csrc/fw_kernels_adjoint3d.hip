@@ -166,8 +166,7 @@ struct QuadCoefs {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const uint32_t code = ((e < 2 ? cw.x : cw.y) >> (16 * (e & 1))) & 0xffffu;
-            q[e] = coded_coef(VEL ? s.rtab_v : s.rtab_p, code != kCodeEscape ? code : 0u);
-            if (code == kCodeEscape) q[e] = escape_coef<VEL, true>(s, c + e);
+            q[e] = coded_coef(VEL ? s.rtab_v : s.rtab_p, code);
         }
     }
 };

@@ -127,15 +127,15 @@ __device__ inline void coef_maps(CellCoef<ND, MODEL>& k, const DevSim& s, Idx c)
 }
 
 // The rest of the chain: the row of the code, or the weights of the set.
-template <int ND, int MODEL, bool VEL, class Idx>
-__device__ inline void coef_tail(CellCoef<ND, MODEL>& k, const DevSim& s, Idx c) {
+template <int ND, int MODEL, bool VEL>
+__device__ inline void coef_tail(CellCoef<ND, MODEL>& k, const DevSim& s) {
     if (MODEL != kCellCoded) {
         load_weights(k.w, s, k.dc, ND, 0);
         return;
     }
     const float* tab = VEL ? s.rwide_v : s.rwide_p;
     const uint32_t c0 = __builtin_amdgcn_readfirstlane(k.code);
-    if (c0 != kCodeEscape && __all(k.code == c0)) {
+    if (__all(k.code == c0)) {
         const scalar_ptr row = as_scalar(tab) + c0 * kWideStride;
         k.ik[0] = row[0];
         k.a[0][0] = row[1];
@@ -146,7 +146,7 @@ __device__ inline void coef_tail(CellCoef<ND, MODEL>& k, const DevSim& s, Idx c)
         for (int m = 0; m < kNCoef; ++m) k.w[m] = row[5 + m];
         return;
     }
-    const float4* row = reinterpret_cast<const float4*>(tab + (k.code != kCodeEscape ? k.code : 0u) * kWideStride);
+    const float4* row = reinterpret_cast<const float4*>(tab + k.code * kWideStride);
     const float4 q0 = row[0], q1 = row[1], q2 = row[2], q3 = row[3];
     k.ik[0] = q0.x;
     k.a[0][0] = q0.y;
@@ -156,17 +156,6 @@ __device__ inline void coef_tail(CellCoef<ND, MODEL>& k, const DevSim& s, Idx c)
     const float w[kNCoef] = {q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y};
 #pragma unroll
     for (int m = 0; m < kNCoef; ++m) k.w[m] = w[m];
-    if (k.code == kCodeEscape) {  // a tuple without a code: the maps
-        const CodedCoef e = escape_coef<VEL, false>(s, (uint32_t)c);
-        k.ik[0] = e.ik;
-        k.a[0][0] = e.a1;
-        k.a[0][1] = e.a2;
-        k.b[0][0] = e.b1;
-        k.b[0][1] = e.b2;
-        const float* ce = s.coef + (int64_t)e.dc * ND * kNCoef;
-#pragma unroll
-        for (int m = 0; m < kNCoef; ++m) k.w[m] = ce[m];
-    }
 }
 
 // TAPE: also write the adjoint tape of the step (DevSim::tape_u, tape_div)
@@ -202,7 +191,7 @@ __global__ __launch_bounds__(256) void k_velocity_cell(DevSim batch, unsigned gx
     }
     rho_c = at(s.rho, 0, c);
     coef_maps<ND, MODEL, true>(k, s, c);
-    coef_tail<ND, MODEL, true>(k, s, c);
+    coef_tail<ND, MODEL, true>(k, s);
 #pragma unroll
     for (int a = 0; a < ND; ++a) {
         if (MODEL != kCellCoded && a > 0 && !s.coef_axes_same) load_weights(k.w, s, k.dc, ND, a);
@@ -264,7 +253,7 @@ __device__ inline void pressure_cell(const DevSim& s, Idx c) {
     }
     const float p = at(s.p, 0, c), K = at(s.K, 0, c);
     coef_maps<ND, MODEL, false>(k, s, c);
-    coef_tail<ND, MODEL, false>(k, s, c);
+    coef_tail<ND, MODEL, false>(k, s);
     float div = 0.f;
 #pragma unroll
     for (int a = 0; a < ND; ++a) {

@@ -154,9 +154,7 @@ __device__ __forceinline__ CodedCoef escape_coef(const DevSim& s, uint32_t c) {
 // a coded grid
 template <bool VEL, bool UNIFORM>
 __device__ __forceinline__ CodedCoef coef_of_code(const DevSim& s, uint32_t c, uint32_t code) {
-    if (code != kCodeEscape) return coded_coef(VEL ? s.rtab_v : s.rtab_p, code);
-    if (VEL) return mapped_coef<UNIFORM>(s.ikv[0], s.av[0][0], s.av[0][1], s.bv[0][0], s.bv[0][1], s.dcmap, c);
-    return mapped_coef<UNIFORM>(s.ikp[0], s.ap[0][0], s.ap[0][1], s.bp[0][0], s.bp[0][1], s.dcmap, c);
+    return code != kCodeEscape ? coded_coef(VEL ? s.rtab_v : s.rtab_p, code) : escape_coef<VEL, UNIFORM>(s, c);
 }
 // the same, reading the code first (the row gather then waits for the code)
 template <bool VEL, bool UNIFORM>

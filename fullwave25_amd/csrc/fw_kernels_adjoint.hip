@@ -80,14 +80,6 @@ __global__ __launch_bounds__(256) void k_adj_sparse(float* lp, const float* grow
 // kernels load a row's operands before the gathers that precede their use, so that the loads are
 // in flight during the gathers. The per-cell kernels use the same structs and the same arithmetic.
 
-// the relaxation coefficients of the cell once its code is in (CODED; escaped cells read the maps)
-template <bool VEL>
-__device__ inline CodedCoef decode_cell(const DevSim& s, int64_t c, uint32_t code) {
-    if (code != kCodeEscape) return coded_coef(VEL ? s.rtab_v : s.rtab_p, code);
-    if (VEL) return mapped_coef<true>(s.ikv[0], s.av[0][0], s.av[0][1], s.bv[0][0], s.bv[0][1], s.dcmap, (uint32_t)c);
-    return mapped_coef<true>(s.ikp[0], s.ap[0][0], s.ap[0][1], s.bp[0][0], s.bp[0][1], s.dcmap, (uint32_t)c);
-}
-
 // operands of the pressure transposed at one cell
 template <int ND, bool EXPO, bool CODED>
 struct PreOps {
@@ -119,7 +111,7 @@ __device__ inline void pre_load(const DevSim& s, const AdjView& w, int64_t c, Pr
 template <int ND, bool EXPO, bool CODED>
 __device__ inline void pre_decode(const DevSim& s, int64_t c, PreOps<ND, EXPO, CODED>& o) {
     if (!CODED || EXPO) return;
-    const CodedCoef k = decode_cell<false>(s, c, o.code);
+    const CodedCoef k = coef_of_code<false, true>(s, (uint32_t)c, o.code);
 #pragma unroll
     for (int a = 0; a < ND; ++a) o.kc[a] = k;
 }
@@ -233,7 +225,7 @@ __device__ inline void vel_load(const DevSim& s, const AdjView& w, int64_t c, Ve
 template <int ND, bool EXPO, bool CODED>
 __device__ inline void vel_decode(const DevSim& s, int64_t c, VelOps<ND, EXPO, CODED>& o) {
     if (!CODED || EXPO) return;
-    const CodedCoef k = decode_cell<true>(s, c, o.code);
+    const CodedCoef k = coef_of_code<true, true>(s, (uint32_t)c, o.code);
 #pragma unroll
     for (int a = 0; a < ND; ++a) o.kc[a] = k;
 }

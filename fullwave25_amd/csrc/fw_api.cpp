@@ -581,7 +581,7 @@ int choose_kernels_unpinned(fw_sim* s) {
     // planes a workgroup only make fewer workgroups) or, where launches are long, a quarter slower than the best of
     // all (members of one family differ by 8 % from the first two on). The plain 3D marching kernels are behind the
     // pipelined ones at every size measured, and time only where those cannot run. Set-up of a handle,
-    // first run included: 131 x 117 x 109 cells 67 -> 6 ms; 400 x 400 x 360 555 -> 70 ms.
+    // first run included: 131 x 117 x 109 cells 67 -> 6 ms; 400 x 400 x 360 555 -> 83 ms.
     std::vector<std::vector<fw::LaunchCfg>> families;
     auto family = [&](int variant, int width, std::initializer_list<int> chunks) {
         families.emplace_back();

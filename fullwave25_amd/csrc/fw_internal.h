@@ -67,7 +67,7 @@ struct DevSim {
     // writes, at every updated cell, tape_u[a][c] = D+_a p / kappa + psi1' + psi2' (exponential
     // model: A D+_a p), and the pressure kernel tape_div[c] = sum_a (D-_a v_a' / kappa + phi1' +
     // phi2') (exponential model: sum_a D-_a v_a'): what the adjoint needs of the forward state.
-    // Single-transmit handles only; the per-cell and tiled 2D kernels write it (launch_velocity
+    // Single-transmit handles only; the per-cell, tiled 2D and brick kernels write it (launch_velocity
     // / launch_pressure take those while a tape is set).
     float* tape_u[kMaxDim];
     float* tape_div;

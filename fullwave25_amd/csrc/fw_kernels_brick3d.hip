@@ -8,10 +8,10 @@
 // arms are staged in LDS with 16-byte loads, 8 (velocity) and 13 (pressure) a lane, all issued before
 // the first is waited for, as are the memory variables and the coefficient rows; a quad's stencil reads
 // are 16-byte LDS reads. us a step, best of the other families -> bricks (16 read and written fields):
-//   88 x 88 x 88      33.9 -> 21.8       131 x 117 x 109   68.0 -> 49.0      200 x 180 x 160   192 -> 148
-//   300 x 64 x 300     206 -> 132        600 x 500 x 200   2126 -> 1782
-// 400 x 400 x 360: velocity 886 -> 838, pressure 839 (marching) and 857. 64 x 64 x 64: 12.9 (per-cell)
-// and 14.9, too few bricks. Exponential model, 131 x 117 x 109: 42.1 -> 37.9; 200 x 180 x 160: 134 -> 103.
+//   88 x 88 x 88      27.1 -> 20.2       131 x 117 x 109   53.4 -> 45.7      200 x 180 x 160   192 -> 149
+//   300 x 64 x 300     192 -> 130        600 x 500 x 200   2126 -> 1782
+// 400 x 400 x 360: velocity 888 -> 831, pressure 846 (marching) and 835. 64 x 64 x 64: 14.0 (per-cell)
+// and 14.8, too few bricks. Exponential model, 131 x 117 x 109: 43.0 -> 35.7; 200 x 180 x 160: 138 -> 89.
 // What bounds it: at 131 x 117 x 109 the phases of a brick (load, compute, store) with two rounds of
 // three workgroups a CU (166 registers, 39 and 49 KB of LDS); large grids the memory traffic.
 // Measured and left out: reading the stencil from the caches with 16-byte loads in place of LDS (131 x

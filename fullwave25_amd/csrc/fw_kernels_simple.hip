@@ -10,8 +10,9 @@
 // set) reads the row (or the weights) with scalar loads. The pressure kernel also does the step's
 // sources, pressure release and sensors at the points of its own cells. Before (axis after axis, each
 // waiting for the stores of the last, the per-cell maps, a boundary launch of its own), us a step:
-// 256 x 224 cells 10.7 -> 7.3; 1003 x 677 35.7 -> 22.9; exponential model on 1152 x 1150 32.0 -> 22.3;
-// 131 x 117 x 109 69.5 -> 67.7 (there the 72 stencil reads a cell bound it, not their latency).
+// 256 x 224 cells 10.7 -> 9.3 (two launches of the host; the kernels take 3.6 and 4.3); 1003 x 677 35.7 ->
+// 22.9; exponential model on 1152 x 1150 32.0 -> 22.3; 131 x 117 x 109 69.5 -> 53.4 (there the 72 stencil
+// reads a cell bound it, and the memory variables go through the caches: cell_memory_streams).
 //
 // A workgroup of 256 lanes takes 4 rows of 64 cells. The arithmetic and its order are the other
 // families'.

@@ -250,7 +250,8 @@ typedef struct fw_adj fw_adj;
  * checkpoints (ceil(nT / checkpoint_every) states), the tape of one segment and scratch.
  * checkpoint_every 0: the whole run when its tape fits in half of the device's free memory,
  * else the segment length that minimises checkpoints plus tape. The handle's velocity and
- * pressure kernels become the tiled 2D or per-cell ones if it had chosen others. */
+ * pressure kernels become ones that write the tape if it had chosen others: the tiled 2D ones, the
+ * 3D bricks on grids of 160 bricks or more, else the per-cell ones. */
 int fw_adj_create(fw_sim* sim, int64_t checkpoint_every, fw_adj** out);
 /* The segment length in use (as chosen for checkpoint_every 0). */
 int fw_adj_checkpoint_every(const fw_adj* adj, int64_t* every);
